@@ -163,19 +163,19 @@ void record_sample(vt_batch *b, hipStream_t s) {
     const int vertices = std::max(0, (int)b->max_depth - 1) + 1 + (b->sampling_mode == 3u ? 1 : 0);
     for (uint32_t base = 0; base < b->total; base += cap) {
         const uint32_t n = std::min(cap, b->total - base);
-        check(vt::launch_reset_counters(cnt, 16, s), "reset");
-        check(vt::launch_batch_generate(bt, base, n, queue_view(b, 0, cap), b->radiance.as<float>(), cnt, grid, s), "generate");
+        const auto pair = [&](int v) { return cnt + vt::kCounterPairs + 2 * v; };
+        check(vt::launch_reset_counters(cnt, vt::kCounterWords, s), "reset");
+        check(vt::launch_batch_generate(bt, base, n, queue_view(b, 0, cap), b->radiance.as<float>(), pair(0), grid, s),
+              "generate");
         int cur = 0;
         for (int v = 0; v < vertices; ++v) {
-            uint32_t *cin = cnt + cur, *cout = cnt + (1 - cur), *csh = cnt + 2;
-            check(vt::launch_reset_counters(cout, 1, s), "reset");
-            check(vt::launch_reset_counters(csh, 1, s), "reset");
+            const uint32_t *cin = pair(v), *csh = pair(v + 1) + 1;
             const vt::PathQueue qin = queue_view(b, cur, cap), qout = queue_view(b, 1 - cur, cap);
             const vt::RayArgs rays{qin.ox, qin.oy, qin.oz, qin.dx, qin.dy, qin.dz, qin.tmin, qin.tmax};
             check(vt::launch_trace_batch(jt, qin.job, rays, hits, nullptr, n, false, cin, b->tree_depth,
                                          b->tuning.trace_block, tgrid, s), "extend");
-            check(vt::launch_batch_shade(bt, qin, hits, qout, sh, vt::Counters{cin, cout, csh}, n, b->radiance.as<float>(),
-                                         b->layered, grid, s), "shade");
+            check(vt::launch_batch_shade(bt, qin, hits, qout, sh, vt::Counters{cin, reinterpret_cast<unsigned long long *>(pair(v + 1))}, n, b->radiance.as<float>(),
+                                         b->layered, s), "shade");
             const vt::RayArgs srays{sh.ox, sh.oy, sh.oz, sh.dx, sh.dy, sh.dz, sh.tmin, sh.tmax};
             check(vt::launch_trace_batch(jt, sh.job, srays, vt::HitArgs{}, b->occluded.as<uint8_t>(), n, true, csh,
                                          b->tree_depth, b->tuning.trace_block, tgrid, s), "shadow");
@@ -289,7 +289,7 @@ vt_status vt_batch_create(vt_context *ctx, const vt_batch_job *jobs, uint32_t co
         b->job_scene_d.upload(b->job_scene.data(), b->job_scene.size() * 4);
         b->first_d.upload(b->first.data(), b->first.size() * 4);
         b->frame_count.alloc(4);
-        b->counters.alloc(64 * 4);
+        b->counters.alloc(vt::kCounterWords * sizeof(uint32_t));
         b->accum.alloc((size_t)b->total * 16);
         upload_tables(b.get());
         reset_frames(b.get());

@@ -1029,6 +1029,38 @@ __device__ __forceinline__ uint32_t wave_append(uint32_t *counter, bool pred) {
     return base + rank;
 }
 
+// Queue slots for a whole block at once.  Two queues share one 64-bit counter (low and high word), so a
+// block of four waves makes one atomic for its continuations and shadow rays, and one more for its cache
+// queries and training records (pair p picks the LDS words).  The counters are single words that every
+// wave of the chip adds to, and such adds retire one at a time: with an atomic per wave and queue, the
+// shading of 4.2M Cornell paths (131k adds) took 1.36 ms, about 10 ns an add whatever the shading cost;
+// with an eighth of them 0.29 ms, 3.3 TB/s of queue traffic.  All threads of the block call it together,
+// once per pair.
+constexpr int kShadeBlock = 256, kShadeWaves = kShadeBlock / 64;
+struct AppendShared {
+    unsigned long long wave[2][kShadeWaves], base[2];
+};
+__device__ __forceinline__ void block_append(AppendShared &lds, int p, unsigned long long *counter, bool want0, bool want1,
+                                             uint32_t (&slot)[2]) {
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const unsigned long long below = (1ull << lane) - 1ull;
+    const unsigned long long m0 = __ballot(want0), m1 = __ballot(want1);
+    if (lane == 0) lds.wave[p][wave] = (unsigned long long)__popcll(m0) | ((unsigned long long)__popcll(m1) << 32);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        unsigned long long sum = 0;
+#pragma unroll
+        for (int w = 0; w < kShadeWaves; ++w) sum += lds.wave[p][w];
+        lds.base[p] = sum ? atomicAdd(counter, sum) : 0ull;
+    }
+    __syncthreads();
+    unsigned long long at = lds.base[p];
+#pragma unroll
+    for (int w = 0; w < kShadeWaves; ++w) at += (uint32_t)w < wave ? lds.wave[p][w] : 0ull;
+    slot[0] = (uint32_t)at + (uint32_t)__popcll(m0 & below);
+    slot[1] = (uint32_t)(at >> 32) + (uint32_t)__popcll(m1 & below);
+}
+
 constexpr uint32_t kPrevDelta = 1u << 16, kPrevNee = 1u << 17, kPrevMis = 1u << 18;
 // BSDF-only paths (mode 3) past the scattering budget: one last continuation that may only reach
 // emission (main.swift:7716-7722, 7785).
@@ -1440,16 +1472,17 @@ __global__ __launch_bounds__(256) void restir_gi_resolve_kernel(FrameArgs f, Res
 
 // Shading of one wavefront vertex per path.  kRestir: sampling mode 0, where a diffuse primary vertex
 // takes its direct light from ReSTIR DI's spatial reuse (main.swift:7484-7580) instead of NEE.
-// Shading of queue slot i (active: i holds a path) by every lane of the wave together: the queue
-// appends are wave-wide.  `job` is carried to the continuation and shadow queues when they have a job
+// Shading of queue slot i (active: i holds a path) by every thread of the block together: the queue
+// appends are block-wide (block_append).  `job` is carried to the continuation and shadow queues when they have a job
 // array (batched rendering).
 template <bool kRestir, bool kLayered>
 __device__ __forceinline__ void shade_path(const RenderScene &sc, const FrameArgs &f, const PathQueue &in,
                                            const HitArgs &hits, const PathQueue &out, const ShadowQueue &sh,
                                            const Counters &c, uint32_t capacity, float *radiance, const RestirArgs &ra,
-                                           const NrcArgs &nrc, uint32_t i, bool active, uint32_t job) {
+                                           const NrcArgs &nrc, uint32_t i, bool active, uint32_t job,
+                                           AppendShared &append) {
     bool cont = false, shadow = false;
-    // Continuation and shadow-ray values produced below (written after the wave-wide appends).
+    // Continuation and shadow-ray values produced below (written after the block-wide appends).
     V3 new_o = v3(0.0f, 0.0f, 0.0f), new_d = v3(0.0f, 0.0f, 1.0f), prev_p = v3(0.0f, 0.0f, 0.0f);
     V3 sh_o = new_o, sh_d = new_d, sh_c = new_o;
     S4 sh_s = s4(0.0f);
@@ -1715,11 +1748,12 @@ __device__ __forceinline__ void shade_path(const RenderScene &sc, const FrameArg
             radiance[3 * (size_t)id + 2] += add.z;
         }
     }
-    const uint32_t slot = wave_append(c.out, cont);
-    const uint32_t sslot = wave_append(c.shadow, shadow);
+    uint32_t at[2];
+    block_append(append, 0, c.out, cont, shadow, at);
+    const uint32_t slot = at[0], sslot = at[1];
     if (f.nrc) {
-        const uint32_t qslot = wave_append(nrc.q_count, query);
-        const uint32_t rslot = wave_append(nrc.r_count, record);
+        block_append(append, 1, nrc.counts, query, record, at);
+        const uint32_t qslot = at[0], rslot = at[1];
         if (query && qslot < capacity) {
             for (int k = 0; k < kNrcInputCount; ++k) nrc.q_in[(size_t)k * nrc.q_stride + qslot] = cin[k];
             nrc.q_thr[qslot] = make_float4(thr.v[0], thr.v[1], thr.v[2], thr.v[3]);  // unchanged: the path ended
@@ -1761,13 +1795,19 @@ __device__ __forceinline__ void shade_path(const RenderScene &sc, const FrameArg
     }
 }
 
+// One thread per queue slot, the block being the unit of the queue appends.  (A grid of a few blocks per
+// CU striding over the queue was tried: the loop made the compiler hoist scene loads into registers,
+// 106 -> 142 and 162 -> 215, an occupancy step lost.)
 template <bool kRestir, bool kLayered, bool kEnv>
-__global__ __launch_bounds__(256) void shade_kernel(RenderScene sc, FrameArgs f, PathQueue in, HitArgs hits,
-                                                    PathQueue out, ShadowQueue sh, Counters c, uint32_t capacity,
-                                                    float *radiance, RestirArgs ra, NrcArgs nrc) {
-    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+__global__ __launch_bounds__(kShadeBlock) void shade_kernel(RenderScene sc, FrameArgs f, PathQueue in, HitArgs hits,
+                                                            PathQueue out, ShadowQueue sh, Counters c, uint32_t capacity,
+                                                            float *radiance, RestirArgs ra, NrcArgs nrc) {
+    __shared__ AppendShared append;
+    const uint32_t i = blockIdx.x * kShadeBlock + threadIdx.x;
     const uint32_t n = min(*c.in, capacity);
-    shade_path<kRestir, kLayered>(sc, frame_env<kEnv>(f), in, hits, out, sh, c, capacity, radiance, ra, nrc, i, i < n, 0u);
+    if (blockIdx.x * kShadeBlock >= n) return;  // the whole block
+    shade_path<kRestir, kLayered>(sc, frame_env<kEnv>(f), in, hits, out, sh, c, capacity, radiance, ra, nrc, i, i < n, 0u,
+                                  append);
 }
 // Material sorting: paths whose hit needs the layered BSDF (GLOSSY above the delta threshold, OPENPBR)
 // are listed from the end of `perm`, all others (Lambert, delta, emitters, misses) from its start, both
@@ -1792,26 +1832,31 @@ __global__ __launch_bounds__(256) void classify_kernel(RenderScene sc, HitArgs h
     if (active && layered) perm[capacity - 1u - b] = i;
 }
 template <bool kLayered>
-__global__ __launch_bounds__(256) void shade_sorted_kernel(RenderScene sc, FrameArgs f, PathQueue in, HitArgs hits,
+__global__ __launch_bounds__(kShadeBlock) void shade_sorted_kernel(RenderScene sc, FrameArgs f, PathQueue in, HitArgs hits,
                                                            PathQueue out, ShadowQueue sh, Counters c, uint32_t capacity,
                                                            float *radiance, NrcArgs nrc, const uint32_t *perm,
                                                            const uint32_t *class_count) {
-    const uint32_t k = blockIdx.x * 256 + threadIdx.x;
-    const bool active = k < min(*class_count, capacity);
+    __shared__ AppendShared append;
+    const uint32_t k = blockIdx.x * kShadeBlock + threadIdx.x;
+    const uint32_t n = min(*class_count, capacity);
+    if (blockIdx.x * kShadeBlock >= n) return;
+    const bool active = k < n;
     const uint32_t i = active ? perm[kLayered ? capacity - 1u - k : k] : 0u;
-    shade_path<false, kLayered>(sc, f, in, hits, out, sh, c, capacity, radiance, RestirArgs{}, nrc, i, active, 0u);
+    shade_path<false, kLayered>(sc, f, in, hits, out, sh, c, capacity, radiance, RestirArgs{}, nrc, i, active, 0u, append);
 }
 
 // The Lambert / delta shading without ReSTIR (a kernel of its own so its register allocation is not
 // shaped by the layered BSDF's).
 template <bool kEnv>
-__global__ __launch_bounds__(256) void shade_lean_kernel(
+__global__ __launch_bounds__(kShadeBlock) void shade_lean_kernel(
     RenderScene sc, FrameArgs f, PathQueue in, HitArgs hits, PathQueue out, ShadowQueue sh, Counters c,
     uint32_t capacity, float *radiance, NrcArgs nrc) {
-    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    __shared__ AppendShared append;
+    const uint32_t i = blockIdx.x * kShadeBlock + threadIdx.x;
     const uint32_t n = min(*c.in, capacity);
-    shade_path<false, false>(sc, frame_env<kEnv>(f), in, hits, out, sh, c, capacity, radiance, RestirArgs{}, nrc, i,
-                             i < n, 0u);
+    if (blockIdx.x * kShadeBlock >= n) return;
+    shade_path<false, false>(sc, frame_env<kEnv>(f), in, hits, out, sh, c, capacity, radiance, RestirArgs{}, nrc, i, i < n,
+                             0u, append);
 }
 
 __global__ __launch_bounds__(256) void resolve_kernel(FrameArgs f, ShadowQueue sh, const uint8_t *occluded,
@@ -1911,7 +1956,7 @@ __global__ __launch_bounds__(64) void bake_metal_kernel(float *out) {
     out[node] = sum / 16384.0f;
 }
 __global__ void reset_kernel(uint32_t *counters, uint32_t n) {
-    if (threadIdx.x < n) counters[threadIdx.x] = 0u;
+    for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) counters[i] = 0u;
 }
 
 // Running mean per pixel over this wavefront's samples in sample order (main.swift:7862-7913):
@@ -1965,20 +2010,21 @@ __global__ __launch_bounds__(256) void batch_generate_kernel(BatchTables bt, uin
     }
 }
 
-// Waves stride together (the loop bound is wave-uniform) so the queue appends see every lane.
+// One thread per queue slot of the launch's capacity (see shade_kernel), not the persistent grid of the
+// other batch kernels.
 template <bool kLayered>
-__global__ __launch_bounds__(256) void batch_shade_kernel(BatchTables bt, PathQueue in, HitArgs hits, PathQueue out,
-                                                          ShadowQueue sh, Counters c, uint32_t capacity, float *radiance) {
+__global__ __launch_bounds__(kShadeBlock) void batch_shade_kernel(BatchTables bt, PathQueue in, HitArgs hits, PathQueue out,
+                                                                  ShadowQueue sh, Counters c, uint32_t capacity,
+                                                                  float *radiance) {
+    __shared__ AppendShared append;
+    const uint32_t i = blockIdx.x * kShadeBlock + threadIdx.x;
     const uint32_t n = min(*c.in, capacity);
-    const uint32_t lane = threadIdx.x & 63u, stride = gridDim.x * 256;
-    for (uint32_t base = blockIdx.x * 256 + (threadIdx.x & ~63u); base < n; base += stride) {
-        const uint32_t i = base + lane;
-        const bool active = i < n;
-        const uint32_t j = active ? in.job[i] : 0u;
-        // Batched jobs render without environment lighting.
-        shade_path<false, kLayered>(bt.scenes[bt.job_scene[j]], frame_env<false>(bt.frames[j]), in, hits, out, sh, c,
-                                    capacity, radiance, RestirArgs{}, NrcArgs{}, i, active, j);
-    }
+    if (blockIdx.x * kShadeBlock >= n) return;
+    const bool active = i < n;
+    const uint32_t j = active ? in.job[i] : 0u;
+    // Batched jobs render without environment lighting.
+    shade_path<false, kLayered>(bt.scenes[bt.job_scene[j]], frame_env<false>(bt.frames[j]), in, hits, out, sh, c, capacity,
+                                radiance, RestirArgs{}, NrcArgs{}, i, active, j, append);
 }
 
 __global__ __launch_bounds__(256) void batch_resolve_kernel(ShadowQueue sh, const uint8_t *occluded, const uint32_t *count,
@@ -2031,7 +2077,7 @@ hipError_t launch_generate(const FrameArgs &f, const PathQueue &q, float *radian
 hipError_t launch_shade(const RenderScene &sc, const FrameArgs &f, const PathQueue &in, const HitArgs &hits,
                         const PathQueue &out, const ShadowQueue &sh, const Counters &c, uint32_t capacity,
                         float *radiance, const NrcArgs &nrc, hipStream_t s) {
-    const dim3 grid((capacity + 255) / 256);
+    const dim3 grid((capacity + kShadeBlock - 1) / kShadeBlock);
     const bool env = frame_has_env(sc, f);
     if (sc.layered && env)
         hipLaunchKernelGGL((shade_kernel<false, true, true>), grid, dim3(256), 0, s, sc, f, in, hits, out, sh, c,
@@ -2051,7 +2097,7 @@ hipError_t launch_shade(const RenderScene &sc, const FrameArgs &f, const PathQue
 hipError_t launch_shade_sorted(const RenderScene &sc, const FrameArgs &f, const PathQueue &in, const HitArgs &hits,
                                const PathQueue &out, const ShadowQueue &sh, const Counters &c, uint32_t capacity,
                                float *radiance, const NrcArgs &nrc, uint32_t *perm, uint32_t *classes, hipStream_t s) {
-    const dim3 grid((capacity + 255) / 256);
+    const dim3 grid((capacity + kShadeBlock - 1) / kShadeBlock);
     hipLaunchKernelGGL(classify_kernel, grid, dim3(256), 0, s, sc, hits, c.in, capacity, perm, classes);
     hipLaunchKernelGGL((shade_sorted_kernel<false>), grid, dim3(256), 0, s, sc, f, in, hits, out, sh, c, capacity, radiance,
                        nrc, perm, classes);
@@ -2063,7 +2109,7 @@ hipError_t launch_shade_sorted(const RenderScene &sc, const FrameArgs &f, const 
 hipError_t launch_shade_restir(const RenderScene &sc, const FrameArgs &f, const PathQueue &in, const HitArgs &hits,
                                const PathQueue &out, const ShadowQueue &sh, const Counters &c, uint32_t capacity,
                                float *radiance, const RestirArgs &ra, const NrcArgs &nrc, hipStream_t s) {
-    const dim3 grid((capacity + 255) / 256);
+    const dim3 grid((capacity + kShadeBlock - 1) / kShadeBlock);
     const bool env = frame_has_env(sc, f);
     if (sc.layered && env)
         hipLaunchKernelGGL((shade_kernel<true, true, true>), grid, dim3(256), 0, s, sc, f, in, hits, out, sh, c,
@@ -2165,7 +2211,8 @@ hipError_t launch_batch_generate(const BatchTables &bt, uint32_t chunk_base, uin
 
 hipError_t launch_batch_shade(const BatchTables &bt, const PathQueue &in, const HitArgs &hits, const PathQueue &out,
                               const ShadowQueue &sh, const Counters &c, uint32_t capacity, float *radiance, bool layered,
-                              uint32_t grid, hipStream_t s) {
+                              hipStream_t s) {
+    const uint32_t grid = (capacity + kShadeBlock - 1) / kShadeBlock;
     if (layered)
         hipLaunchKernelGGL((batch_shade_kernel<true>), dim3(grid), dim3(256), 0, s, bt, in, hits, out, sh, c, capacity, radiance);
     else

@@ -131,7 +131,8 @@ struct NrcArgs {
     float4 *q_thr;       // throughput reaching it, per lane
     float *q_wl;         // wavelength number
     uint32_t *q_id;      // path id
-    uint32_t *q_count;
+    unsigned long long *counts;  // queries (low word), records (high word)
+    const uint32_t *q_count;     // the words of `counts`
     uint32_t q_stride;   // query capacity
     float *q_out;        // [cap][4] cache outputs
     float4 *sacc;        // [paths] spectral radiance a training path has gathered so far (by path id)
@@ -139,7 +140,7 @@ struct NrcArgs {
     float4 *r_thr;       // throughput reaching it
     float4 *r_snap;      // sacc of its path when it was reached
     uint32_t *r_id;
-    uint32_t *r_count;
+    const uint32_t *r_count;
     uint32_t r_cap;
     float *r_target;     // [rcap][4] built after the wavefront: (sacc final - snap) / thr * unit
     // The network's unit: its outputs and targets are spectral radiance times `unit` (1 / the mean of
@@ -169,9 +170,15 @@ struct ShadowQueue {
     uint32_t *job = nullptr;  // batched rendering: the ray's job
 };
 
+// A vertex's queue lengths: the paths that reach it in the low word of a 64-bit counter, the shadow rays
+// its predecessor cast in the high word, so a block of shading threads claims both with one atomic.
 struct Counters {
-    uint32_t *in, *out, *shadow;
+    const uint32_t *in;
+    unsigned long long *out;
 };
+// The counters of a wavefront, cleared once at its start: words 0, 1 the cache's queries and records, 2, 3
+// the material classes, then a pair per vertex (at most 255 vertices and the one past them).
+constexpr uint32_t kCounterPairs = 8, kMaxVertices = 255, kCounterWords = kCounterPairs + 2 * (kMaxVertices + 1);
 
 // Batched rendering: many images (jobs) of many scenes in one wavefront.  A sample's work items are
 // the jobs' pixels back to back: item g is pixel g - first[j] of job j, first[j] <= g < first[j + 1],
@@ -238,7 +245,7 @@ hipError_t launch_batch_generate(const BatchTables &bt, uint32_t chunk_base, uin
                                  float *radiance, uint32_t *count, uint32_t grid, hipStream_t s);
 hipError_t launch_batch_shade(const BatchTables &bt, const PathQueue &in, const HitArgs &hits, const PathQueue &out,
                               const ShadowQueue &sh, const Counters &c, uint32_t capacity, float *radiance, bool layered,
-                              uint32_t grid, hipStream_t s);
+                              hipStream_t s);
 hipError_t launch_batch_resolve(const ShadowQueue &sh, const uint8_t *occluded, const uint32_t *count, uint32_t capacity,
                                 float *radiance, uint32_t grid, hipStream_t s);
 hipError_t launch_batch_accumulate(const BatchTables &bt, uint32_t chunk_base, uint32_t chunk_n, const float *radiance,

@@ -169,7 +169,8 @@ vt::NrcArgs nrc_view(vt_renderer *r, uint32_t *counters) {
     a.q_wl = reinterpret_cast<float *>(q + cap * 15 * 4);
     a.q_id = reinterpret_cast<uint32_t *>(q + cap * 16 * 4);
     a.q_out = reinterpret_cast<float *>(q + cap * 17 * 4);
-    a.q_count = counters + 3;
+    a.counts = reinterpret_cast<unsigned long long *>(counters);
+    a.q_count = counters;
     a.q_stride = (uint32_t)cap;
     char *rr = r->nrc_records.as<char>();
     a.r_in = reinterpret_cast<float *>(rr);
@@ -177,7 +178,7 @@ vt::NrcArgs nrc_view(vt_renderer *r, uint32_t *counters) {
     a.r_snap = reinterpret_cast<float4 *>(rr + rcap * 15 * 4);
     a.r_id = reinterpret_cast<uint32_t *>(rr + rcap * 19 * 4);
     a.r_target = reinterpret_cast<float *>(rr + rcap * 20 * 4);
-    a.r_count = counters + 4;
+    a.r_count = counters + 1;
     a.r_cap = (uint32_t)rcap;
     a.sacc = r->nrc_sacc.as<float4>();
     a.unit = 1.0f;
@@ -546,7 +547,7 @@ vt_status vt_renderer_create(vt_context *ctx, vt_renderer **out) {
         if (!ctx || !out) return fail(VT_ERROR_INVALID_ARGUMENT, "context and out must not be NULL");
         auto r = std::make_unique<vt_renderer>();
         r->ctx = ctx;
-        r->counters.alloc(16 * sizeof(uint32_t));
+        r->counters.alloc(vt::kCounterWords * sizeof(uint32_t));
         check(hipHostMalloc((void **)&r->host_count, sizeof(uint32_t), hipHostMallocDefault), "hipHostMalloc");
         *out = r.release();
         return VT_OK;
@@ -578,7 +579,7 @@ vt_status vt_renderer_cache_records(vt_renderer *r, float *inputs, float *target
         if (r->nrc_rcap == 0 || !r->counters.ptr) return VT_OK;
         check(hipDeviceSynchronize(), "hipDeviceSynchronize");
         uint32_t made = 0;
-        check(hipMemcpy(&made, r->counters.as<uint32_t>() + 4, 4, hipMemcpyDeviceToHost), "hipMemcpy");
+        check(hipMemcpy(&made, r->counters.as<uint32_t>() + 1, 4, hipMemcpyDeviceToHost), "hipMemcpy");
         *count = made;
         const uint32_t n = std::min({made, r->nrc_rcap, max_records});
         const vt::NrcArgs a = nrc_view(r, r->counters.as<uint32_t>());
@@ -747,9 +748,12 @@ static vt_status render_frame(vt_renderer *r, vt_scene *scene, const vt_frame_pa
             f.z_temporal = p->z_temporal;
             f.frame0 = r->frame_index;
             const uint32_t n = f.samples * npix;
-            check(vt::launch_reset_counters(cnt, 16, s), "reset");
+            // Vertex b's counters: pair(b)[0] the paths that reach it, pair(b)[1] the shadow rays cast
+            // at vertex b - 1.
+            const auto pair = [&](int b) { return cnt + vt::kCounterPairs + 2 * b; };
+            check(vt::launch_reset_counters(cnt, vt::kCounterWords, s), "reset");
             int cur = 0;
-            check(vt::launch_generate(f, r->q[0].view(r->capacity), r->radiance.as<float>(), cnt + 0, s), "generate");
+            check(vt::launch_generate(f, r->q[0].view(r->capacity), r->radiance.as<float>(), pair(0), s), "generate");
             vt::NrcArgs na{};
             if (use_cache) {
                 na = nrc_view(r, cnt);
@@ -782,20 +786,18 @@ static vt_status render_frame(vt_renderer *r, vt_scene *scene, const vt_frame_pa
             // Vertices: the scattering budget bounds non-delta events only; with delta materials in the
             // scene, keep extending (checking the live count every 8 vertices) until no path is left.
             const int base = f.scattering_limit + 1 + (f.sampling_mode == 3u ? 1 : 0);
-            const int cap = scene->has_delta ? 255 : base;
+            const int cap = scene->has_delta ? (int)vt::kMaxVertices : base;
             for (int b = 0; b < cap; ++b) {
                 if (b >= base && (b - base) % 8 == 0) {
-                    check(hipMemcpyAsync(r->host_count, cnt + cur, 4, hipMemcpyDeviceToHost, s), "hipMemcpyAsync");
+                    check(hipMemcpyAsync(r->host_count, pair(b), 4, hipMemcpyDeviceToHost, s), "hipMemcpyAsync");
                     check(hipStreamSynchronize(s), "hipStreamSynchronize");
                     if (*r->host_count == 0) break;
                 }
-                uint32_t *cin = cnt + cur, *cout = cnt + (1 - cur), *csh = cnt + 2;
-                check(vt::launch_reset_counters(cout, 1, s), "reset");
-                check(vt::launch_reset_counters(csh, 1, s), "reset");
+                const uint32_t *cin = pair(b), *csh = pair(b + 1) + 1;
                 const vt::PathQueue qin = r->q[cur].view(r->capacity), qout = r->q[1 - cur].view(r->capacity);
                 vt::RayArgs rays{qin.ox, qin.oy, qin.oz, qin.dx, qin.dy, qin.dz, qin.tmin, qin.tmax};
                 check(vt::launch_trace(scene->view, rays, hits, nullptr, n, false, nullptr, s, cin), "extend");
-                vt::Counters c{cin, cout, csh};
+                const vt::Counters c{cin, reinterpret_cast<unsigned long long *>(pair(b + 1))};
                 if (restir && b == 0) {
                     check(vt::launch_restir_initial(sc, f, qin, hits, ra, s), "restir pass 1");
                     if (gi) {
@@ -815,10 +817,10 @@ static vt_status render_frame(vt_renderer *r, vt_scene *scene, const vt_frame_pa
                     check(vt::launch_shade_restir(sc, f, qin, hits, qout, sh, c, n, r->radiance.as<float>(), ra, na, s),
                           "shade");
                 } else if (p->material_sort && scene->mixed) {
-                    // Material sorting (classes counted in counters 5 and 6).
-                    check(vt::launch_reset_counters(cnt + 5, 2, s), "reset");
+                    // Material sorting (classes counted in counters 2 and 3).
+                    check(vt::launch_reset_counters(cnt + 2, 2, s), "reset");
                     check(vt::launch_shade_sorted(sc, f, qin, hits, qout, sh, c, n, r->radiance.as<float>(), na,
-                                                  r->perm.as<uint32_t>(), cnt + 5, s), "shade");
+                                                  r->perm.as<uint32_t>(), cnt + 2, s), "shade");
                 } else {
                     check(vt::launch_shade(sc, f, qin, hits, qout, sh, c, n, r->radiance.as<float>(), na, s), "shade");
                 }
