@@ -16,10 +16,10 @@ using vt::fail;
 
 struct vt_nrc {
     vt_context *ctx = nullptr;
-    DeviceBuffer params, grads, m, v, ema, wbf16, wema, loss;
+    DeviceBuffer params, grads, partials, m, v, ema, wbf16, wema, loss;
     uint32_t step = 0;
     vt::NrcDevice view() const {
-        return vt::NrcDevice{params.as<float>(), grads.as<float>(), m.as<float>(), v.as<float>(), ema.as<float>(),
+        return vt::NrcDevice{params.as<float>(), m.as<float>(), v.as<float>(), ema.as<float>(), partials.as<float>(),
                              wbf16.as<uint16_t>(), wema.as<uint16_t>()};
     }
 };
@@ -67,7 +67,6 @@ std::vector<float> initial_params(uint32_t seed) {
 void upload_params(vt_nrc *n, const float *p) {
     check(hipMemcpy(n->params.ptr, p, (size_t)vt::kNrcParams * 4, hipMemcpyHostToDevice), "hipMemcpy");
     check(vt::launch_nrc_sync(n->view(), nullptr), "nrc sync");
-    check(vt::launch_nrc_zero(n->grads.as<float>(), vt::kNrcParams, nullptr), "nrc zero");
     check(vt::launch_nrc_zero(n->m.as<float>(), vt::kNrcParams, nullptr), "nrc zero");
     check(vt::launch_nrc_zero(n->v.as<float>(), vt::kNrcParams, nullptr), "nrc zero");
     check(hipDeviceSynchronize(), "hipDeviceSynchronize");
@@ -87,6 +86,7 @@ vt_status vt_nrc_create(vt_context *ctx, uint32_t seed, vt_nrc **out) {
         const size_t bytes = (size_t)vt::kNrcParams * 4;
         n->params.alloc(bytes);
         n->grads.alloc(bytes);
+        n->partials.alloc(bytes * vt::kNrcTrainBlocks);
         n->m.alloc(bytes);
         n->v.alloc(bytes);
         n->ema.alloc((size_t)vt::kNrcParams * 4);
@@ -141,7 +141,7 @@ vt_status vt_nrc_train(vt_nrc *n, const float *inputs, const float *targets, uin
         check(hipSetDevice(n->ctx->device), "hipSetDevice");
         hipStream_t s = (hipStream_t)stream;
         check(vt::launch_nrc_backward(n->view(), inputs, targets, count, (float)count * vt::kNrcOut, nullptr, s), "nrc backward");
-        check(vt::launch_nrc_adam(n->view(), ++n->step, learning_rate, s), "nrc adam");
+        check(vt::launch_nrc_adam(n->view(), ++n->step, learning_rate, s, count), "nrc adam");
         return VT_OK;
     });
 }
@@ -151,16 +151,15 @@ vt_status vt_nrc_gradients(vt_nrc *n, const float *inputs, const float *targets,
     return vt::guarded_call([&]() -> vt_status {
         if (!n || (count && (!inputs || !targets)) || !grads) return fail(VT_ERROR_INVALID_ARGUMENT, "arguments must not be NULL");
         check(hipSetDevice(n->ctx->device), "hipSetDevice");
-        check(vt::launch_nrc_zero(n->grads.as<float>(), vt::kNrcParams, nullptr), "nrc zero");
         check(vt::launch_nrc_zero(n->loss.as<float>(), 1, nullptr), "nrc zero");
         check(vt::launch_nrc_backward(n->view(), inputs, targets, count, (float)count * vt::kNrcOut, n->loss.as<float>(), nullptr),
               "nrc backward");
+        check(vt::launch_nrc_reduce(n->view(), count, n->grads.as<float>(), nullptr), "nrc reduce");
         check(hipDeviceSynchronize(), "hipDeviceSynchronize");
         check(hipMemcpy(grads, n->grads.ptr, (size_t)vt::kNrcParams * 4, hipMemcpyDeviceToHost), "hipMemcpy");
         float l = 0.0f;
         check(hipMemcpy(&l, n->loss.ptr, 4, hipMemcpyDeviceToHost), "hipMemcpy");
         if (loss) *loss = count ? l / ((float)count * vt::kNrcOut) : 0.0f;
-        check(vt::launch_nrc_zero(n->grads.as<float>(), vt::kNrcParams, nullptr), "nrc zero");
         return VT_OK;
     });
 }

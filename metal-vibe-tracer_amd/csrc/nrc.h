@@ -23,9 +23,13 @@ constexpr int kNrcW5 = kNrcOutPad * kNrcHidden;             // 1024
 constexpr int kNrcParams = kNrcW1 + 3 * kNrcWh + kNrcW5;    // 30720
 constexpr float kNrcEmaDecay = 0.95f;
 
+// Blocks of a training launch at most, and so sets of partial gradients (one per CU).
+constexpr uint32_t kNrcTrainBlocks = 256;
+
 struct NrcDevice {
-    float *params, *grads, *m, *v, *ema;  // kNrcParams each
-    uint16_t *wbf16, *wema;                // kNrcParams bf16 bits: params (training), ema (inference)
+    float *params, *m, *v, *ema;  // kNrcParams each
+    float *partials;              // kNrcTrainBlocks x kNrcParams: a backward launch's sums per block
+    uint16_t *wbf16, *wema;       // kNrcParams bf16 bits: params (training), ema (inference)
 };
 
 // out[q * 4 + c] = y_c(inputs of query q) with the averaged weights, for q < n, or for q < min(*count, n)
@@ -39,15 +43,16 @@ struct NrcSlice {
     const uint32_t *count = nullptr;
     uint32_t limit = 0, parts = 1, part = 0;
 };
-// grads += d loss / d params over samples [0, n), or over the slice when slice.count is given, the loss
+// partials = d loss / d params over samples [0, n), or over the slice when slice.count is given, the loss
 // normalised by `norm` outputs (norm <= 0: 4 x the samples present); loss_sum (if not null) += the
-// per-sample losses.
+// per-sample losses.  Read by launch_nrc_reduce / launch_nrc_adam with the same n and slice.
 hipError_t launch_nrc_backward(const NrcDevice &d, const float *inputs, const float *targets, uint32_t n, float norm,
                                float *loss_sum, hipStream_t s, const NrcSlice &slice = NrcSlice{}, uint32_t stride = 0);
-// Adam step `step` (1-based) on params from grads, then ema = decay ema + (1 - decay) params; refreshes
-// both bf16 copies and clears grads.  With
-// slice.count given, the step is skipped (grads cleared) when the slice of at most n samples is empty.
-hipError_t launch_nrc_adam(const NrcDevice &d, uint32_t step, float lr, hipStream_t s, uint32_t n = 0,
+// grads = the sum of the partials of a backward launch over n samples.
+hipError_t launch_nrc_reduce(const NrcDevice &d, uint32_t n, float *grads, hipStream_t s);
+// Adam step `step` (1-based) on params from the partials of the backward launch over the same n and slice,
+// then ema = decay ema + (1 - decay) params; refreshes both bf16 copies.  Skipped when the slice is empty.
+hipError_t launch_nrc_adam(const NrcDevice &d, uint32_t step, float lr, hipStream_t s, uint32_t n,
                            const NrcSlice &slice = NrcSlice{});
 // ema = params and both bf16 copies (after the params are set from the host).
 hipError_t launch_nrc_sync(const NrcDevice &d, hipStream_t s);

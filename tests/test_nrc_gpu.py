@@ -79,6 +79,28 @@ def test_gradient_check(gpu_ctx):
     cache.close()
 
 
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 127, 128, 129, 300, 32769])
+def test_gradients_at_tile_edges(gpu_ctx, n):
+    # Around a wave's 16 samples, a block's 128 and one block's second group (256 blocks x 128 + 1).
+    # Against the oracle that rounds where the kernel does, gradients agree to fp32 summation order but
+    # for activations whose sum lies at a bf16 rounding boundary: each moves one of its sample's terms by
+    # a bf16 step, 2^-8 relative, so the whole by less than that.
+    cache = vt.NRC(gpu_ctx, seed=3)
+    p = _params(2)
+    cache.params = p
+    rng = np.random.default_rng(n)
+    x = rng.random((n, 11)).astype(np.float32)
+    t = rng.random((n, 4)).astype(np.float32)
+    g, loss = cache.gradients(_dev(x), _dev(t))
+    ref = onrc.split(onrc.gradients(p.astype(np.float64), x, t, bf16=True))
+    err = [np.linalg.norm(a - b) / np.linalg.norm(b) for a, b in zip(onrc.split(g), ref)]
+    print(f"n {n}: per layer " + " ".join(f"{e:.1e}" for e in err), flush=True)
+    assert max(err) < 2.0 ** -8
+    again, _ = cache.gradients(_dev(x), _dev(t))
+    assert np.array_equal(g, again)   # summed in a fixed order
+    cache.close()
+
+
 def test_adam_step_matches_oracle(gpu_ctx):
     cache = vt.NRC(gpu_ctx, seed=3)
     p = _params(4)
