@@ -16,11 +16,21 @@ using vt::fail;
 
 struct vt_nrc {
     vt_context *ctx = nullptr;
-    DeviceBuffer params, grads, partials, m, v, ema, wbf16, wema, loss;
+    // One allocation: params, grads, m, v, ema (fp32), the two bf16 copies, the loss sum, and the partial
+    // gradients of a backward launch's blocks.
+    DeviceBuffer store;
+    static constexpr size_t kSet = (size_t)vt::kNrcParams * 4;
+    static constexpr size_t kBf16 = 5 * kSet, kLoss = kBf16 + kSet, kPartials = kLoss + 256;
+    static constexpr size_t kBytes = kPartials + kSet * vt::kNrcTrainBlocks;
     uint32_t step = 0;
+    float *params() const { return store.as<float>(); }
+    float *grads() const { return params() + vt::kNrcParams; }
+    float *loss() const { return reinterpret_cast<float *>(store.as<char>() + kLoss); }
     vt::NrcDevice view() const {
-        return vt::NrcDevice{params.as<float>(), m.as<float>(), v.as<float>(), ema.as<float>(), partials.as<float>(),
-                             wbf16.as<uint16_t>(), wema.as<uint16_t>()};
+        float *p = params();
+        uint16_t *w = reinterpret_cast<uint16_t *>(store.as<char>() + kBf16);
+        return vt::NrcDevice{p, p + 2 * vt::kNrcParams, p + 3 * vt::kNrcParams, p + 4 * vt::kNrcParams,
+                             reinterpret_cast<float *>(store.as<char>() + kPartials), w, w + vt::kNrcParams};
     }
 };
 
@@ -65,10 +75,9 @@ std::vector<float> initial_params(uint32_t seed) {
 }
 
 void upload_params(vt_nrc *n, const float *p) {
-    check(hipMemcpy(n->params.ptr, p, (size_t)vt::kNrcParams * 4, hipMemcpyHostToDevice), "hipMemcpy");
+    check(hipMemcpy(n->params(), p, (size_t)vt::kNrcParams * 4, hipMemcpyHostToDevice), "hipMemcpy");
     check(vt::launch_nrc_sync(n->view(), nullptr), "nrc sync");
-    check(vt::launch_nrc_zero(n->m.as<float>(), vt::kNrcParams, nullptr), "nrc zero");
-    check(vt::launch_nrc_zero(n->v.as<float>(), vt::kNrcParams, nullptr), "nrc zero");
+    check(vt::launch_nrc_zero(n->view().m, 2 * vt::kNrcParams, nullptr), "nrc zero");  // m and v
     check(hipDeviceSynchronize(), "hipDeviceSynchronize");
     n->step = 0;
 }
@@ -83,16 +92,7 @@ vt_status vt_nrc_create(vt_context *ctx, uint32_t seed, vt_nrc **out) {
         check(hipSetDevice(ctx->device), "hipSetDevice");
         auto n = std::make_unique<vt_nrc>();
         n->ctx = ctx;
-        const size_t bytes = (size_t)vt::kNrcParams * 4;
-        n->params.alloc(bytes);
-        n->grads.alloc(bytes);
-        n->partials.alloc(bytes * vt::kNrcTrainBlocks);
-        n->m.alloc(bytes);
-        n->v.alloc(bytes);
-        n->ema.alloc((size_t)vt::kNrcParams * 4);
-        n->wbf16.alloc((size_t)vt::kNrcParams * 2);
-        n->wema.alloc((size_t)vt::kNrcParams * 2);
-        n->loss.alloc(4);
+        n->store.alloc(vt_nrc::kBytes);
         std::vector<float> p = initial_params(seed);
         upload_params(n.get(), p.data());
         *out = n.release();
@@ -107,7 +107,7 @@ vt_status vt_nrc_get_params(vt_nrc *n, float *params) {
         if (!n || !params) return fail(VT_ERROR_INVALID_ARGUMENT, "cache and params must not be NULL");
         check(hipSetDevice(n->ctx->device), "hipSetDevice");
         check(hipDeviceSynchronize(), "hipDeviceSynchronize");
-        check(hipMemcpy(params, n->params.ptr, (size_t)vt::kNrcParams * 4, hipMemcpyDeviceToHost), "hipMemcpy");
+        check(hipMemcpy(params, n->params(), (size_t)vt::kNrcParams * 4, hipMemcpyDeviceToHost), "hipMemcpy");
         return VT_OK;
     });
 }
@@ -151,14 +151,14 @@ vt_status vt_nrc_gradients(vt_nrc *n, const float *inputs, const float *targets,
     return vt::guarded_call([&]() -> vt_status {
         if (!n || (count && (!inputs || !targets)) || !grads) return fail(VT_ERROR_INVALID_ARGUMENT, "arguments must not be NULL");
         check(hipSetDevice(n->ctx->device), "hipSetDevice");
-        check(vt::launch_nrc_zero(n->loss.as<float>(), 1, nullptr), "nrc zero");
-        check(vt::launch_nrc_backward(n->view(), inputs, targets, count, (float)count * vt::kNrcOut, n->loss.as<float>(), nullptr),
+        check(vt::launch_nrc_zero(n->loss(), 1, nullptr), "nrc zero");
+        check(vt::launch_nrc_backward(n->view(), inputs, targets, count, (float)count * vt::kNrcOut, n->loss(), nullptr),
               "nrc backward");
-        check(vt::launch_nrc_reduce(n->view(), count, n->grads.as<float>(), nullptr), "nrc reduce");
+        check(vt::launch_nrc_reduce(n->view(), count, n->grads(), nullptr), "nrc reduce");
         check(hipDeviceSynchronize(), "hipDeviceSynchronize");
-        check(hipMemcpy(grads, n->grads.ptr, (size_t)vt::kNrcParams * 4, hipMemcpyDeviceToHost), "hipMemcpy");
+        check(hipMemcpy(grads, n->grads(), (size_t)vt::kNrcParams * 4, hipMemcpyDeviceToHost), "hipMemcpy");
         float l = 0.0f;
-        check(hipMemcpy(&l, n->loss.ptr, 4, hipMemcpyDeviceToHost), "hipMemcpy");
+        check(hipMemcpy(&l, n->loss(), 4, hipMemcpyDeviceToHost), "hipMemcpy");
         if (loss) *loss = count ? l / ((float)count * vt::kNrcOut) : 0.0f;
         return VT_OK;
     });
