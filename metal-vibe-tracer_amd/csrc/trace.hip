@@ -24,13 +24,13 @@ constexpr int kRefillIdle = 12;
 template <int kStack, int kBlk = kBlock>
 struct LdsStack {
     uint32_t (*base)[kBlk];
-    uint32_t (*bits)[kBlk];
+    uint16_t (*bits)[kBlk];  // imask << 8 | slots still to visit
     int lane;
     int sp;
     int cap;  // groups the stack may hold: kStack, or less under TraceScene::stack_cap
     __device__ __forceinline__ void push(uint32_t b, uint32_t m) {
         base[sp][lane] = b;
-        bits[sp][lane] = m;
+        bits[sp][lane] = (uint16_t)m;
         ++sp;
     }
     __device__ __forceinline__ bool full() const { return sp >= cap; }
@@ -49,7 +49,7 @@ __global__ __launch_bounds__(kBlock) void trace_kernel(const U4 *__restrict__ no
                                                        float root_max, unsigned long long *__restrict__ counters,
                                                        uint32_t *__restrict__ fault, int cap) {
     __shared__ uint32_t stack_base[kStack][kBlock];
-    __shared__ uint32_t stack_bits[kStack][kBlock];
+    __shared__ uint16_t stack_bits[kStack][kBlock];
     const int lane = threadIdx.x;
     const uint32_t i = blockIdx.x * kBlock + lane;
     if (count) n = min(n, *count);
@@ -74,8 +74,8 @@ __global__ __launch_bounds__(kBlock) void trace_kernel(const U4 *__restrict__ no
     }
 }
 
-// Persistent traversal with lane refill.  Each block owns a contiguous range of the rays (the grid is
-// sized to what the chip holds at once); its waves draw batches of 64 ray indices from an LDS counter,
+// Persistent traversal with lane refill.  The grid is sized to what the chip holds at once; the waves of a
+// block draw batches of 64 ray indices, the block's share of the rays, from an LDS counter,
 // and a lane whose ray finishes takes the next index at once, so a wave no longer idles until its
 // slowest ray ends.  Node visits are per lane (trav_nodes); the triangles the wave's lanes reach in a
 // step are tested by the whole wave together (wave_triangles).  Per ray the arithmetic, the nodes
@@ -161,9 +161,10 @@ __device__ __forceinline__ void wave_lds_order() {
 // that lane's ray through cross-lane permutes, runs the same Woop test, and folds a hit into the
 // owner's LDS slot with an atomic minimum of (order-preserving t bits << 32 | face) -- the nearest t,
 // equal t going to the smaller face, as the one-lane rule.  The winner of each round stores its t and
-// barycentrics; the key's identity picks it since a face is tested at most once per ray.  A hit at t
-// must also lie in [tmin, tmax) (the one-lane rule's first accepted hit needs t < tmax).  Any-hit
-// queries only raise the owner's flag.  Must be called by all 64 lanes together.
+// barycentrics; the key's identity picks it since a face is tested at most once per ray.  They stay in the
+// owner's LDS slot until its ray ends, as do its triangle-test constants (woop, packed by pack_woop): both
+// are read only around triangle tests, and the registers are worth a wave per SIMD.  Any-hit queries only
+// raise the owner's flag.  Must be called by all 64 lanes together.
 // Exclusive prefix over the wave of per-lane counts below 32 (pre) and their sum (total): one ballot per
 // bit of the count.
 __device__ __forceinline__ void wave_prefix(uint32_t cnt, unsigned long long below, uint32_t &pre, uint32_t &total) {
@@ -177,21 +178,25 @@ __device__ __forceinline__ void wave_prefix(uint32_t cnt, unsigned long long bel
     }
 }
 
+__device__ __forceinline__ F4 pack_woop(const WoopRay &w) {
+    return F4{w.sx, w.sy, w.sz, bits_to_float((uint32_t)(w.kx | (w.ky << 2) | (w.kz << 4)))};
+}
+
 template <bool ANY, int kBlk, class Source>
 __device__ __forceinline__ void wave_triangles(const Source &src, const typename Source::Lane &sl, TravState &ts,
-                                               uint32_t trimask, uint32_t tri_base, uint32_t lane, uint32_t pre,
-                                               uint32_t total, unsigned long long *key, float (*hit_tb)[kBlk]) {
+                                               uint32_t trimask, uint32_t tri_base, uint32_t tri_bits, uint32_t lane, uint32_t pre,
+                                               uint32_t total, const F4 *woop, unsigned long long *key, float (*hit_tb)[kBlk]) {
     const uint32_t cnt = __popc(trimask);
     if (total == 0u) return;
     const uint32_t wave0 = threadIdx.x & ~63u;
     unsigned long long key0 = 0ull;
     if (cnt) {
-        if (!ANY) key0 = ((unsigned long long)ord_bits(ts.res.t) << 32) | (uint32_t)ts.res.face;
+        // No hit yet counts as face 0, so that a hit at exactly tmax is not nearer.
+        if (!ANY) key0 = ((unsigned long long)ord_bits(ts.res.t) << 32) | (uint32_t)max(ts.res.face, 0);
         key[threadIdx.x] = key0;
     }
     wave_lds_order();
-    const int kpack = ts.w.kx | (ts.w.ky << 2) | (ts.w.kz << 4);
-    const uint64_t tri_bits = reinterpret_cast<uint64_t>(src.tri_ptr(sl));
+    const uint64_t tri_addr = reinterpret_cast<uint64_t>(src.tri_ptr(sl));
     for (uint32_t j0 = 0; j0 < total; j0 += 64u) {
         const uint32_t j = j0 + lane;
         uint32_t owner = 0;
@@ -203,31 +208,34 @@ __device__ __forceinline__ void wave_triangles(const Source &src, const typename
         const int o = (int)owner;
         const uint32_t k = j - (uint32_t)__shfl((int)pre, o);
         const uint32_t omask = (uint32_t)__shfl((int)trimask, o), obase = (uint32_t)__shfl((int)tri_base, o);
-        const int kp = __shfl(kpack, o);
+        const uint32_t obits = (uint32_t)__shfl((int)tri_bits, o);
+        const F4 wo = woop[wave0 + owner];
+        const uint32_t kp = float_to_bits(wo.w);
         WoopRay w;
-        w.kx = kp & 3;
-        w.ky = (kp >> 2) & 3;
-        w.kz = kp >> 4;
-        w.sx = __shfl(ts.w.sx, o);
-        w.sy = __shfl(ts.w.sy, o);
-        w.sz = __shfl(ts.w.sz, o);
+        w.kx = (int)(kp & 3u);
+        w.ky = (int)((kp >> 2) & 3u);
+        w.kz = (int)(kp >> 4);
+        w.sx = wo.x;
+        w.sy = wo.y;
+        w.sz = wo.z;
         const float ox = __shfl(ts.ox, o), oy = __shfl(ts.oy, o), oz = __shfl(ts.oz, o);
-        const float tmin = __shfl(ts.tmin, o), tmax = __shfl(ts.tmax, o);
+        const float tmin = __shfl(ts.tmin, o);
+        const float tmax = ANY ? __shfl(ts.res.t, o) : 0.0f;
         const F4 *tris;
         if constexpr (Source::kShared) {
             tris = src.tri_ptr(sl);
         } else {
-            const uint32_t lo = (uint32_t)__shfl((int)(uint32_t)tri_bits, o);
-            const uint32_t hi = (uint32_t)__shfl((int)(uint32_t)(tri_bits >> 32), o);
+            const uint32_t lo = (uint32_t)__shfl((int)(uint32_t)tri_addr, o);
+            const uint32_t hi = (uint32_t)__shfl((int)(uint32_t)(tri_addr >> 32), o);
             tris = reinterpret_cast<const F4 *>(((uint64_t)hi << 32) | lo);
         }
         bool hit = false;
         unsigned long long mine = 0ull;
         float t = 0.0f, b1 = 0.0f, b2 = 0.0f;
         if (j < total) {
-            const F4 *tp = tris + 3 * (size_t)(obase + nth_set_bit(omask, k));
+            const F4 *tp = tris + 3 * (size_t)(obase + tri_rank(obits, nth_set_bit(omask, k)));
             const F4 p0 = tp[0], p1 = tp[1], p2 = tp[2];
-            if (woop_triangle(w, ox, oy, oz, p0, p1, p2, t, b1, b2) && t >= tmin && t < tmax) {
+            if (woop_triangle(w, ox, oy, oz, p0, p1, p2, t, b1, b2) && t >= tmin && (!ANY || t < tmax)) {
                 hit = true;
                 if (ANY) {
                     key[wave0 + owner] = 1ull;
@@ -254,8 +262,6 @@ __device__ __forceinline__ void wave_triangles(const Source &src, const typename
         } else if (got != key0) {
             ts.res.t = hit_tb[0][threadIdx.x];
             ts.res.face = (int32_t)(uint32_t)got;
-            ts.res.b1 = hit_tb[1][threadIdx.x];
-            ts.res.b2 = hit_tb[2][threadIdx.x];
         }
     }
     wave_lds_order();
@@ -265,14 +271,22 @@ template <bool ANY, int kStack, int kBlk, class Source>
 __device__ __forceinline__ void refill_trace(const Source &src, const RayArgs &rays, const HitArgs &hits,
                                              uint8_t *__restrict__ occluded, uint32_t n) {
     __shared__ uint32_t stack_base[kStack][kBlk];
-    __shared__ uint32_t stack_bits[kStack][kBlk];
+    __shared__ uint16_t stack_bits[kStack][kBlk];
     __shared__ uint32_t next;
     __shared__ unsigned long long tri_key[kBlk];
     __shared__ float tri_hit[ANY ? 1 : 3][kBlk];
+    __shared__ F4 woop[kBlk];
     constexpr uint32_t kNone = 0xffffffffu;
-    const uint32_t chunk = ((n + gridDim.x - 1) / gridDim.x + 63u) & ~63u;
-    const uint32_t begin = min(n, blockIdx.x * chunk), end = min(n, begin + chunk);
-    if (threadIdx.x == 0) next = begin;
+    // The rays are dealt out in units of a few batches of 64, a unit to each block in turn, so cheap and dear
+    // regions of an image are spread over the blocks (against one contiguous range per block: 10 M terrain
+    // bounce rays 681 -> 640 us, field shadow rays 213 -> 189 us) and a launch of few rays over the CUs.
+    // (Renumbering the blocks so that each XCD's share is contiguous lost it all again: the XCDs' shares
+    // are uneven, and their L2s hold the same upper tree anyway.)
+    const uint32_t batches = n / 64u + (n % 64u != 0u), blocks = gridDim.x;
+    constexpr uint32_t kWaves = kBlk / 64;
+    uint32_t shift = 0;  // unit = 1 << shift: a batch per wave of the block, fewer when the rays are few
+    while ((2u << shift) <= kWaves && (2u << shift) <= batches / blocks) ++shift;
+    if (threadIdx.x == 0) next = 0;
     __syncthreads();
     const uint32_t lane = threadIdx.x & 63u;
     const unsigned long long below = (1ull << lane) - 1ull;
@@ -282,7 +296,7 @@ __device__ __forceinline__ void refill_trace(const Source &src, const RayArgs &r
     uint32_t ray = kNone;
     // The lane's pending triangles (from its last node visit, not yet tested) and whether its ray has
     // no node left to visit.
-    uint32_t trimask = 0, tri_base = 0;
+    uint32_t trimask = 0, tri_base = 0, tri_bits = 0;
     bool done = false;
     // Wave-uniform: the wave's current batch of 64 indices and how many of them are handed out.
     uint32_t batch = 0, used = 64;
@@ -297,25 +311,28 @@ __device__ __forceinline__ void refill_trace(const Source &src, const RayArgs &r
             const uint32_t avail = 64u - used;
             uint32_t idx = batch + used + rank;
             if (cnt > avail) {
-                uint32_t fresh = 0;
-                if (lane == 0) fresh = atomicAdd(&next, 64u);
-                fresh = __shfl(fresh, 0);
+                uint32_t draw = 0;
+                if (lane == 0) draw = atomicAdd(&next, 1u);
+                draw = __builtin_amdgcn_readfirstlane(draw);
+                const uint32_t at = ((blockIdx.x + (draw >> shift) * blocks) << shift) + (draw & ((1u << shift) - 1u));
+                exhausted = at >= batches;
+                const uint32_t fresh = exhausted ? n : at * 64u;
                 if (rank >= avail) idx = fresh + (rank - avail);
                 batch = fresh;
                 used = cnt - avail;
-                if (fresh >= end) exhausted = true;
             } else {
                 used += cnt;
             }
-            if (ray == kNone && idx < end) {
+            if (ray == kNone && idx < n) {
                 const TraceRay r{rays.ox[idx], rays.oy[idx], rays.oz[idx], rays.dx[idx], rays.dy[idx], rays.dz[idx],
                                  rays.tmin[idx], rays.tmax[idx]};
                 if (src.begin(idx, sl)) {
                     ray = idx;
                     trav_init(ts, r, src.root(sl));
+                    woop[threadIdx.x] = pack_woop(woop_ray(r.dx, r.dy, r.dz));
                     st.sp = 0;
                     st.cap = src.stack_cap(sl, kStack);
-                    done = false;
+                    done = !(r.tmax == r.tmax);  // nothing is nearer than a NaN
                 } else if (ANY) {
                     occluded[idx] = 0;
                 } else {
@@ -332,15 +349,14 @@ __device__ __forceinline__ void refill_trace(const Source &src, const RayArgs &r
         if (!live && exhausted) break;
         // A lane holding untested triangles waits (its next node visit needs the hits they may give),
         // so triangles of several steps are tested together: the wave flushes once a quarter of its
-        // live lanes wait or 64 tests are pending (a CPU replay of the benchmark rays: 0.97 -> 0.62
-        // rounds per step on bounce rays, about 11% fewer issue cycles).  Nodes visited and results
-        // are unchanged.
-        if (busy && !done && trimask == 0u) done = trav_nodes<false>(ts, src.node_ptr(sl), st, trimask, tri_base);
+        // live lanes wait (a CPU replay of the benchmark rays: 0.97 -> 0.62 rounds per step on bounce
+        // rays, about 11% fewer issue cycles).  Nodes visited and results are unchanged.
+        if (busy && !done && trimask == 0u) done = trav_nodes<false>(ts, src.node_ptr(sl), st, trimask, tri_base, tri_bits);
         const unsigned long long waiting = __ballot(busy && (done || trimask != 0u));
-        uint32_t pre, total;
-        wave_prefix(__popc(trimask), below, pre, total);
-        if (total >= 64u || 4u * (uint32_t)__popcll(waiting) >= (uint32_t)__popcll(live)) {
-            wave_triangles<ANY, kBlk>(src, sl, ts, trimask, tri_base, lane, pre, total, tri_key, tri_hit);
+        if (4u * (uint32_t)__popcll(waiting) >= (uint32_t)__popcll(live)) {
+            uint32_t pre, total;
+            wave_prefix(__popc(trimask), below, pre, total);
+            wave_triangles<ANY, kBlk>(src, sl, ts, trimask, tri_base, tri_bits, lane, pre, total, woop, tri_key, tri_hit);
             trimask = 0u;
         }
         if (busy && ((done && trimask == 0u) || (ANY && ts.res.occluded))) {
@@ -351,9 +367,10 @@ __device__ __forceinline__ void refill_trace(const Source &src, const RayArgs &r
             if (ANY) {
                 occluded[ray] = ts.res.occluded ? 1 : 0;
             } else {
+                const bool hit = ts.res.face >= 0;
                 hits.t[ray] = ts.res.t;
-                hits.b1[ray] = ts.res.b1;
-                hits.b2[ray] = ts.res.b2;
+                hits.b1[ray] = hit ? tri_hit[1][threadIdx.x] : 0.0f;
+                hits.b2[ray] = hit ? tri_hit[2][threadIdx.x] : 0.0f;
                 hits.face[ray] = ts.res.face;
                 if (hits.instance) hits.instance[ray] = 0u;
             }
@@ -362,19 +379,26 @@ __device__ __forceinline__ void refill_trace(const Source &src, const RayArgs &r
     }
 }
 
-// Work-group of the persistent kernel: a block's waves share its range of rays, so larger blocks
-// balance uneven rays better (512 lanes: icosphere-field camera rays 0.356 -> 0.237 ms against 128);
-// deeper stacks take 256 so that LDS still holds 5 waves per SIMD.
+// Work-group of the persistent kernel: 512 lanes while LDS then holds 5 to 6 waves per SIMD, 256 for the
+// deepest stacks.  Trees up to depth 11, which the 10 M triangle terrain has, get a stack of 10 groups:
+// with one of 12 their blocks were 256 lanes and 5 % slower on its camera rays.
 template <int kStack>
 constexpr int refill_block() {
-    return kStack <= 8 ? 512 : 256;
+    return kStack <= 10 ? 512 : 256;
+}
+// Waves per SIMD the registers are budgeted for (80 for six).  Six won for any-hit rays and for the
+// shallow stacks of small scenes (Cornell image 9.49 against 9.83 ms), five for closest hits in deep
+// trees, whose rays wait on memory and whose caches a sixth wave only divides (10 M terrain, 2 M rays:
+// camera 480 -> 456 us, bounce 641 -> 630 us).
+template <bool ANY, int kStack>
+constexpr int refill_waves() {
+    return kStack > 12 ? 1 : ANY || kStack <= 8 ? 6 : 5;  // LDS bounds the deeper stacks
 }
 
 template <bool ANY, int kStack>
-__global__ __launch_bounds__(refill_block<kStack>()) void trace_refill_kernel(const U4 *__restrict__ nodes, const F4 *__restrict__ tris,
-                                                              RayArgs rays, HitArgs hits, uint8_t *__restrict__ occluded,
-                                                              uint32_t n, const uint32_t *__restrict__ count,
-                                                              float root_max, uint32_t *__restrict__ fault, int cap) {
+__global__ __launch_bounds__(refill_block<kStack>(), (refill_waves<ANY, kStack>())) void trace_refill_kernel(
+    const U4 *__restrict__ nodes, const F4 *__restrict__ tris, RayArgs rays, HitArgs hits, uint8_t *__restrict__ occluded,
+    uint32_t n, const uint32_t *__restrict__ count, float root_max, uint32_t *__restrict__ fault, int cap) {
     if (count) n = min(n, *count);
     refill_trace<ANY, kStack, refill_block<kStack>()>(OneScene{nodes, tris, root_max, fault, cap}, rays, hits, occluded,
                                                       n);
@@ -392,8 +416,8 @@ __global__ __launch_bounds__(refill_block<kStack>()) void trace_refill_kernel(co
 template <bool ANY, int kTop, int kBot>
 __global__ __launch_bounds__(kBlock) void trace_tlas_kernel(TlasScene sc, RayArgs rays, HitArgs hits,
                                                             uint8_t *__restrict__ occluded, uint32_t n) {
-    __shared__ uint32_t top_base[kTop][kBlock], top_bits[kTop][kBlock];
-    __shared__ uint32_t bot_base[kBot][kBlock], bot_bits[kBot][kBlock];
+    __shared__ uint32_t top_base[kTop][kBlock], bot_base[kBot][kBlock];
+    __shared__ uint16_t top_bits[kTop][kBlock], bot_bits[kBot][kBlock];
     const int lane = threadIdx.x;
     const uint32_t i = blockIdx.x * kBlock + lane;
     if (i >= n) return;
@@ -401,10 +425,11 @@ __global__ __launch_bounds__(kBlock) void trace_tlas_kernel(TlasScene sc, RayArg
     LdsStack<kTop> top{top_base, top_bits, lane, 0, kTop};
     LdsStack<kBot> bot{bot_base, bot_bits, lane, 0, kBot};
     TravState ts, bs;
+    WoopRay bw{};
     trav_init_e(ts, r, sc.enlarge * (max_abs3(r.ox, r.oy, r.oz) + sc.reach));
     float bt = r.tmax, bb1 = 0.0f, bb2 = 0.0f;
     int32_t bface = -1, sentinel = -1;
-    uint32_t binst = 0xffffffffu, cur = 0u, items = 0u, base = 0u;
+    uint32_t binst = 0xffffffffu, cur = 0u, items = 0u, base = 0u, bits = 0u;
     bool occ = false, overflow = false, top_done = false, in_asset = false;
     const U4 *tn = reinterpret_cast<const U4 *>(sc.nodes);
     const U4 *bn = nullptr;
@@ -421,7 +446,7 @@ __global__ __launch_bounds__(kBlock) void trace_tlas_kernel(TlasScene sc, RayArg
         const uint32_t waiting = (uint32_t)__popcll(__ballot(want_top)), live = (uint32_t)__popcll(__ballot(1));
         if (want_top) {
             if (4u * waiting >= live) {
-                top_done = trav_nodes<false>(ts, tn, top, items, base);
+                top_done = trav_nodes<false>(ts, tn, top, items, base, bits);
                 overflow |= ts.res.overflow;
             }
             continue;
@@ -429,9 +454,11 @@ __global__ __launch_bounds__(kBlock) void trace_tlas_kernel(TlasScene sc, RayArg
         if (!in_asset) {
             const uint32_t b = __builtin_ctz(items);
             items &= items - 1u;
-            const InstanceRecord &R = sc.instances[base + b];
+            const InstanceRecord &R = sc.instances[base + tri_rank(bits, b)];
             if (R.faces == 0) continue;
-            trav_init(bs, instance_ray(R.local, r, bt), R.root_max);
+            const TraceRay lr = instance_ray(R.local, r, bt);
+            trav_init(bs, lr, R.root_max);
+            bw = woop_ray(lr.dx, lr.dy, lr.dz);
             // Equal t: a hit of this instance wins over the current one only from a smaller index.
             sentinel = (bface >= 0 && R.index < binst) ? 0x7fffffff : -1;
             bs.res.face = sentinel;
@@ -441,7 +468,7 @@ __global__ __launch_bounds__(kBlock) void trace_tlas_kernel(TlasScene sc, RayArg
             cur = R.index;
             in_asset = true;
         }
-        if (trav_step<ANY, false>(bs, bn, btr, bot)) {
+        if (trav_step<ANY, false>(bs, bw, bn, btr, bot)) {
             in_asset = false;
             overflow |= bs.res.overflow;
             if (ANY) {
@@ -583,7 +610,7 @@ __global__ __launch_bounds__(256) void trace_median_kernel(const F4 *__restrict_
 // job job[i], whose scene is job_trace[job[i]]; rays of one job are contiguous in the queues, so a wave
 // rarely spans two scenes.
 template <bool ANY, int kStack, int kBlk>
-__global__ __launch_bounds__(kBlk) void batch_trace_kernel(const TraceScene *__restrict__ job_trace,
+__global__ __launch_bounds__(kBlk, (kStack <= 12 && kBlk <= 256 ? 5 : 1)) void batch_trace_kernel(const TraceScene *__restrict__ job_trace,
                                                            const uint32_t *__restrict__ job, RayArgs rays, HitArgs hits,
                                                            uint8_t *__restrict__ occluded, uint32_t n,
                                                            const uint32_t *__restrict__ count) {
@@ -595,14 +622,15 @@ __global__ __launch_bounds__(kBlk) void batch_trace_kernel(const TraceScene *__r
 
 namespace {
 
-// Blocks of the refill kernel that are resident at once on the current device (at least 1), capped by
-// the blocks n rays need; the occupancy query is made once per kernel.
+// Blocks of the refill kernel that are resident at once on the current device (at least 1), at most one
+// per batch of 64 rays (a launch of few rays leaves most waves of a block idle but reaches every CU); the
+// occupancy query is made once per kernel.
 uint32_t refill_grid(const void *kernel, uint32_t n, int block) {
     struct Entry {
         const void *k;
         uint32_t blocks;
     };
-    static Entry cache[8] = {};
+    static Entry cache[16] = {};
     static std::mutex lock;
     std::lock_guard<std::mutex> guard(lock);
     uint32_t resident = 0;
@@ -620,7 +648,7 @@ uint32_t refill_grid(const void *kernel, uint32_t n, int block) {
                 break;
             }
     }
-    const uint32_t need = (n + (uint32_t)block - 1) / (uint32_t)block;
+    const uint32_t need = n / 64u + (n % 64u != 0u);
     return need < resident ? (need > 0 ? need : 1) : resident;
 }
 
@@ -676,6 +704,23 @@ hipError_t launch_trace_stats_scratch(int device, const TraceScene &scene, const
         if (e != hipSuccess) return e;
     }
     hipLaunchKernelGGL(sum_pairs_kernel, dim3(1), dim3(64), 0, stream, p, out);
+    return hipGetLastError();
+}
+
+// Node8 records (bvh8.h) re-encoded in place for the traversal (traverse8.h), a record a thread.
+__global__ __launch_bounds__(256) void encode_nodes_kernel(U4 *nodes, uint32_t n) {
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    U4 in[5], out[5];
+#pragma unroll
+    for (int k = 0; k < 5; ++k) in[k] = nodes[5 * (size_t)i + k];
+    encode_node(in, out);
+#pragma unroll
+    for (int k = 0; k < 5; ++k) nodes[5 * (size_t)i + k] = out[k];
+}
+hipError_t launch_encode_nodes(void *nodes, uint32_t n, hipStream_t stream) {
+    if (n == 0) return hipSuccess;
+    hipLaunchKernelGGL(encode_nodes_kernel, dim3((n + 255) / 256), dim3(256), 0, stream, static_cast<U4 *>(nodes), n);
     return hipGetLastError();
 }
 
@@ -775,6 +820,7 @@ hipError_t launch_trace(const TraceScene &scene, const RayArgs &rays, const HitA
         else hipLaunchKernelGGL((trace_refill_kernel<false, S>), dim3(g), dim3(b), 0, stream, nd, tr, rays, hits, occluded, n, count, scene.root_max, scene.fault, cap < S ? cap : S); \
     } while (0)
         if (need <= 8) VT_REFILL(8);
+        else if (need <= 10) VT_REFILL(10);
         else if (need <= 12) VT_REFILL(12);
         else if (need <= 16) VT_REFILL(16);
         else VT_REFILL(24);

@@ -14,7 +14,7 @@ struct HitArgs {
     uint32_t *instance;
 };
 struct TraceScene {
-    const void *nodes;  // Node8 records (bvh8.h)
+    const void *nodes;  // the 8-wide nodes, encoded for the traversal (launch_encode_nodes), or MeshNode records
     const void *tris;   // TriRecord records
     uint32_t node_count;
     uint32_t depth;  // tree depth (root = 1); the traversal stack holds depth - 1 groups
@@ -25,7 +25,7 @@ struct TraceScene {
     // hook; 0 = no cap) can raise it.
     uint32_t *fault;
     uint32_t stack_cap;
-    // 0: Node8 records (the 8-wide tree); 1: MeshNode records (the reference's flat binary median
+    // 0: the 8-wide tree; 1: MeshNode records (the reference's flat binary median
     // hierarchy, bvh8.h), walked by trace_median_kernel with a stack of kMedianStack entries.
     uint32_t kind = 0;
 };
@@ -36,7 +36,7 @@ constexpr uint32_t kMedianStack = 32;
 // each tracing its asset's hierarchy with the object-space ray.
 struct alignas(16) InstanceRecord {
     float local[3][4];  // rows of the world-to-object matrix: x = row.xyz . p + row.w
-    const void *nodes;  // the asset's Node8 records
+    const void *nodes;  // the asset's encoded nodes
     const void *tris;   // the asset's TriRecord records
     float root_max;     // the asset's max |local coordinate| (its box enlargement term)
     uint32_t index;     // the instance's position in the caller's list
@@ -45,13 +45,17 @@ struct alignas(16) InstanceRecord {
 };
 static_assert(sizeof(InstanceRecord) == 80, "InstanceRecord is five 16-byte words");
 struct TlasScene {
-    const void *nodes;                  // Node8 records over instance bounds
+    const void *nodes;                  // encoded nodes over instance bounds
     const InstanceRecord *instances;    // leaf order
     uint32_t node_count, depth;         // of the instance hierarchy
     uint32_t blas_depth;                // deepest asset hierarchy
     float enlarge, reach;               // per-ray growth of the instance boxes: enlarge (|origin|max + reach)
     uint32_t *fault;                    // raised (bit 0) by a ray whose node-group stack filled
 };
+// Re-encodes n Node8 records (bvh8.h) in place, in device memory, as the traversal reads them
+// (traverse8.h).  Every 8-wide hierarchy goes through it once, when it is published.
+hipError_t launch_encode_nodes(void *nodes, uint32_t n, hipStream_t stream);
+
 // Closest hit (hits.instance = the instance's index, 0xffffffff on a miss) or any hit over a
 // two-level scene.  Among hits at exactly equal t the smaller instance index wins, then the smaller
 // face index.

@@ -1,5 +1,16 @@
-// traverse8.h -- per-ray traversal of the 8-wide compressed BVH (layout in bvh8.h), shared by
-// every kernel that traces (closest-hit, any-hit, and the integrator's extend/shadow stages).
+// traverse8.h -- per-ray traversal of the 8-wide compressed BVH, shared by every kernel that traces
+// (closest-hit, any-hit, and the integrator's extend/shadow stages).
+//
+// The builder's Node8 records (bvh8.h) are re-encoded on the device when a hierarchy is published
+// (encode_node) into the form the node test reads with the fewest instructions, 80 bytes as before, five
+// 16-byte words:
+//   w0   grid origin px, py, pz; the high halves of the x and y steps (low and high 16 bits)
+//   w1   first child, first triangle; the high half of the z step (high 16 bits); the triangles of the
+//        leaf children, three bits per slot (bit 3 s + q: slot s has a q-th triangle), and the inner
+//        children (bits 24 + s)
+//   w2-4 per axis, word k: low and high plane of slot 2 k, low and high plane of slot 2 k + 1
+// A step is a power of two, so its high 16 bits are all of it; it is stored times 2^24, because the node
+// test reads a plane byte as the fp16 number with those bits, q 2^-24.
 //
 // The node-group stack is abstracted (Stack::push/pop/size) so a kernel keeps it in LDS.
 // Arithmetic follows the reference exactly where results depend on it:
@@ -109,8 +120,6 @@ VT_HD bool woop_triangle(const WoopRay &w, float ox, float oy, float oz, F4 p0, 
     return true;
 }
 
-VT_HD uint32_t byte_of(uint32_t lo4, uint32_t hi4, int s) { return ((s < 4 ? lo4 : hi4) >> (8 * (s & 3))) & 0xffu; }
-
 struct TraceRay {
     float ox, oy, oz, dx, dy, dz, tmin, tmax;
 };
@@ -125,11 +134,11 @@ struct TraceResult {
 };
 
 // Per-ray traversal state, so a ray can be advanced one node visit at a time (the persistent
-// kernels refill a lane with a new ray as soon as its ray finishes).
+// kernels refill a lane with a new ray as soon as its ray finishes).  The ray's triangle-test constants
+// (WoopRay) are kept apart: the wave-cooperative kernels hold them in LDS.
 struct TravState {
-    WoopRay w;
-    float ox, oy, oz, tmin, tmax;
-    float e, invx, invy, invz;  // e: the reference's box enlargement for this ray
+    float ox, oy, oz, tmin;
+    float invx, invy, invz, ex, ey, ez;  // 1 / direction; e / |direction|, e the reference's box enlargement
     uint32_t oct;  // direction sign bits (x 1, y 2, z 4); the closest hit so far is res.t
     // Current node group: first child index and (imask << 8 | visit-order bits still to visit).
     uint32_t cur_base, cur_bits, node;
@@ -144,13 +153,10 @@ VT_HD void trav_init_e(TravState &st, const TraceRay &r, float e) {
     st.res.occluded = false;
     st.res.overflow = false;
     st.res.nodes = st.res.tris = 0;
-    st.w = woop_ray(r.dx, r.dy, r.dz);
     st.ox = r.ox;
     st.oy = r.oy;
     st.oz = r.oz;
     st.tmin = r.tmin;
-    st.tmax = r.tmax;
-    st.e = e;
     // A component below 1e-8 in magnitude (the reference's parallel threshold) is taken as +-1e-8 with
     // its sign: the slab of a parallel axis then spans about -+1e8 x the origin's distance to its
     // planes -- the whole ray when the origin lies inside the (e-enlarged) slab, nothing reachable
@@ -159,6 +165,9 @@ VT_HD void trav_init_e(TravState &st, const TraceRay &r, float e) {
     st.invx = 1.0f / (fabsf(r.dx) < 1e-8f ? (sx ? -1e-8f : 1e-8f) : r.dx);
     st.invy = 1.0f / (fabsf(r.dy) < 1e-8f ? (sy ? -1e-8f : 1e-8f) : r.dy);
     st.invz = 1.0f / (fabsf(r.dz) < 1e-8f ? (sz ? -1e-8f : 1e-8f) : r.dz);
+    st.ex = e * fabsf(st.invx);
+    st.ey = e * fabsf(st.invy);
+    st.ez = e * fabsf(st.invz);
     st.oct = sx | (sy << 1) | (sz << 2);
     st.cur_base = 0;
     st.cur_bits = 0;
@@ -189,60 +198,114 @@ VT_HD TraceRay instance_ray(const float (&local)[3][4], const TraceRay &r, float
     return l;
 }
 
+#if defined(__HIPCC__)
+// The traversal's node (see the head of this file) of a builder's Node8, both as five 16-byte words.
+__device__ __forceinline__ void encode_node(const U4 (&n)[5], U4 (&o)[5]) {
+    const uint32_t imask = n[0].w >> 24;
+    uint32_t half[3];
+    for (int a = 0; a < 3; ++a) {
+        // 2^(e - 127) as the builder's grid has it (0 for e = 0), times 2^24.  Beyond the float range the
+        // step is infinite and the node is never entered; geometry of that size has no hits, since the
+        // triangle test's products overflow long before.
+        const uint32_t e = (n[0].w >> (8 * a)) & 0xffu;
+        half[a] = e == 0u ? 0u : (e + 24u < 255u ? e + 24u : 255u) << 7;
+    }
+    uint32_t tri = 0;
+    for (int s = 0; s < 8; ++s) {
+        const uint32_t meta = ((s < 4 ? n[1].z : n[1].w) >> (8 * (s & 3))) & 0xffu;
+        if (meta & 0x80u) continue;
+        tri |= ((1u << (meta & 3u)) - 1u) << (3 * s);
+    }
+    o[0] = U4{n[0].x, n[0].y, n[0].z, half[0] | (half[1] << 16)};
+    o[1] = U4{n[1].x, n[1].y, half[2] << 16, tri | (imask << 24)};
+    const uint32_t lo[3][2] = {{n[2].x, n[2].y}, {n[2].z, n[2].w}, {n[3].x, n[3].y}};
+    const uint32_t hi[3][2] = {{n[3].z, n[3].w}, {n[4].x, n[4].y}, {n[4].z, n[4].w}};
+    for (int a = 0; a < 3; ++a) {
+        uint32_t w[4];
+        for (int k = 0; k < 4; ++k) {
+            const int sh = 16 * (k & 1);
+            const uint32_t l = lo[a][k >> 1] >> sh, h = hi[a][k >> 1] >> sh;
+            w[k] = (l & 0xffu) | ((h & 0xffu) << 8) | ((l & 0xff00u) << 8) | ((h & 0xff00u) << 16);
+        }
+        o[2 + a] = U4{w[0], w[1], w[2], w[3]};
+    }
+}
+
+// Two bytes of w as two fp16 numbers q 2^-24: bytes 0 and 2 (sel kPlaneLo) or 1 and 3 (kPlaneHi).
+constexpr uint32_t kPlaneLo = 0x0c020c00u, kPlaneHi = 0x0c030c01u;
+typedef _Float16 h2v __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ h2v plane_pair(uint32_t w, uint32_t sel) {
+    return __builtin_bit_cast(h2v, __builtin_amdgcn_perm(w, w, sel));
+}
+
+// Position of triangle bit p of a node with triangle bits tv (24 bits, tv's high byte ignored): the
+// triangles below it.
+__device__ __forceinline__ uint32_t tri_rank(uint32_t tv, uint32_t p) { return __builtin_popcount(tv & ((1u << p) - 1u)); }
+
 // Node half of a step: tests st.node's 8 child boxes, pushes the current group if inner children were
 // hit, and moves st.node to the next node near to far.  Returns the triangles of the leaf children hit
-// (trimask: bits relative to tri_base, at most 24) and true when no node is left to visit (the
+// (trimask: bits of the node's triangle word tri_bits, whose first triangle is tri_base; triangle p of
+// trimask is record tri_base + tri_rank(tri_bits, p)) and true when no node is left to visit (the
 // triangles returned must still be tested).  The next node does not depend on those triangles, so
 // testing them after the move gives the same result as testing them first.
+//
+// The kernels are bound by the instructions of this test.  Per child: six fused multiply-adds that read
+// their plane as fp16 in place (v_fma_mix_f32), four min / max, a compare and an add-with-carry that
+// shifts the result into the hit mask; per node: 24 byte permutes that pick the near and far planes by
+// the ray's direction signs, and a few words' worth of bit arithmetic for the leaves' triangles and the
+// visiting order.  Converting each byte (48 v_cvt_f32_ubyte), choosing near and far words per axis and
+// handling each child's leaf or inner kind in a branch took about 290 vector and 140 scalar instructions
+// a visit where this takes 200 and 40 (camera rays of the icosphere field 209 -> 168 us with the dealing
+// of rays in trace.hip, bounce rays of the 10 M terrain 775 -> 630 us, 2 M rays each).
 template <bool STATS, class Stack>
-VT_HD bool trav_nodes(TravState &st, const U4 *__restrict__ nodes, Stack &stack, uint32_t &trimask,
-                      uint32_t &tri_base) {
+__device__ __forceinline__ bool trav_nodes(TravState &st, const U4 *__restrict__ nodes, Stack &stack, uint32_t &trimask,
+                                           uint32_t &tri_base, uint32_t &tri_bits) {
     const U4 *np = nodes + 5 * (size_t)st.node;
     const U4 w0 = np[0], w1 = np[1], w2 = np[2], w3 = np[3], w4 = np[4];
     if (STATS) ++st.res.nodes;
-    const float px = bits_to_float(w0.x), py = bits_to_float(w0.y), pz = bits_to_float(w0.z);
-    const float sx = bits_to_float((w0.w & 0xffu) << 23);
-    const float sy = bits_to_float(((w0.w >> 8) & 0xffu) << 23);
-    const float sz = bits_to_float(((w0.w >> 16) & 0xffu) << 23);
-    const uint32_t imask = w0.w >> 24;
-    // Slab distances of plane q of an axis: ((q s + p) - o -+ e) / d = q (s / d) + (p - o -+ e) / d, one
-    // fma per plane.  The near plane of an axis is its low plane for a positive direction, its high
-    // plane otherwise, so the byte words are chosen once per node and no per-child min / max is needed.
-    // The boxes are the reference's e-enlarged ones; the rounding differs from the reference's
-    // (plane - o -+ e) / d by a few ulps of terms no larger than the scene, far inside the enlargement,
-    // so no box the reference enters is culled.
-    const bool nx = (st.oct & 1u) != 0u, ny = (st.oct & 2u) != 0u, nz = (st.oct & 4u) != 0u;
-    const float bx = sx * st.invx, by = sy * st.invy, bz = sz * st.invz;
-    const float dx = px - st.ox, dy = py - st.oy, dz = pz - st.oz;
-    const float alx = (dx - st.e) * st.invx, ahx = (dx + st.e) * st.invx;
-    const float aly = (dy - st.e) * st.invy, ahy = (dy + st.e) * st.invy;
-    const float alz = (dz - st.e) * st.invz, ahz = (dz + st.e) * st.invz;
-    const float anx = nx ? ahx : alx, afx = nx ? alx : ahx;
-    const float any_ = ny ? ahy : aly, afy = ny ? aly : ahy;
-    const float anz = nz ? ahz : alz, afz = nz ? alz : ahz;
-    const uint32_t nxa = nx ? w3.z : w2.x, nxb = nx ? w3.w : w2.y, fxa = nx ? w2.x : w3.z, fxb = nx ? w2.y : w3.w;
-    const uint32_t nya = ny ? w4.x : w2.z, nyb = ny ? w4.y : w2.w, fya = ny ? w2.z : w4.x, fyb = ny ? w2.w : w4.y;
-    const uint32_t nza = nz ? w4.z : w3.x, nzb = nz ? w4.w : w3.y, fza = nz ? w3.x : w4.z, fzb = nz ? w3.y : w4.w;
-    uint32_t hitbits = 0;
-    trimask = 0;
-    tri_base = w1.y;
+    // Slab distances of plane q of an axis: ((q s + p) - o -+ e) / d = q (s / d) + (p - o) / d -+ e / |d|,
+    // one fma per plane.  The near plane of an axis is its low plane for a positive direction, its high
+    // plane otherwise.  The boxes are the reference's e-enlarged ones; the rounding differs from the
+    // reference's (plane - o -+ e) / d by a few ulps of terms no larger than the scene, far inside the
+    // enlargement, so no box the reference enters is culled.
+    const float bx = bits_to_float(w0.w << 16) * st.invx, by = bits_to_float(w0.w & 0xffff0000u) * st.invy;
+    const float bz = bits_to_float(w1.z) * st.invz;
+    const float dx = bits_to_float(w0.x) - st.ox, dy = bits_to_float(w0.y) - st.oy, dz = bits_to_float(w0.z) - st.oz;
+    const float nx = __builtin_fmaf(dx, st.invx, -st.ex), fx = __builtin_fmaf(dx, st.invx, st.ex);
+    const float ny = __builtin_fmaf(dy, st.invy, -st.ey), fy = __builtin_fmaf(dy, st.invy, st.ey);
+    const float nz = __builtin_fmaf(dz, st.invz, -st.ez), fz = __builtin_fmaf(dz, st.invz, st.ez);
+    const uint32_t selx = (st.oct & 1u) ? kPlaneHi : kPlaneLo, sely = (st.oct & 2u) ? kPlaneHi : kPlaneLo;
+    const uint32_t selz = (st.oct & 4u) ? kPlaneHi : kPlaneLo;
+    constexpr uint32_t kOther = kPlaneLo ^ kPlaneHi;
+    const uint32_t wx[4] = {w2.x, w2.y, w2.z, w2.w}, wy[4] = {w3.x, w3.y, w3.z, w3.w}, wz[4] = {w4.x, w4.y, w4.z, w4.w};
+    uint32_t hit = 0;  // bit s: the box of slot s is hit (slots without a child are masked below)
 #pragma unroll
-    for (int s = 0; s < 8; ++s) {
-        const uint32_t meta = byte_of(w1.z, w1.w, s);
-        const float tnx = __builtin_fmaf((float)byte_of(nxa, nxb, s), bx, anx);
-        const float tny = __builtin_fmaf((float)byte_of(nya, nyb, s), by, any_);
-        const float tnz = __builtin_fmaf((float)byte_of(nza, nzb, s), bz, anz);
-        const float tfx = __builtin_fmaf((float)byte_of(fxa, fxb, s), bx, afx);
-        const float tfy = __builtin_fmaf((float)byte_of(fya, fyb, s), by, afy);
-        const float tfz = __builtin_fmaf((float)byte_of(fza, fzb, s), bz, afz);
-        const float tn = fmaxf(fmaxf(tnx, tny), fmaxf(tnz, st.tmin));
-        const float tf = fminf(fminf(tfx, tfy), fminf(tfz, st.res.t));
-        if (tn <= tf && meta != 0u) {
-            if (meta & 0x80u) hitbits |= 1u << (s ^ st.oct);
-            else trimask |= ((1u << (meta & 3u)) - 1u) << (meta >> 2);
+    for (int k = 3; k >= 0; --k) {
+        const h2v pnx = plane_pair(wx[k], selx), pfx = plane_pair(wx[k], selx ^ kOther);
+        const h2v pny = plane_pair(wy[k], sely), pfy = plane_pair(wy[k], sely ^ kOther);
+        const h2v pnz = plane_pair(wz[k], selz), pfz = plane_pair(wz[k], selz ^ kOther);
+#pragma unroll
+        for (int c = 1; c >= 0; --c) {
+            const float tnx = __builtin_fmaf((float)pnx[c], bx, nx), tfx = __builtin_fmaf((float)pfx[c], bx, fx);
+            const float tny = __builtin_fmaf((float)pny[c], by, ny), tfy = __builtin_fmaf((float)pfy[c], by, fy);
+            const float tnz = __builtin_fmaf((float)pnz[c], bz, nz), tfz = __builtin_fmaf((float)pfz[c], bz, fz);
+            const float tn = fmaxf(fmaxf(tnx, tny), fmaxf(tnz, st.tmin));
+            const float tf = fminf(fminf(tfx, tfy), fminf(tfz, st.res.t));
+            // hit = 2 hit + (tn <= tf)
+            asm("v_cmp_le_f32 vcc, %1, %2\n\tv_addc_co_u32 %0, vcc, %0, %0, vcc" : "+v"(hit) : "v"(tn), "v"(tf) : "vcc");
         }
+        __builtin_amdgcn_sched_barrier(0);  // a pair of slots at a time: fewer registers, one wave more per SIMD
     }
-    if (hitbits) {
+    // Each slot's bit spread to its three triangle bits.
+    uint32_t spread = (hit | (hit << 8)) & 0x00f00fu;
+    spread = (spread | (spread << 4)) & 0x0c30c3u;
+    spread = (spread | (spread << 2)) & 0x249249u;
+    tri_bits = w1.w;
+    tri_base = w1.y;
+    trimask = (spread * 7u) & w1.w;
+    // Visiting order: slot s at bit s ^ oct, i.e. neighbours of 1, 2 and 4 swapped where the octant says.
+    uint32_t order = hit & (w1.w >> 24);
+    if (order) {
         if (st.cur_bits & 0xffu) {
             // The launcher sizes the stack to the tree's depth, so a full stack never occurs; if it did,
             // the ray stops (never an out-of-bounds access) and the kernel reports it.
@@ -253,8 +316,12 @@ VT_HD bool trav_nodes(TravState &st, const U4 *__restrict__ nodes, Stack &stack,
             }
             stack.push(st.cur_base, st.cur_bits);
         }
+        const uint32_t s1 = st.oct & 1u, s2 = st.oct & 2u, s4 = st.oct & 4u;
+        order = ((order & 0x55u) << s1) | ((order & 0xaau) >> s1);
+        order = ((order & 0x33u) << s2) | ((order & 0xccu) >> s2);
+        order = ((order & 0x0fu) << s4) | ((order & 0xf0u) >> s4);
         st.cur_base = w1.x;
-        st.cur_bits = (imask << 8) | hitbits;
+        st.cur_bits = ((w1.w >> 16) & 0xff00u) | order;
     }
     if ((st.cur_bits & 0xffu) == 0u) {
         if (stack.empty()) return true;
@@ -266,27 +333,30 @@ VT_HD bool trav_nodes(TravState &st, const U4 *__restrict__ nodes, Stack &stack,
     st.node = st.cur_base + __builtin_popcount((st.cur_bits >> 8) & ((1u << slot) - 1u));
     return false;
 }
+#endif
 
 // A hit of the ray at t on face: the closest-hit rule (nearest t in [tmin, current t), equal t going
 // to the smaller face index).  For the any-hit query any t in [tmin, tmax) ends the ray.
 template <bool ANY>
 VT_HD bool trav_accept(const TravState &st, float t, int32_t face) {
-    if (ANY) return t >= st.tmin && t < st.tmax;
+    if (ANY) return t >= st.tmin && t < st.res.t;  // still tmax: an any-hit query ends at its first hit
     return t >= st.tmin && (t < st.res.t || (t == st.res.t && st.res.face >= 0 && face < st.res.face));
 }
 
 // Triangle half of a step, one lane alone: tests the triangles trav_nodes returned.  Returns true
 // when an any-hit query found a hit.
+#if defined(__HIPCC__)
 template <bool ANY, bool STATS>
-VT_HD bool trav_tris(TravState &st, const F4 *__restrict__ tris, uint32_t trimask, uint32_t tri_base) {
+__device__ __forceinline__ bool trav_tris(TravState &st, const WoopRay &w, const F4 *__restrict__ tris, uint32_t trimask, uint32_t tri_base,
+                                          uint32_t tri_bits) {
     while (trimask) {
         const uint32_t b = __builtin_ctz(trimask);
         trimask &= trimask - 1u;
-        const F4 *tp = tris + 3 * (size_t)(tri_base + b);
+        const F4 *tp = tris + 3 * (size_t)(tri_base + tri_rank(tri_bits, b));
         const F4 p0 = tp[0], p1 = tp[1], p2 = tp[2];
         if (STATS) ++st.res.tris;
         float t, b1, b2;
-        if (!woop_triangle(st.w, st.ox, st.oy, st.oz, p0, p1, p2, t, b1, b2)) continue;
+        if (!woop_triangle(w, st.ox, st.oy, st.oz, p0, p1, p2, t, b1, b2)) continue;
         const int32_t face = (int32_t)float_to_bits(p0.w);
         if (!trav_accept<ANY>(st, t, face)) continue;
         if (ANY) {
@@ -304,22 +374,24 @@ VT_HD bool trav_tris(TravState &st, const F4 *__restrict__ tris, uint32_t trimas
 // One step of one ray: a node visit and the triangles of the leaves it hits.  Returns true when the
 // ray is finished (result in st.res).
 template <bool ANY, bool STATS, class Stack>
-VT_HD bool trav_step(TravState &st, const U4 *__restrict__ nodes, const F4 *__restrict__ tris, Stack &stack) {
-    uint32_t trimask, tri_base;
-    const bool done = trav_nodes<STATS>(st, nodes, stack, trimask, tri_base);
-    if (trav_tris<ANY, STATS>(st, tris, trimask, tri_base)) return true;
+__device__ __forceinline__ bool trav_step(TravState &st, const WoopRay &w, const U4 *__restrict__ nodes, const F4 *__restrict__ tris, Stack &stack) {
+    uint32_t trimask, tri_base, tri_bits;
+    const bool done = trav_nodes<STATS>(st, nodes, stack, trimask, tri_base, tri_bits);
+    if (trav_tris<ANY, STATS>(st, w, tris, trimask, tri_base, tri_bits)) return true;
     return done;
 }
 
-// Traverses one ray.  nodes: Node8 records as 5 U4 each; tris: TriRecord as 3 F4 each.
+// Traverses one ray.  nodes: encoded nodes as 5 U4 each; tris: TriRecord as 3 F4 each.
 template <bool ANY, bool STATS, class Stack>
-VT_HD TraceResult traverse(const U4 *__restrict__ nodes, const F4 *__restrict__ tris, float root_max,
-                           const TraceRay &r, Stack &stack) {
+__device__ __forceinline__ TraceResult traverse(const U4 *__restrict__ nodes, const F4 *__restrict__ tris, float root_max,
+                                                const TraceRay &r, Stack &stack) {
     TravState st;
     trav_init(st, r, root_max);
-    while (!trav_step<ANY, STATS>(st, nodes, tris, stack)) {
+    const WoopRay w = woop_ray(r.dx, r.dy, r.dz);
+    while (!trav_step<ANY, STATS>(st, w, nodes, tris, stack)) {
     }
     return st.res;
 }
+#endif
 
 }  // namespace vt
