@@ -167,20 +167,26 @@ void record_sample(vt_batch *b, hipStream_t s) {
         check(vt::launch_reset_counters(cnt, vt::kCounterWords, s), "reset");
         check(vt::launch_batch_generate(bt, base, n, queue_view(b, 0, cap), b->radiance.as<float>(), pair(0), grid, s),
               "generate");
+        const auto path_rays = [&](const vt::PathQueue &q) {
+            return vt::RayArgs{q.ox, q.oy, q.oz, q.dx, q.dy, q.dz, q.tmin, q.tmax};
+        };
+        const vt::RayArgs srays{sh.ox, sh.oy, sh.oz, sh.dx, sh.dy, sh.dz, sh.tmin, sh.tmax};
+        const vt::ResolveArgs resolve{sh.id, sh.r, sh.g, sh.b, sh.s, b->radiance.as<float>(), nullptr, 1u, 0u, 1u};
+        // The hits of the paths reaching vertex v (v < vertices) and the shadow rays of vertex v - 1 (v > 0).
+        const auto trace = [&](const vt::PathQueue &q, int v) {
+            check(vt::launch_trace_vertex_batch(jt, q.job, path_rays(q), hits, v < vertices ? pair(v) : nullptr, sh.job, srays,
+                                                b->occluded.as<uint8_t>(), v > 0 ? pair(v) + 1 : nullptr, resolve, n,
+                                                b->tree_depth, b->tuning.trace_block, tgrid, s),
+                  "trace");
+        };
         int cur = 0;
+        trace(queue_view(b, 0, cap), 0);
         for (int v = 0; v < vertices; ++v) {
-            const uint32_t *cin = pair(v), *csh = pair(v + 1) + 1;
             const vt::PathQueue qin = queue_view(b, cur, cap), qout = queue_view(b, 1 - cur, cap);
-            const vt::RayArgs rays{qin.ox, qin.oy, qin.oz, qin.dx, qin.dy, qin.dz, qin.tmin, qin.tmax};
-            check(vt::launch_trace_batch(jt, qin.job, rays, hits, nullptr, n, false, cin, b->tree_depth,
-                                         b->tuning.trace_block, tgrid, s), "extend");
-            check(vt::launch_batch_shade(bt, qin, hits, qout, sh, vt::Counters{cin, reinterpret_cast<unsigned long long *>(pair(v + 1))}, n, b->radiance.as<float>(),
-                                         b->layered, s), "shade");
-            const vt::RayArgs srays{sh.ox, sh.oy, sh.oz, sh.dx, sh.dy, sh.dz, sh.tmin, sh.tmax};
-            check(vt::launch_trace_batch(jt, sh.job, srays, vt::HitArgs{}, b->occluded.as<uint8_t>(), n, true, csh,
-                                         b->tree_depth, b->tuning.trace_block, tgrid, s), "shadow");
-            check(vt::launch_batch_resolve(sh, b->occluded.as<uint8_t>(), csh, n, b->radiance.as<float>(), grid, s),
-                  "resolve");
+            check(vt::launch_batch_shade(bt, qin, hits, qout, sh,
+                                         vt::Counters{pair(v), reinterpret_cast<unsigned long long *>(pair(v + 1))}, n,
+                                         b->radiance.as<float>(), b->layered, s), "shade");
+            trace(qout, v + 1);
             cur = 1 - cur;
         }
         check(vt::launch_batch_accumulate(bt, base, n, b->radiance.as<float>(), b->accum.as<float>(), grid, s),

@@ -12,6 +12,7 @@
 #include <stdint.h>
 
 #include "render_kernels.h"
+#include "resolve.h"
 #include "zsampler.h"
 #include "traverse8.h"
 
@@ -25,12 +26,7 @@ constexpr float kTwoPi = 6.28318530717958647692f;
 constexpr int kIcdfSegments = 1024;
 constexpr int kSamples = 471;
 
-// ---------------------------------------------------------------- RNG (main.swift:91-117)
-__device__ __forceinline__ uint32_t pcg_hash(uint32_t input) {
-    uint32_t state = input * 747796405u + 2891336453u;
-    uint32_t word = ((state >> ((state >> 28u) + 4u)) ^ state) * 277803737u;
-    return (word >> 22u) ^ word;
-}
+// ---------------------------------------------------------------- RNG (main.swift:91-117; pcg_hash: resolve.h)
 __device__ __forceinline__ float rand_f(uint32_t &seed) {
     seed = pcg_hash(seed);
     return (float)(seed >> 8u) * (1.0f / 16777216.0f);
@@ -1071,10 +1067,8 @@ constexpr uint32_t kRecorded = 1u << 20;
 constexpr uint32_t kGiSecondary = 1u << 21;
 
 // ---------------------------------------------------------------- learned radiance cache
-// Training paths: 1 in f.train_period, by a hash of pixel and sample index.
 __device__ __forceinline__ bool nrc_training(const FrameArgs &f, uint32_t id) {
-    const uint32_t smp = id / f.npix, pix = id - smp * f.npix;
-    return pcg_hash((pix * 0x9E3779B9u) ^ ((f.sample_index0 + smp) * 0x85EBCA6Bu)) % f.train_period == 0u;
+    return nrc_training_path(f.npix, f.sample_index0, f.train_period, id);
 }
 // The 11 cache inputs of a vertex: position in the scene box, direction toward the previous vertex,
 // shading normal (both mapped to [0, 1]), roughness (1 for Lambert), wavelength number.
@@ -1859,22 +1853,6 @@ __global__ __launch_bounds__(kShadeBlock) void shade_lean_kernel(
                              0u, append);
 }
 
-__global__ __launch_bounds__(256) void resolve_kernel(FrameArgs f, ShadowQueue sh, const uint8_t *occluded,
-                                                      const uint32_t *count, uint32_t capacity, float *radiance,
-                                                      NrcArgs nrc) {
-    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= min(*count, capacity)) return;
-    if (occluded[i]) return;
-    const uint32_t id = sh.id[i];
-    radiance[3 * (size_t)id] += sh.r[i];
-    radiance[3 * (size_t)id + 1] += sh.g[i];
-    radiance[3 * (size_t)id + 2] += sh.b[i];
-    if (f.nrc && nrc_training(f, id)) {
-        const float4 v = sh.s[i];
-        add_f4(nrc.sacc + id, S4{{v.x, v.y, v.z, v.w}});
-    }
-}
-
 // radiance[id] += rgb(thr * max(y, 0) / unit) for every cache query (its answer y at the path's lanes).
 __global__ __launch_bounds__(256) void cache_resolve_kernel(RenderScene sc, NrcArgs nrc, uint32_t capacity, float *radiance) {
     const uint32_t q = blockIdx.x * 256 + threadIdx.x;
@@ -2027,18 +2005,6 @@ __global__ __launch_bounds__(kShadeBlock) void batch_shade_kernel(BatchTables bt
                                 radiance, RestirArgs{}, NrcArgs{}, i, active, j, append);
 }
 
-__global__ __launch_bounds__(256) void batch_resolve_kernel(ShadowQueue sh, const uint8_t *occluded, const uint32_t *count,
-                                                            uint32_t capacity, float *radiance) {
-    const uint32_t n = min(*count, capacity), stride = gridDim.x * 256;
-    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += stride) {
-        if (occluded[i]) continue;
-        const uint32_t id = sh.id[i];
-        radiance[3 * (size_t)id] += sh.r[i];
-        radiance[3 * (size_t)id + 1] += sh.g[i];
-        radiance[3 * (size_t)id + 2] += sh.b[i];
-    }
-}
-
 // accum[g] (rgba32f, one pixel per work item) folds in the chunk's radiance as sample *frame_count + 1.
 __global__ __launch_bounds__(256) void batch_accumulate_kernel(BatchTables bt, uint32_t chunk_base, uint32_t chunk_n,
                                                                const float *radiance, float *accum) {
@@ -2157,13 +2123,6 @@ hipError_t launch_restir_gi_resolve(const FrameArgs &f, const RestirArgs &ra, fl
     return hipGetLastError();
 }
 
-hipError_t launch_resolve(const FrameArgs &f, const ShadowQueue &sh, const uint8_t *occluded, const uint32_t *count,
-                          uint32_t capacity, float *radiance, const NrcArgs &nrc, hipStream_t s) {
-    hipLaunchKernelGGL(resolve_kernel, dim3((capacity + 255) / 256), dim3(256), 0, s, f, sh, occluded, count, capacity,
-                       radiance, nrc);
-    return hipGetLastError();
-}
-
 hipError_t launch_cache_resolve(const RenderScene &sc, const NrcArgs &nrc, uint32_t capacity, float *radiance,
                                 hipStream_t s) {
     hipLaunchKernelGGL(cache_resolve_kernel, dim3((capacity + 255) / 256), dim3(256), 0, s, sc, nrc, capacity, radiance);
@@ -2217,12 +2176,6 @@ hipError_t launch_batch_shade(const BatchTables &bt, const PathQueue &in, const 
         hipLaunchKernelGGL((batch_shade_kernel<true>), dim3(grid), dim3(256), 0, s, bt, in, hits, out, sh, c, capacity, radiance);
     else
         hipLaunchKernelGGL((batch_shade_kernel<false>), dim3(grid), dim3(256), 0, s, bt, in, hits, out, sh, c, capacity, radiance);
-    return hipGetLastError();
-}
-
-hipError_t launch_batch_resolve(const ShadowQueue &sh, const uint8_t *occluded, const uint32_t *count, uint32_t capacity,
-                                float *radiance, uint32_t grid, hipStream_t s) {
-    hipLaunchKernelGGL(batch_resolve_kernel, dim3(grid), dim3(256), 0, s, sh, occluded, count, capacity, radiance);
     return hipGetLastError();
 }
 

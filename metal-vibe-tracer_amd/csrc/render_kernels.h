@@ -1,9 +1,9 @@
 // render_kernels.h -- device data of the wavefront path tracer and its launch interface.
 //
-// The frame runs as a wavefront: generate (camera rays) -> [extend (closest hit) -> shade
-// (emission with MIS, next-event sample, Russian roulette, BSDF sample, compaction of surviving
-// paths) -> shadow (any hit) -> resolve (add unoccluded next-event contributions)] per bounce ->
-// accumulate.  Every queue is structure-of-arrays and compacted with one atomic per wavefront.
+// The frame runs as a wavefront: generate (camera rays) -> extend (closest hit) -> [shade (emission with
+// MIS, next-event sample, Russian roulette, BSDF sample, compaction of surviving paths) -> trace (the
+// survivors' closest hits, the shadow rays' any hits, and the contributions of those unoccluded)] per
+// vertex -> accumulate.  Every queue is structure-of-arrays and compacted with one atomic per block.
 #pragma once
 #include <hip/hip_runtime_api.h>
 #include <stdint.h>
@@ -221,8 +221,6 @@ hipError_t launch_restir_gi_resolve(const FrameArgs &f, const RestirArgs &ra, fl
 hipError_t launch_shade_restir(const RenderScene &sc, const FrameArgs &f, const PathQueue &in, const HitArgs &hits,
                                const PathQueue &out, const ShadowQueue &sh, const Counters &c, uint32_t capacity,
                                float *radiance, const RestirArgs &ra, const NrcArgs &nrc, hipStream_t s);
-hipError_t launch_resolve(const FrameArgs &f, const ShadowQueue &sh, const uint8_t *occluded, const uint32_t *count,
-                          uint32_t capacity, float *radiance, const NrcArgs &nrc, hipStream_t s);
 // Adds each cache query's answer: radiance[id] += rgb(thr * max(y, 0)) at the path's wavelengths.
 hipError_t launch_cache_resolve(const RenderScene &sc, const NrcArgs &nrc, uint32_t capacity, float *radiance,
                                 hipStream_t s);
@@ -246,8 +244,6 @@ hipError_t launch_batch_generate(const BatchTables &bt, uint32_t chunk_base, uin
 hipError_t launch_batch_shade(const BatchTables &bt, const PathQueue &in, const HitArgs &hits, const PathQueue &out,
                               const ShadowQueue &sh, const Counters &c, uint32_t capacity, float *radiance, bool layered,
                               hipStream_t s);
-hipError_t launch_batch_resolve(const ShadowQueue &sh, const uint8_t *occluded, const uint32_t *count, uint32_t capacity,
-                                float *radiance, uint32_t grid, hipStream_t s);
 hipError_t launch_batch_accumulate(const BatchTables &bt, uint32_t chunk_base, uint32_t chunk_n, const float *radiance,
                                    float *accum, uint32_t grid, hipStream_t s);
 hipError_t launch_batch_advance(const BatchTables &bt, hipStream_t s);

@@ -787,17 +787,21 @@ static vt_status render_frame(vt_renderer *r, vt_scene *scene, const vt_frame_pa
             // scene, keep extending (checking the live count every 8 vertices) until no path is left.
             const int base = f.scattering_limit + 1 + (f.sampling_mode == 3u ? 1 : 0);
             const int cap = scene->has_delta ? (int)vt::kMaxVertices : base;
+            const auto path_rays = [&](const vt::PathQueue &q) {
+                return vt::RayArgs{q.ox, q.oy, q.oz, q.dx, q.dy, q.dz, q.tmin, q.tmax};
+            };
+            const vt::ResolveArgs resolve{sh.id, sh.r, sh.g, sh.b, sh.s, r->radiance.as<float>(),
+                                          use_cache ? na.sacc : nullptr, f.npix, f.sample_index0, f.train_period};
+            check(vt::launch_trace(scene->view, path_rays(r->q[0].view(r->capacity)), hits, nullptr, n, false, nullptr, s, pair(0)),
+                  "extend");
             for (int b = 0; b < cap; ++b) {
                 if (b >= base && (b - base) % 8 == 0) {
                     check(hipMemcpyAsync(r->host_count, pair(b), 4, hipMemcpyDeviceToHost, s), "hipMemcpyAsync");
                     check(hipStreamSynchronize(s), "hipStreamSynchronize");
                     if (*r->host_count == 0) break;
                 }
-                const uint32_t *cin = pair(b), *csh = pair(b + 1) + 1;
                 const vt::PathQueue qin = r->q[cur].view(r->capacity), qout = r->q[1 - cur].view(r->capacity);
-                vt::RayArgs rays{qin.ox, qin.oy, qin.oz, qin.dx, qin.dy, qin.dz, qin.tmin, qin.tmax};
-                check(vt::launch_trace(scene->view, rays, hits, nullptr, n, false, nullptr, s, cin), "extend");
-                const vt::Counters c{cin, reinterpret_cast<unsigned long long *>(pair(b + 1))};
+                const vt::Counters c{pair(b), reinterpret_cast<unsigned long long *>(pair(b + 1))};
                 if (restir && b == 0) {
                     check(vt::launch_restir_initial(sc, f, qin, hits, ra, s), "restir pass 1");
                     if (gi) {
@@ -824,10 +828,11 @@ static vt_status render_frame(vt_renderer *r, vt_scene *scene, const vt_frame_pa
                 } else {
                     check(vt::launch_shade(sc, f, qin, hits, qout, sh, c, n, r->radiance.as<float>(), na, s), "shade");
                 }
-                vt::RayArgs srays{sh.ox, sh.oy, sh.oz, sh.dx, sh.dy, sh.dz, sh.tmin, sh.tmax};
-                check(vt::launch_trace(scene->view, srays, vt::HitArgs{}, r->occluded.as<uint8_t>(), n, true, nullptr, s, csh),
-                      "shadow");
-                check(vt::launch_resolve(f, sh, r->occluded.as<uint8_t>(), csh, n, r->radiance.as<float>(), na, s), "resolve");
+                // The next vertex's hits, and this vertex's shadow rays with their contributions.
+                const vt::RayArgs srays{sh.ox, sh.oy, sh.oz, sh.dx, sh.dy, sh.dz, sh.tmin, sh.tmax};
+                check(vt::launch_trace_vertex(scene->view, path_rays(qout), hits, b + 1 < cap ? pair(b + 1) : nullptr, srays,
+                                              r->occluded.as<uint8_t>(), pair(b + 1) + 1, resolve, n, s),
+                      "trace");
                 if (restir && b == 0 && gi) {
                     // The spatial reuse's x1 -> x2 connections.
                     const vt::GiWork &w = ra.gw;

@@ -9,6 +9,7 @@
 
 #include <mutex>
 
+#include "resolve.h"
 #include "trace_kernels.h"
 #include "traverse8.h"
 
@@ -267,30 +268,42 @@ __device__ __forceinline__ void wave_triangles(const Source &src, const typename
     wave_lds_order();
 }
 
-template <bool ANY, int kStack, int kBlk, class Source>
+// LDS of a block of the persistent kernels, kHits: with room for closest hits.  Each lane's part is its
+// own wave's, but for `next`: the batches drawn so far from the block's share of each of two queues.
+template <int kStack, int kBlk, bool kHits>
+struct RefillLds {
+    uint32_t stack_base[kStack][kBlk];
+    uint16_t stack_bits[kStack][kBlk];
+    unsigned long long tri_key[kBlk];
+    float tri_hit[kHits ? 3 : 1][kBlk];
+    F4 woop[kBlk];
+    uint32_t next[2];
+};
+// The rays are dealt out in units of a few batches of 64, a unit to each block in turn, so cheap and dear
+// regions of an image are spread over the blocks (against one contiguous range per block: 10 M terrain
+// bounce rays 681 -> 640 us, field shadow rays 213 -> 189 us) and a launch of few rays over the CUs.
+// (Renumbering the blocks so that each XCD's share is contiguous lost it all again: the XCDs' shares
+// are uneven, and their L2s hold the same upper tree anyway.)
+struct Deal {
+    uint32_t batches, shift;  // unit = 1 << shift: a batch per wave of the block, fewer when the rays are few
+    __device__ __forceinline__ Deal(uint32_t n, uint32_t waves) : batches(n / 64u + (n % 64u != 0u)), shift(0) {
+        while ((2u << shift) <= waves && (2u << shift) <= batches / gridDim.x) ++shift;
+    }
+    // The block's draw-th batch; none from `batches` on.
+    __device__ __forceinline__ uint32_t batch(uint32_t draw) const {
+        return ((blockIdx.x + (draw >> shift) * gridDim.x) << shift) + (draw & ((1u << shift) - 1u));
+    }
+};
+
+// Traces the block's share of n rays; `next` is zero when the block's first wave gets here.
+template <bool ANY, int kStack, int kBlk, class Source, class Lds>
 __device__ __forceinline__ void refill_trace(const Source &src, const RayArgs &rays, const HitArgs &hits,
-                                             uint8_t *__restrict__ occluded, uint32_t n) {
-    __shared__ uint32_t stack_base[kStack][kBlk];
-    __shared__ uint16_t stack_bits[kStack][kBlk];
-    __shared__ uint32_t next;
-    __shared__ unsigned long long tri_key[kBlk];
-    __shared__ float tri_hit[ANY ? 1 : 3][kBlk];
-    __shared__ F4 woop[kBlk];
+                                             uint8_t *__restrict__ occluded, uint32_t n, Lds &lds, uint32_t &next) {
     constexpr uint32_t kNone = 0xffffffffu;
-    // The rays are dealt out in units of a few batches of 64, a unit to each block in turn, so cheap and dear
-    // regions of an image are spread over the blocks (against one contiguous range per block: 10 M terrain
-    // bounce rays 681 -> 640 us, field shadow rays 213 -> 189 us) and a launch of few rays over the CUs.
-    // (Renumbering the blocks so that each XCD's share is contiguous lost it all again: the XCDs' shares
-    // are uneven, and their L2s hold the same upper tree anyway.)
-    const uint32_t batches = n / 64u + (n % 64u != 0u), blocks = gridDim.x;
-    constexpr uint32_t kWaves = kBlk / 64;
-    uint32_t shift = 0;  // unit = 1 << shift: a batch per wave of the block, fewer when the rays are few
-    while ((2u << shift) <= kWaves && (2u << shift) <= batches / blocks) ++shift;
-    if (threadIdx.x == 0) next = 0;
-    __syncthreads();
+    const Deal deal(n, kBlk / 64);
     const uint32_t lane = threadIdx.x & 63u;
     const unsigned long long below = (1ull << lane) - 1ull;
-    LdsStack<kStack, kBlk> st{stack_base, stack_bits, (int)threadIdx.x, 0, kStack};
+    LdsStack<kStack, kBlk> st{lds.stack_base, lds.stack_bits, (int)threadIdx.x, 0, kStack};
     TravState ts;
     typename Source::Lane sl{};
     uint32_t ray = kNone;
@@ -314,8 +327,8 @@ __device__ __forceinline__ void refill_trace(const Source &src, const RayArgs &r
                 uint32_t draw = 0;
                 if (lane == 0) draw = atomicAdd(&next, 1u);
                 draw = __builtin_amdgcn_readfirstlane(draw);
-                const uint32_t at = ((blockIdx.x + (draw >> shift) * blocks) << shift) + (draw & ((1u << shift) - 1u));
-                exhausted = at >= batches;
+                const uint32_t at = deal.batch(draw);
+                exhausted = at >= deal.batches;
                 const uint32_t fresh = exhausted ? n : at * 64u;
                 if (rank >= avail) idx = fresh + (rank - avail);
                 batch = fresh;
@@ -329,7 +342,7 @@ __device__ __forceinline__ void refill_trace(const Source &src, const RayArgs &r
                 if (src.begin(idx, sl)) {
                     ray = idx;
                     trav_init(ts, r, src.root(sl));
-                    woop[threadIdx.x] = pack_woop(woop_ray(r.dx, r.dy, r.dz));
+                    lds.woop[threadIdx.x] = pack_woop(woop_ray(r.dx, r.dy, r.dz));
                     st.sp = 0;
                     st.cap = src.stack_cap(sl, kStack);
                     done = !(r.tmax == r.tmax);  // nothing is nearer than a NaN
@@ -356,7 +369,7 @@ __device__ __forceinline__ void refill_trace(const Source &src, const RayArgs &r
         if (4u * (uint32_t)__popcll(waiting) >= (uint32_t)__popcll(live)) {
             uint32_t pre, total;
             wave_prefix(__popc(trimask), below, pre, total);
-            wave_triangles<ANY, kBlk>(src, sl, ts, trimask, tri_base, tri_bits, lane, pre, total, woop, tri_key, tri_hit);
+            wave_triangles<ANY, kBlk>(src, sl, ts, trimask, tri_base, tri_bits, lane, pre, total, lds.woop, lds.tri_key, lds.tri_hit);
             trimask = 0u;
         }
         if (busy && ((done && trimask == 0u) || (ANY && ts.res.occluded))) {
@@ -369,8 +382,8 @@ __device__ __forceinline__ void refill_trace(const Source &src, const RayArgs &r
             } else {
                 const bool hit = ts.res.face >= 0;
                 hits.t[ray] = ts.res.t;
-                hits.b1[ray] = hit ? tri_hit[1][threadIdx.x] : 0.0f;
-                hits.b2[ray] = hit ? tri_hit[2][threadIdx.x] : 0.0f;
+                hits.b1[ray] = hit ? lds.tri_hit[1][threadIdx.x] : 0.0f;
+                hits.b2[ray] = hit ? lds.tri_hit[2][threadIdx.x] : 0.0f;
                 hits.face[ray] = ts.res.face;
                 if (hits.instance) hits.instance[ray] = 0u;
             }
@@ -399,9 +412,51 @@ template <bool ANY, int kStack>
 __global__ __launch_bounds__(refill_block<kStack>(), (refill_waves<ANY, kStack>())) void trace_refill_kernel(
     const U4 *__restrict__ nodes, const F4 *__restrict__ tris, RayArgs rays, HitArgs hits, uint8_t *__restrict__ occluded,
     uint32_t n, const uint32_t *__restrict__ count, float root_max, uint32_t *__restrict__ fault, int cap) {
+    constexpr int kBlk = refill_block<kStack>();
+    __shared__ RefillLds<kStack, kBlk, !ANY> lds;
+    if (threadIdx.x == 0) lds.next[0] = 0;
+    __syncthreads();
     if (count) n = min(n, *count);
-    refill_trace<ANY, kStack, refill_block<kStack>()>(OneScene{nodes, tris, root_max, fault, cap}, rays, hits, occluded,
-                                                      n);
+    refill_trace<ANY, kStack, kBlk>(OneScene{nodes, tris, root_max, fault, cap}, rays, hits, occluded, n, lds, lds.next[0]);
+}
+
+// One wavefront vertex in one launch: each wave traces its part of the continuation rays, goes on with its
+// part of the shadow rays while the block's other waves still finish theirs, and once the block's
+// shadow rays are known, the block adds the contributions of those that see their light -- the rays it
+// traced, in queue order, so the reads are coalesced.  As three launches a vertex (closest, any,
+// resolve) a 320 x 180 preview of 4 vertices took 233 us, as one 204, an OpenPBR frame of 8 vertices 3.41
+// ms, now 2.98.
+template <int kStack, int kBlk, class PathSource, class ShadowSource, class Lds>
+__device__ __forceinline__ void trace_vertex(const PathSource &psrc, const RayArgs &rays, const HitArgs &hits, uint32_t paths,
+                                             const ShadowSource &ssrc, const RayArgs &shadow, uint8_t *occluded,
+                                             uint32_t shadows, const ResolveArgs &resolve, Lds &lds) {
+    if (threadIdx.x < 2) lds.next[threadIdx.x] = 0;
+    __syncthreads();
+    refill_trace<false, kStack, kBlk>(psrc, rays, hits, nullptr, paths, lds, lds.next[0]);
+    refill_trace<true, kStack, kBlk>(ssrc, shadow, HitArgs{}, occluded, shadows, lds, lds.next[1]);
+    __syncthreads();
+    const Deal deal(shadows, kBlk / 64);
+    for (uint32_t draw = threadIdx.x / 64u;; draw += kBlk / 64) {
+        const uint32_t at = deal.batch(draw);
+        if (at >= deal.batches) break;
+        const uint32_t i = at * 64u + (threadIdx.x & 63u);
+        if (i < shadows && !occluded[i]) resolve_ray(resolve, i);
+    }
+}
+template <int kStack>
+__global__ __launch_bounds__(refill_block<kStack>(), (refill_waves<false, kStack>())) void trace_vertex_kernel(
+    const U4 *__restrict__ nodes, const F4 *__restrict__ tris, RayArgs rays, HitArgs hits, const uint32_t *path_count,
+    RayArgs shadow, uint8_t *occluded, const uint32_t *shadow_count, ResolveArgs resolve, uint32_t n, float root_max,
+    uint32_t *__restrict__ fault, int cap) {
+    constexpr int kBlk = refill_block<kStack>();
+    __shared__ RefillLds<kStack, kBlk, true> lds;
+    const OneScene src{nodes, tris, root_max, fault, cap};
+    trace_vertex<kStack, kBlk>(src, rays, hits, path_count ? min(n, *path_count) : 0u, src, shadow, occluded,
+                               min(n, *shadow_count), resolve, lds);
+}
+__global__ __launch_bounds__(256) void resolve_kernel(ResolveArgs a, const uint8_t *occluded, const uint32_t *count, uint32_t n) {
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i < min(n, *count) && !occluded[i]) resolve_ray(a, i);
 }
 
 // Two-level traversal, one ray per lane (main.swift:1843-1900 mesh_closest, 1902-1983 mesh_occluded,
@@ -606,16 +661,18 @@ __global__ __launch_bounds__(256) void trace_median_kernel(const F4 *__restrict_
     }
 }
 
-// Batched rendering: rays of many scenes in one persistent launch with lane refill.  Ray i belongs to
+// Batched rendering: a vertex's rays of many scenes in one persistent launch.  Ray i of a queue belongs to
 // job job[i], whose scene is job_trace[job[i]]; rays of one job are contiguous in the queues, so a wave
 // rarely spans two scenes.
-template <bool ANY, int kStack, int kBlk>
-__global__ __launch_bounds__(kBlk, (kStack <= 12 && kBlk <= 256 ? 5 : 1)) void batch_trace_kernel(const TraceScene *__restrict__ job_trace,
-                                                           const uint32_t *__restrict__ job, RayArgs rays, HitArgs hits,
-                                                           uint8_t *__restrict__ occluded, uint32_t n,
-                                                           const uint32_t *__restrict__ count) {
-    n = min(n, *count);
-    refill_trace<ANY, kStack, kBlk>(JobScenes{job_trace, job}, rays, hits, occluded, n);
+template <int kStack, int kBlk>
+__global__ __launch_bounds__(kBlk, (kStack <= 12 && kBlk <= 256 ? 5 : 1)) void batch_trace_kernel(
+    const TraceScene *__restrict__ job_trace, const uint32_t *__restrict__ path_job, RayArgs rays, HitArgs hits,
+    const uint32_t *path_count, const uint32_t *__restrict__ shadow_job, RayArgs shadow, uint8_t *occluded,
+    const uint32_t *shadow_count, ResolveArgs resolve, uint32_t n) {
+    __shared__ RefillLds<kStack, kBlk, true> lds;
+    trace_vertex<kStack, kBlk>(JobScenes{job_trace, path_job}, rays, hits, path_count ? min(n, *path_count) : 0u,
+                               JobScenes{job_trace, shadow_job}, shadow, occluded,
+                               shadow_count ? min(n, *shadow_count) : 0u, resolve, lds);
 }
 
 }  // namespace
@@ -724,19 +781,17 @@ hipError_t launch_encode_nodes(void *nodes, uint32_t n, hipStream_t stream) {
     return hipGetLastError();
 }
 
-hipError_t launch_trace_batch(const TraceScene *job_trace, const uint32_t *job, const RayArgs &rays, const HitArgs &hits,
-                              uint8_t *occluded, uint32_t n, bool any, const uint32_t *count, uint32_t max_depth,
-                              uint32_t block, uint32_t grid, hipStream_t stream) {
+hipError_t launch_trace_vertex_batch(const TraceScene *job_trace, const uint32_t *path_job, const RayArgs &rays,
+                                     const HitArgs &hits, const uint32_t *path_count, const uint32_t *shadow_job,
+                                     const RayArgs &shadow, uint8_t *occluded, const uint32_t *shadow_count,
+                                     const ResolveArgs &resolve, uint32_t n, uint32_t max_depth, uint32_t block, uint32_t grid,
+                                     hipStream_t stream) {
     if (n == 0) return hipSuccess;
     const int need = max_depth > 1 ? (int)max_depth - 1 : 1;
     if (need > 24 || (block != 64 && block != 128 && block != 256 && block != 512) || grid == 0) return hipErrorInvalidValue;
 #define VT_BATCH(S, B)                                                                                                 \
-    do {                                                                                                               \
-        if (any) hipLaunchKernelGGL((batch_trace_kernel<true, S, B>), dim3(grid), dim3(B), 0, stream, job_trace, job,   \
-                                    rays, hits, occluded, n, count);                                                   \
-        else hipLaunchKernelGGL((batch_trace_kernel<false, S, B>), dim3(grid), dim3(B), 0, stream, job_trace, job,      \
-                                rays, hits, occluded, n, count);                                                       \
-    } while (0)
+    hipLaunchKernelGGL((batch_trace_kernel<S, B>), dim3(grid), dim3(B), 0, stream, job_trace, path_job, rays, hits,     \
+                       path_count, shadow_job, shadow, occluded, shadow_count, resolve, n)
 #define VT_BATCH_STACK(S)                                                                                              \
     do {                                                                                                               \
         if (block == 64) VT_BATCH(S, 64);                                                                              \
@@ -750,6 +805,37 @@ hipError_t launch_trace_batch(const TraceScene *job_trace, const uint32_t *job, 
     else VT_BATCH_STACK(24);
 #undef VT_BATCH_STACK
 #undef VT_BATCH
+    return hipGetLastError();
+}
+
+hipError_t launch_trace_vertex(const TraceScene &scene, const RayArgs &rays, const HitArgs &hits, const uint32_t *path_count,
+                               const RayArgs &shadow, uint8_t *occluded, const uint32_t *shadow_count,
+                               const ResolveArgs &resolve, uint32_t n, hipStream_t stream) {
+    if (n == 0) return hipSuccess;
+    const int need = scene.depth > 1 ? (int)scene.depth - 1 : 1;
+    if (scene.node_count == 0 || scene.kind != 0u || need > 24) {
+        // No 8-wide hierarchy: a launch for each part.
+        hipError_t e = path_count ? launch_trace(scene, rays, hits, nullptr, n, false, nullptr, stream, path_count) : hipSuccess;
+        if (e != hipSuccess) return e;
+        e = launch_trace(scene, shadow, HitArgs{}, occluded, n, true, nullptr, stream, shadow_count);
+        if (e != hipSuccess) return e;
+        hipLaunchKernelGGL(resolve_kernel, dim3(n / 256u + (n % 256u != 0u)), dim3(256), 0, stream, resolve, occluded,
+                           shadow_count, n);
+        return hipGetLastError();
+    }
+    const U4 *nd = reinterpret_cast<const U4 *>(scene.nodes);
+    const F4 *tr = reinterpret_cast<const F4 *>(scene.tris);
+    const int cap = scene.stack_cap ? (int)scene.stack_cap : 24;
+#define VT_VERTEX(S)                                                                                                   \
+    hipLaunchKernelGGL((trace_vertex_kernel<S>), dim3(refill_grid((const void *)trace_vertex_kernel<S>, n, refill_block<S>())), \
+                       dim3(refill_block<S>()), 0, stream, nd, tr, rays, hits, path_count, shadow, occluded, shadow_count,     \
+                       resolve, n, scene.root_max, scene.fault, cap < S ? cap : S)
+    if (need <= 8) VT_VERTEX(8);
+    else if (need <= 10) VT_VERTEX(10);
+    else if (need <= 12) VT_VERTEX(12);
+    else if (need <= 16) VT_VERTEX(16);
+    else VT_VERTEX(24);
+#undef VT_VERTEX
     return hipGetLastError();
 }
 

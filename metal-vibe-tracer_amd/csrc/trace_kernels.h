@@ -69,6 +69,23 @@ hipError_t launch_trace(const TraceScene &scene, const RayArgs &rays, const HitA
                         uint32_t n, bool any, unsigned long long *counters, hipStream_t stream,
                         const uint32_t *count = nullptr);
 
+// The contributions of a wavefront's shadow rays (ray i's to path id[i], resolve.h).  sacc is null unless
+// a radiance cache trains on the paths.
+struct ResolveArgs {
+    const uint32_t *id;
+    const float *r, *g, *b;
+    const float4 *s;
+    float *radiance;
+    float4 *sacc;
+    uint32_t npix, sample_index0, train_period;
+};
+// One wavefront vertex's rays in one launch: the closest hits of min(n, *path_count) continuation rays into
+// `hits`, the any hits of min(n, *shadow_count) shadow rays into `occluded`, and the contributions of the
+// shadow rays that see their light (resolve).  path_count null: no continuation rays.
+hipError_t launch_trace_vertex(const TraceScene &scene, const RayArgs &rays, const HitArgs &hits, const uint32_t *path_count,
+                               const RayArgs &shadow, uint8_t *occluded, const uint32_t *shadow_count,
+                               const ResolveArgs &resolve, uint32_t n, hipStream_t stream);
+
 // The counting traversal of launch_trace (counters variant) with its partial counters in the
 // library's static device scratch (kStatsScratchWords u64, 64 pairs) instead of an allocation:
 // zeroes the scratch with a kernel, traces into the caller's hits / occluded, and sums the pairs into
@@ -81,10 +98,13 @@ hipError_t launch_trace_stats_scratch(int device, const TraceScene &scene, const
                                       uint8_t *occluded, uint32_t n, bool any, unsigned long long *out,
                                       hipStream_t stream);
 
-// Batched rendering: ray i traces the scene job_trace[job[i]], for i < min(n, *count), on a
+// launch_trace_vertex of batched rendering: ray i of a queue traces the scene job_trace[job[i]], on a
 // persistent grid of `grid` blocks of `block` (64, 128, 256 or 512) lanes; max_depth is the deepest tree.
-hipError_t launch_trace_batch(const TraceScene *job_trace, const uint32_t *job, const RayArgs &rays, const HitArgs &hits,
-                              uint8_t *occluded, uint32_t n, bool any, const uint32_t *count, uint32_t max_depth,
-                              uint32_t block, uint32_t grid, hipStream_t stream);
+// path_count or shadow_count null: none of those rays.
+hipError_t launch_trace_vertex_batch(const TraceScene *job_trace, const uint32_t *path_job, const RayArgs &rays,
+                                     const HitArgs &hits, const uint32_t *path_count, const uint32_t *shadow_job,
+                                     const RayArgs &shadow, uint8_t *occluded, const uint32_t *shadow_count,
+                                     const ResolveArgs &resolve, uint32_t n, uint32_t max_depth, uint32_t block, uint32_t grid,
+                                     hipStream_t stream);
 
 }  // namespace vt
