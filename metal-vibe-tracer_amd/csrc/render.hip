@@ -1153,6 +1153,40 @@ __global__ __launch_bounds__(256) void generate_kernel(FrameArgs f, PathQueue q,
     generate_path(f, i - s * f.npix, f.sample_index0 + s, q, i, radiance);
 }
 
+// The pixels of ReSTIR's pass 1: the G-buffer and an empty reservoir for a pixel whose camera ray missed or
+// met another than a diffuse surface; the diffuse pixels are listed, block by block in image order, for
+// restir_initial_kernel.
+__global__ __launch_bounds__(256) void restir_gbuffer_kernel(RenderScene sc, FrameArgs f, PathQueue q, HitArgs hits,
+                                                             RestirBuffers cur, uint32_t *list, unsigned long long *count) {
+    __shared__ AppendShared append;
+    const uint32_t pix = blockIdx.x * kShadeBlock + threadIdx.x;
+    bool diffuse = false;
+    if (pix < f.npix) {
+        float4 gpos = make_float4(0.0f, 0.0f, 0.0f, -1.0f);
+        uint2 gnorm = pack_half4(0.0f, 0.0f, 0.0f, -1.0f);
+        const int face = hits.face[pix];
+        if (face >= 0) {
+            const V3 dir = v3(q.dx[pix], q.dy[pix], q.dz[pix]);
+            const Surface s = surface_at(sc, (uint32_t)face, hits.b1[pix], hits.b2[pix], dir);
+            const uint32_t type = material(sc, s.slot).type;
+            diffuse = type == kDiffuse;
+            gpos = make_float4(s.p.x, s.p.y, s.p.z, hits.t[pix]);
+            gnorm = pack_half4(s.n.x, s.n.y, s.n.z, (float)type);
+        }
+        if (!diffuse) {
+            const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            cur.gpos[pix] = gpos;
+            cur.gnorm[pix] = gnorm;
+            cur.posdir[pix] = zero;
+            cur.emitpdf[pix] = zero;
+            cur.weights[pix] = zero;
+        }
+    }
+    uint32_t at[2];
+    block_append(append, 0, count, diffuse, false, at);
+    if (diffuse) list[at[0]] = pix;
+}
+
 // Pass 1 of ReSTIR DI for one sample (restir_temporal_kernel, main.swift:4842-4940): one thread per
 // pixel over the camera wavefront (queue slot = pixel).  Writes the G-buffer and the pixel's
 // reservoir: RIS over ra.candidates light samples on the pixel's un-decorrelated PCG stream
@@ -1160,17 +1194,24 @@ __global__ __launch_bounds__(256) void generate_kernel(FrameArgs f, PathQueue q,
 // (restir_di_merge :4692-4704) and the encode (restir_di_encode :4708-4716).
 // Without the environment the kernel fits 128 registers, 4 waves per SIMD (asked for explicitly: the
 // light-tree walk is latency-bound and a fourth wave is worth more than the few registers it saves).
+//
+// It runs over the list of diffuse pixels that restir_gbuffer_kernel made: only they have reservoirs, and
+// run over the image the kernel, bound by vector issue, had idle lanes for all others (terrain of half
+// Lambert, half GGX faces, 1080p, 32 candidates: 5.03 ms, now 3.51 and 0.11 for the list).
 template <bool kEnv>
 __global__ __launch_bounds__(256, kEnv ? 1 : 4) void restir_initial_kernel(RenderScene sc, FrameArgs fa, PathQueue q,
-                                                                          HitArgs hits, RestirArgs ra) {
+                                                                          HitArgs hits, RestirArgs ra,
+                                                                          const uint32_t *list, const uint32_t *count) {
     const FrameArgs f = frame_env<kEnv>(fa);
     __shared__ LtTop top;
     __shared__ float top_l[kLtTopInner][256], top_r[kLtTopInner][256];
+    if (blockIdx.x * 256 >= *count) return;  // the whole block
     const bool cached = sc.tree_node_count != 0u;
     if (cached && threadIdx.x < (unsigned)kLtTopAll) lt_top_fill(sc, top, threadIdx.x);
     __syncthreads();
-    const uint32_t pix = blockIdx.x * 256 + threadIdx.x;
-    if (pix >= f.npix) return;
+    const uint32_t k = blockIdx.x * 256 + threadIdx.x;
+    if (k >= *count) return;
+    const uint32_t pix = list[k];
     float4 gpos = make_float4(0.0f, 0.0f, 0.0f, -1.0f);
     uint2 gnorm = pack_half4(0.0f, 0.0f, 0.0f, -1.0f);
     float4 posdir = make_float4(0.0f, 0.0f, 0.0f, 0.0f), emitpdf = posdir, weights = posdir;
@@ -2093,11 +2134,14 @@ hipError_t launch_shade_restir(const RenderScene &sc, const FrameArgs &f, const 
 }
 
 hipError_t launch_restir_initial(const RenderScene &sc, const FrameArgs &f, const PathQueue &q, const HitArgs &hits,
-                                 const RestirArgs &ra, hipStream_t s) {
+                                 const RestirArgs &ra, uint32_t *list, uint32_t *count, hipStream_t s) {
+    const dim3 grid((f.npix + 255) / 256);
+    hipLaunchKernelGGL(restir_gbuffer_kernel, grid, dim3(kShadeBlock), 0, s, sc, f, q, hits, ra.cur, list,
+                       reinterpret_cast<unsigned long long *>(count));
     if (frame_has_env(sc, f))
-        hipLaunchKernelGGL(restir_initial_kernel<true>, dim3((f.npix + 255) / 256), dim3(256), 0, s, sc, f, q, hits, ra);
+        hipLaunchKernelGGL(restir_initial_kernel<true>, grid, dim3(256), 0, s, sc, f, q, hits, ra, list, count);
     else
-        hipLaunchKernelGGL(restir_initial_kernel<false>, dim3((f.npix + 255) / 256), dim3(256), 0, s, sc, f, q, hits, ra);
+        hipLaunchKernelGGL(restir_initial_kernel<false>, grid, dim3(256), 0, s, sc, f, q, hits, ra, list, count);
     return hipGetLastError();
 }
 

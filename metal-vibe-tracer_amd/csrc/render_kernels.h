@@ -177,7 +177,7 @@ struct Counters {
     unsigned long long *out;
 };
 // The counters of a wavefront, cleared once at its start: words 0, 1 the cache's queries and records, 2, 3
-// the material classes, then a pair per vertex (at most 255 vertices and the one past them).
+// the material classes, 4, 5 ReSTIR's diffuse pixels, then a pair per vertex (at most 255 vertices and the one past them).
 constexpr uint32_t kCounterPairs = 8, kMaxVertices = 255, kCounterWords = kCounterPairs + 2 * (kMaxVertices + 1);
 
 // Batched rendering: many images (jobs) of many scenes in one wavefront.  A sample's work items are
@@ -202,9 +202,10 @@ hipError_t launch_shade_sorted(const RenderScene &sc, const FrameArgs &f, const 
                                const PathQueue &out, const ShadowQueue &sh, const Counters &c, uint32_t capacity,
                                float *radiance, const NrcArgs &nrc, uint32_t *perm, uint32_t *classes, hipStream_t s);
 // Pass 1 of ReSTIR DI (restir_temporal_kernel): G-buffer, RIS candidates, temporal merge, encode,
-// for the wavefront's single sample (q holds the camera paths in pixel order, hits their hits).
+// for the wavefront's single sample (q holds the camera paths in pixel order, hits their hits).  list: room
+// for npix pixel indices; count: two cleared counter words, 8-byte aligned.
 hipError_t launch_restir_initial(const RenderScene &sc, const FrameArgs &f, const PathQueue &q, const HitArgs &hits,
-                                 const RestirArgs &ra, hipStream_t s);
+                                 const RestirArgs &ra, uint32_t *list, uint32_t *count, hipStream_t s);
 // ReSTIR GI after pass 1: the x1 -> x2 rays (ra.gw); once they are traced, the light sample at each
 // diffuse x2 and its shadow ray (stage 2); then, with the shadow rays traced, the initial reservoir,
 // the temporal merge and the encode into ra.gcur.
