@@ -286,10 +286,10 @@ typedef struct vt_frame_params {
                                    2: the same estimator with the cache frozen (no training) */
     uint32_t cache_train_period; /* 0 means 16 */
     float cache_learning_rate;   /* 0 means 1e-3 */
-    uint32_t material_sort;      /* 1: at vertices past the first, split the paths by shading class (the
-                                    layered BSDF or not) and shade each class with its own kernel; the
-                                    image is the same.  0 (default) shades every path in one kernel,
-                                    which measured faster on the configurations here */
+    uint32_t material_sort;      /* 1: shade the paths of a vertex in the order of their shading class (the
+                                    layered BSDF or not), so a wave runs one of them; the image is the
+                                    same.  0 (default): only where that is faster, from about 2^16 paths
+                                    in scenes with both classes */
     uint32_t sampler;            /* 0: every pixel draws from its PCG stream (the reference's PCG mode);
                                     1: the Z++ sampler (main.swift:122-305): the pixel's key and each
                                     draw's sampling event as in the reference's Z mode (ReSTIR's light

@@ -177,8 +177,10 @@ struct Counters {
     unsigned long long *out;
 };
 // The counters of a wavefront, cleared once at its start: words 0, 1 the cache's queries and records, 2, 3
-// the material classes, 4, 5 ReSTIR's diffuse pixels, then a pair per vertex (at most 255 vertices and the one past them).
-constexpr uint32_t kCounterPairs = 8, kMaxVertices = 255, kCounterWords = kCounterPairs + 2 * (kMaxVertices + 1);
+// ReSTIR's diffuse pixels, then a pair per vertex (at most 255 vertices and the one past them) and, per
+// vertex, its paths of each material class.
+constexpr uint32_t kCounterPairs = 8, kMaxVertices = 255, kCounterClasses = kCounterPairs + 2 * (kMaxVertices + 1),
+                   kCounterWords = kCounterClasses + 2 * kMaxVertices;
 
 // Batched rendering: many images (jobs) of many scenes in one wavefront.  A sample's work items are
 // the jobs' pixels back to back: item g is pixel g - first[j] of job j, first[j] <= g < first[j + 1],
@@ -193,14 +195,11 @@ struct BatchTables {
 };
 
 hipError_t launch_generate(const FrameArgs &f, const PathQueue &q, float *radiance, uint32_t *count, hipStream_t s);
+// perm (room for capacity slots) not null: the paths are shaded in the order of their shading class; classes:
+// two cleared counter words.
 hipError_t launch_shade(const RenderScene &sc, const FrameArgs &f, const PathQueue &in, const HitArgs &hits,
                         const PathQueue &out, const ShadowQueue &sh, const Counters &c, uint32_t capacity,
-                        float *radiance, const NrcArgs &nrc, hipStream_t s);
-// launch_shade with material sorting: paths are split by whether their hit needs the layered BSDF
-// (perm: capacity slots, classes: 2 zeroed device counters) and each class is shaded by its own kernel.
-hipError_t launch_shade_sorted(const RenderScene &sc, const FrameArgs &f, const PathQueue &in, const HitArgs &hits,
-                               const PathQueue &out, const ShadowQueue &sh, const Counters &c, uint32_t capacity,
-                               float *radiance, const NrcArgs &nrc, uint32_t *perm, uint32_t *classes, hipStream_t s);
+                        float *radiance, const NrcArgs &nrc, uint32_t *perm, uint32_t *classes, hipStream_t s);
 // Pass 1 of ReSTIR DI (restir_temporal_kernel): G-buffer, RIS candidates, temporal merge, encode,
 // for the wavefront's single sample (q holds the camera paths in pixel order, hits their hits).  list: room
 // for npix pixel indices; count: two cleared counter words, 8-byte aligned.
@@ -221,7 +220,8 @@ hipError_t launch_restir_gi_resolve(const FrameArgs &f, const RestirArgs &ra, fl
 // shading with one visibility ray, then the path suffix.
 hipError_t launch_shade_restir(const RenderScene &sc, const FrameArgs &f, const PathQueue &in, const HitArgs &hits,
                                const PathQueue &out, const ShadowQueue &sh, const Counters &c, uint32_t capacity,
-                               float *radiance, const RestirArgs &ra, const NrcArgs &nrc, hipStream_t s);
+                               float *radiance, const RestirArgs &ra, const NrcArgs &nrc, uint32_t *perm,
+                               uint32_t *classes, hipStream_t s);
 // Adds each cache query's answer: radiance[id] += rgb(thr * max(y, 0)) at the path's wavelengths.
 hipError_t launch_cache_resolve(const RenderScene &sc, const NrcArgs &nrc, uint32_t capacity, float *radiance,
                                 hipStream_t s);

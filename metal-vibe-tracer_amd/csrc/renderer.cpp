@@ -787,6 +787,8 @@ static vt_status render_frame(vt_renderer *r, vt_scene *scene, const vt_frame_pa
             // scene, keep extending (checking the live count every 8 vertices) until no path is left.
             const int base = f.scattering_limit + 1 + (f.sampling_mode == 3u ? 1 : 0);
             const int cap = scene->has_delta ? (int)vt::kMaxVertices : base;
+            // Shading in material order pays from about 2^16 paths (classify_kernel).
+            uint32_t *perm = scene->mixed && (p->material_sort || n >= (1u << 16)) ? r->perm.as<uint32_t>() : nullptr;
             const auto path_rays = [&](const vt::PathQueue &q) {
                 return vt::RayArgs{q.ox, q.oy, q.oz, q.dx, q.dy, q.dz, q.tmin, q.tmax};
             };
@@ -803,7 +805,7 @@ static vt_status render_frame(vt_renderer *r, vt_scene *scene, const vt_frame_pa
                 const vt::PathQueue qin = r->q[cur].view(r->capacity), qout = r->q[1 - cur].view(r->capacity);
                 const vt::Counters c{pair(b), reinterpret_cast<unsigned long long *>(pair(b + 1))};
                 if (restir && b == 0) {
-                    check(vt::launch_restir_initial(sc, f, qin, hits, ra, r->perm.as<uint32_t>(), cnt + 4, s), "restir pass 1");
+                    check(vt::launch_restir_initial(sc, f, qin, hits, ra, r->perm.as<uint32_t>(), cnt + 2, s), "restir pass 1");
                     if (gi) {
                         // ReSTIR GI's x1 -> x2 rays, the light samples at x2 and their shadow rays, then
                         // the reservoirs.
@@ -818,15 +820,14 @@ static vt_status render_frame(vt_renderer *r, vt_scene *scene, const vt_frame_pa
                               "restir gi shadow");
                         check(vt::launch_restir_gi_finish(sc, f, qin, hits, ra, s), "restir gi reservoirs");
                     }
-                    check(vt::launch_shade_restir(sc, f, qin, hits, qout, sh, c, n, r->radiance.as<float>(), ra, na, s),
+                    check(vt::launch_shade_restir(sc, f, qin, hits, qout, sh, c, n, r->radiance.as<float>(), ra, na,
+                                                  perm,
+                                           cnt + vt::kCounterClasses + 2 * b, s),
                           "shade");
-                } else if (p->material_sort && scene->mixed) {
-                    // Material sorting (classes counted in counters 2 and 3).
-                    check(vt::launch_reset_counters(cnt + 2, 2, s), "reset");
-                    check(vt::launch_shade_sorted(sc, f, qin, hits, qout, sh, c, n, r->radiance.as<float>(), na,
-                                                  r->perm.as<uint32_t>(), cnt + 2, s), "shade");
                 } else {
-                    check(vt::launch_shade(sc, f, qin, hits, qout, sh, c, n, r->radiance.as<float>(), na, s), "shade");
+                    check(vt::launch_shade(sc, f, qin, hits, qout, sh, c, n, r->radiance.as<float>(), na, perm,
+                                           cnt + vt::kCounterClasses + 2 * b, s),
+                          "shade");
                 }
                 // The next vertex's hits, and this vertex's shadow rays with their contributions.
                 const vt::RayArgs srays{sh.ox, sh.oy, sh.oz, sh.dx, sh.dy, sh.dz, sh.tmin, sh.tmax};

@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 
 import oracle
+import scenes
 import vt
 
 pytestmark = pytest.mark.gpu
@@ -67,3 +68,43 @@ def test_record_counts(gpu_ctx, w, h):
     r.close()
     scene.close()
     cache.close()
+
+
+@pytest.mark.parametrize("w,h", [(1, 1), (16, 16), (257, 1), (64, 32), (2049, 1), (73, 61)])
+@pytest.mark.parametrize("mode", [0, 1])
+def test_material_order_changes_nothing(gpu_ctx, w, h, mode):
+    # Frames below 2^16 paths are shaded in queue order by default, in the order of their shading class on
+    # request: the same image, bit for bit, around the 2048 paths a block lists at a time.
+    mesh, mats = scenes.materials_cornell("opaque")
+    scene = gpu_ctx.set_mesh(mesh)
+    scene.set_materials(scenes.vt_materials(mats))
+    imgs = []
+    for sort in (False, True):
+        r = vt.Renderer(gpu_ctx)
+        r.render(scene, w, h, vt.orbit_eye(), TARGET, 42.0, max_depth=5, samples=2, sample_index=1, sampling_mode=mode,
+                 material_sort=sort)
+        imgs.append(r.readback())
+        r.close()
+    scene.close()
+    print(f"{w}x{h} mode {mode}: mean {imgs[0][..., :3].mean():.6f}", flush=True)
+    assert np.array_equal(imgs[0], imgs[1])
+
+
+@pytest.mark.parametrize("w,h", [(1, 1), (16, 16), (257, 1), (33, 17)])
+def test_restir_lists_every_diffuse_pixel(gpu_ctx, w, h):
+    # ReSTIR's first pass runs over a list of the diffuse pixels: around a block of 256, against the oracle
+    # (up to 5% of the pixels may differ beyond rounding, the materials' ReSTIR parity bar, at least one).
+    mesh, mats = scenes.materials_cornell("opaque")
+    scene = gpu_ctx.set_mesh(mesh)
+    scene.set_materials(scenes.vt_materials(mats))
+    r = vt.Renderer(gpu_ctx)
+    r.render(scene, w, h, vt.orbit_eye(), TARGET, 42.0, max_depth=3, samples=2, sample_index=1, sampling_mode=0,
+             indirect_reuse=1)
+    got = r.readback()[..., :3].astype(np.float64)
+    r.close()
+    scene.close()
+    frame = dict(width=w, height=h, eye=vt.orbit_eye(), target=TARGET, fov=42.0, max_depth=3, indirect_reuse=1)
+    ref = oracle.render_restir(oracle.Scene(mesh.vertices, mesh.faces), mats, frame, 1, 2, candidates=4).reshape(h, w, 3)
+    bad = (~np.isclose(got, ref, rtol=1e-3, atol=1e-4).all(axis=2)).sum()
+    print(f"restir {w}x{h}: {bad} pixels differ", flush=True)
+    assert bad <= max(1, int(0.05 * w * h))
