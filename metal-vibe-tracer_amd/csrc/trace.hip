@@ -29,6 +29,7 @@ struct LdsStack {
     int lane;
     int sp;
     int cap;  // groups the stack may hold: kStack, or less under TraceScene::stack_cap
+    int floor = 0;  // groups below belong to an outer hierarchy
     __device__ __forceinline__ void push(uint32_t b, uint32_t m) {
         base[sp][lane] = b;
         bits[sp][lane] = (uint16_t)m;
@@ -40,7 +41,7 @@ struct LdsStack {
         b = base[sp][lane];
         m = bits[sp][lane];
     }
-    __device__ __forceinline__ bool empty() const { return sp == 0; }
+    __device__ __forceinline__ bool empty() const { return sp == floor; }
 };
 
 template <bool ANY, bool STATS, int kStack>
@@ -160,7 +161,7 @@ __device__ __forceinline__ void wave_lds_order() {
 // numbered by a prefix sum over the lanes' counts and handed out 64 at a time: test j belongs to the
 // lane whose range holds j (binary search over the prefixes) and is its k-th triangle; the worker reads
 // that lane's ray through cross-lane permutes, runs the same Woop test, and folds a hit into the
-// owner's LDS slot with an atomic minimum of (order-preserving t bits << 32 | face) -- the nearest t,
+// owner's LDS slot with an atomic minimum of (order-preserving t bits << 32 | face + 1) -- the nearest t,
 // equal t going to the smaller face, as the one-lane rule.  The winner of each round stores its t and
 // barycentrics; the key's identity picks it since a face is tested at most once per ray.  They stay in the
 // owner's LDS slot until its ray ends, as do its triangle-test constants (woop, packed by pack_woop): both
@@ -192,8 +193,9 @@ __device__ __forceinline__ void wave_triangles(const Source &src, const typename
     const uint32_t wave0 = threadIdx.x & ~63u;
     unsigned long long key0 = 0ull;
     if (cnt) {
-        // No hit yet counts as face 0, so that a hit at exactly tmax is not nearer.
-        if (!ANY) key0 = ((unsigned long long)ord_bits(ts.res.t) << 32) | (uint32_t)max(ts.res.face, 0);
+        // The low word is face + 1: no hit yet counts as 0, below every face, so that a hit at exactly tmax
+        // is not nearer and no test's key equals the starting one.
+        if (!ANY) key0 = ((unsigned long long)ord_bits(ts.res.t) << 32) | ((uint32_t)ts.res.face + 1u);
         key[threadIdx.x] = key0;
     }
     wave_lds_order();
@@ -241,7 +243,7 @@ __device__ __forceinline__ void wave_triangles(const Source &src, const typename
                 if (ANY) {
                     key[wave0 + owner] = 1ull;
                 } else {
-                    mine = ((unsigned long long)ord_bits(t) << 32) | float_to_bits(p0.w);
+                    mine = ((unsigned long long)ord_bits(t) << 32) | (float_to_bits(p0.w) + 1u);
                     atomicMin(&key[wave0 + owner], mine);
                 }
             }
@@ -262,7 +264,7 @@ __device__ __forceinline__ void wave_triangles(const Source &src, const typename
             if (got) ts.res.occluded = true;
         } else if (got != key0) {
             ts.res.t = hit_tb[0][threadIdx.x];
-            ts.res.face = (int32_t)(uint32_t)got;
+            ts.res.face = (int32_t)((uint32_t)got - 1u);
         }
     }
     wave_lds_order();
@@ -459,97 +461,206 @@ __global__ __launch_bounds__(256) void resolve_kernel(ResolveArgs a, const uint8
     if (i < min(n, *count) && !occluded[i]) resolve_ray(a, i);
 }
 
-// Two-level traversal, one ray per lane (main.swift:1843-1900 mesh_closest, 1902-1983 mesh_occluded,
-// software branch).  The instance hierarchy is walked as a one-level one whose leaves name instances,
-// with the boxes grown by enlarge (|origin|max + reach); a leaf's instance traces its asset with the
-// object-space ray, up to the closest hit so far.  Each level keeps its node-group stack in LDS.
-// Both levels run in one loop: each iteration a lane steps either the instance hierarchy or its
-// current instance's asset, so lanes between instances need not wait for another lane's whole asset
-// traversal, as they would with the asset walk nested inside the instance walk.
+// Two-level traversal (main.swift:1843-1900 mesh_closest, 1902-1983 mesh_occluded, software branch), on the
+// persistent kernel's scheme: lanes refill as their rays end and the wave tests triangles together.  The
+// instance hierarchy is walked as a one-level one whose leaves name instances, with the boxes grown by
+// enlarge (|origin|max + reach); a leaf's instance traces its asset with the object-space ray, up to the
+// closest hit so far.  A lane is on one level at a time and both visit nodes in the same instructions.
+// Entering an instance (its record, the ray's transform, six divisions) costs the wave as much as a refill,
+// so lanes wait for it in the same way; while a lane is inside, its place on the instance level rests in
+// LDS: the ray's origin and reciprocals, the next node, the pending group and instances.
 // Ties: the closest-hit rule compares (t, instance, face), so the result does not depend on the order
-// instances are visited in.
-template <bool ANY, int kTop, int kBot>
-__global__ __launch_bounds__(kBlock) void trace_tlas_kernel(TlasScene sc, RayArgs rays, HitArgs hits,
-                                                            uint8_t *__restrict__ occluded, uint32_t n) {
-    __shared__ uint32_t top_base[kTop][kBlock], bot_base[kBot][kBlock];
-    __shared__ uint16_t top_bits[kTop][kBlock], bot_bits[kBot][kBlock];
-    const int lane = threadIdx.x;
-    const uint32_t i = blockIdx.x * kBlock + lane;
-    if (i >= n) return;
-    const TraceRay r{rays.ox[i], rays.oy[i], rays.oz[i], rays.dx[i], rays.dy[i], rays.dz[i], rays.tmin[i], rays.tmax[i]};
-    LdsStack<kTop> top{top_base, top_bits, lane, 0, kTop};
-    LdsStack<kBot> bot{bot_base, bot_bits, lane, 0, kBot};
-    TravState ts, bs;
-    WoopRay bw{};
-    trav_init_e(ts, r, sc.enlarge * (max_abs3(r.ox, r.oy, r.oz) + sc.reach));
-    float bt = r.tmax, bb1 = 0.0f, bb2 = 0.0f;
+// instances are visited in.  At equal t a hit of this instance wins over the current one only if its index
+// is smaller: the current hit's face then counts as the largest number, else as 0.
+//
+// Bound by the node test's instructions, a quarter of them at lanes' different levels, and by entering.
+// 1024 instances of 1280 triangles, 2 M rays, against a ray per lane until its wave's slowest ends and
+// one-lane triangle tests: camera rays 306 -> 243 us, random rays 870 -> 418, any-hit 806 -> 366.  Waiting to
+// enter until half of the live lanes want it took 249 / 437 / 386 us; an eighth 245 / 426 / 377; making the
+// instance level's ray anew on the way back, which fits a fifth wave per SIMD, 262 / 439 / 379.
+constexpr int kTlasBlock = 256;
+struct InstanceTris {
+    static constexpr bool kShared = false;
+    struct Lane {
+        const F4 *tris;
+    };
+    __device__ __forceinline__ const F4 *tri_ptr(const Lane &l) const { return l.tris; }
+};
+// Where a lane left the instance level: next node (kNoTopNode: none), pending group, and the instances of
+// the last leaf still to enter (bits as trav_nodes returns them).
+enum : int { kTopNode, kTopBase, kTopBits, kItems, kItemBase, kItemBits, kTopWords };
+constexpr uint32_t kNoTopNode = 0xffffffffu;
+
+template <bool ANY, int kStack>
+__global__ __launch_bounds__(kTlasBlock, (kStack <= 10 ? 4 : 1)) void trace_tlas_kernel(TlasScene sc, RayArgs rays, HitArgs hits,
+                                                                   uint8_t *__restrict__ occluded, uint32_t n) {
+    __shared__ RefillLds<kStack, kTlasBlock, !ANY> lds;
+    __shared__ float top_ray[6][kTlasBlock];
+    __shared__ uint32_t top[kTopWords][kTlasBlock];
+    if (threadIdx.x == 0) lds.next[0] = 0;
+    __syncthreads();
+    constexpr uint32_t kNone = 0xffffffffu;
+    enum { kTop, kEnter, kMesh };
+    const Deal deal(n, kTlasBlock / 64);
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+    const unsigned long long below = (1ull << lane) - 1ull;
+    LdsStack<kStack, kTlasBlock> st{lds.stack_base, lds.stack_bits, (int)tid, 0, kStack};
+    const InstanceTris src;
+    InstanceTris::Lane sl{};
+    TravState ts;
+    uint32_t ray = kNone, trimask = 0, tri_base = 0, tri_bits = 0;
+    uint32_t cur = 0, binst = 0xffffffffu;  // the instance the lane is in, and its closest hit's
     int32_t bface = -1, sentinel = -1;
-    uint32_t binst = 0xffffffffu, cur = 0u, items = 0u, base = 0u, bits = 0u;
-    bool occ = false, overflow = false, top_done = false, in_asset = false;
-    const U4 *tn = reinterpret_cast<const U4 *>(sc.nodes);
-    const U4 *bn = nullptr;
-    const F4 *btr = nullptr;
+    const U4 *nodes = nullptr;
+    int mode = kTop;
+    bool done = false, overflow = false;  // done: no node left on the lane's level
+    uint32_t batch = 0, used = 64;
+    bool exhausted = false;
     for (;;) {
-        const bool want_top = !in_asset && items == 0u;
-        if (want_top && top_done) break;
-        // The instance hierarchy is stepped once at least a quarter of the wave's remaining lanes wait
-        // for it; until then those lanes idle while the others walk their assets, so lanes that enter
-        // their instances together stay together.  Instanced icosphere field (1024 instances, 2M
-        // rays): camera 0.718 -> 0.664 ms, bounce 1.858 -> 1.229 ms against the nested walk; stepping
-        // for any waiting lane gave 0.794 / 1.454 ms, waiting for half 0.674 / 1.245, three quarters
-        // 0.713 / 1.432.
-        const uint32_t waiting = (uint32_t)__popcll(__ballot(want_top)), live = (uint32_t)__popcll(__ballot(1));
-        if (want_top) {
-            if (4u * waiting >= live) {
-                top_done = trav_nodes<false>(ts, tn, top, items, base, bits);
+        const unsigned long long need = __ballot(ray == kNone);
+        if (!exhausted && __popcll(need) >= kRefillIdle) {
+            const uint32_t cnt = (uint32_t)__popcll(need), rank = (uint32_t)__popcll(need & below);
+            const uint32_t avail = 64u - used;
+            uint32_t idx = batch + used + rank;
+            if (cnt > avail) {
+                uint32_t draw = 0;
+                if (lane == 0) draw = atomicAdd(&lds.next[0], 1u);
+                draw = __builtin_amdgcn_readfirstlane(draw);
+                const uint32_t at = deal.batch(draw);
+                exhausted = at >= deal.batches;
+                const uint32_t fresh = exhausted ? n : at * 64u;
+                if (rank >= avail) idx = fresh + (rank - avail);
+                batch = fresh;
+                used = cnt - avail;
+            } else {
+                used += cnt;
+            }
+            if (ray == kNone && idx < n) {
+                const TraceRay r{rays.ox[idx], rays.oy[idx], rays.oz[idx], rays.dx[idx], rays.dy[idx], rays.dz[idx],
+                                 rays.tmin[idx], rays.tmax[idx]};
+                ray = idx;
+                trav_init_e(ts, r, sc.enlarge * (max_abs3(r.ox, r.oy, r.oz) + sc.reach));
+                top_ray[0][tid] = ts.ox;
+                top_ray[1][tid] = ts.oy;
+                top_ray[2][tid] = ts.oz;
+                top_ray[3][tid] = ts.invx;
+                top_ray[4][tid] = ts.invy;
+                top_ray[5][tid] = ts.invz;
+                st.sp = st.floor = 0;
+                nodes = reinterpret_cast<const U4 *>(sc.nodes);
+                bface = -1;
+                binst = 0xffffffffu;
+                overflow = false;
+                mode = kTop;
+                done = !(r.tmax == r.tmax);  // nothing is nearer than a NaN
+            }
+        }
+        const bool busy = ray != kNone;
+        const unsigned long long live = __ballot(busy);
+        if (!live && exhausted) break;
+        const uint32_t lives = (uint32_t)__popcll(live);
+        // Enter instances, enough lanes at a time, or as soon as no lane can do anything else.
+        const unsigned long long enter = __ballot(busy && mode == kEnter);
+        const unsigned long long steps = __ballot(busy && mode != kEnter && !done && trimask == 0u);
+        if (enter && (__popcll(enter) >= kRefillIdle || 4u * (uint32_t)__popcll(enter) >= lives || !steps)) {
+            if (busy && mode == kEnter) {
+                uint32_t items = top[kItems][tid];
+                const uint32_t b = __builtin_ctz(items);
+                top[kItems][tid] = items & (items - 1u);
+                const InstanceRecord &R = sc.instances[top[kItemBase][tid] + tri_rank(top[kItemBits][tid], b)];
+                const TraceRay r{rays.ox[ray], rays.oy[ray], rays.oz[ray], rays.dx[ray], rays.dy[ray], rays.dz[ray],
+                                 ts.tmin, 0.0f};
+                const TraceRay l = instance_ray(R.local, r, ts.res.t);
+                trav_init(ts, l, R.root_max);
+                lds.woop[tid] = pack_woop(woop_ray(l.dx, l.dy, l.dz));
+                cur = R.index;
+                sentinel = (bface >= 0 && cur < binst) ? 0x7fffffff : -1;
+                ts.res.face = sentinel;
+                nodes = reinterpret_cast<const U4 *>(R.nodes);
+                sl.tris = reinterpret_cast<const F4 *>(R.tris);
+                mode = kMesh;
+                done = R.faces == 0u;
+            }
+        }
+        if (busy && mode != kEnter && !done && trimask == 0u) {
+            uint32_t mask;
+            done = trav_nodes<false>(ts, nodes, st, mask, tri_base, tri_bits);
+            if (mode == kMesh) {
+                trimask = mask;
+            } else if (mask) {
+                top[kTopNode][tid] = done ? kNoTopNode : ts.node;
+                top[kTopBase][tid] = ts.cur_base;
+                top[kTopBits][tid] = ts.cur_bits;
+                top[kItems][tid] = mask;
+                top[kItemBase][tid] = tri_base;
+                top[kItemBits][tid] = tri_bits;
+                st.floor = st.sp;
                 overflow |= ts.res.overflow;
+                mode = kEnter;
+                done = false;
             }
-            continue;
         }
-        if (!in_asset) {
-            const uint32_t b = __builtin_ctz(items);
-            items &= items - 1u;
-            const InstanceRecord &R = sc.instances[base + tri_rank(bits, b)];
-            if (R.faces == 0) continue;
-            const TraceRay lr = instance_ray(R.local, r, bt);
-            trav_init(bs, lr, R.root_max);
-            bw = woop_ray(lr.dx, lr.dy, lr.dz);
-            // Equal t: a hit of this instance wins over the current one only from a smaller index.
-            sentinel = (bface >= 0 && R.index < binst) ? 0x7fffffff : -1;
-            bs.res.face = sentinel;
-            bot.sp = 0;
-            bn = reinterpret_cast<const U4 *>(R.nodes);
-            btr = reinterpret_cast<const F4 *>(R.tris);
-            cur = R.index;
-            in_asset = true;
+        const unsigned long long waiting = __ballot(busy && (done || trimask != 0u));
+        if (4u * (uint32_t)__popcll(waiting) >= lives || (!steps && waiting)) {
+            uint32_t pre, total;
+            wave_prefix(__popc(trimask), below, pre, total);
+            wave_triangles<ANY, kTlasBlock>(src, sl, ts, trimask, tri_base, tri_bits, lane, pre, total, lds.woop, lds.tri_key,
+                                            lds.tri_hit);
+            trimask = 0u;
         }
-        if (trav_step<ANY, false>(bs, bw, bn, btr, bot)) {
-            in_asset = false;
-            overflow |= bs.res.overflow;
-            if (ANY) {
-                if (bs.res.occluded) {
-                    occ = true;
-                    break;
-                }
-            } else if (bs.res.face != sentinel) {
-                bt = bs.res.t;
-                bb1 = bs.res.b1;
-                bb2 = bs.res.b2;
-                bface = bs.res.face;
+        bool end = busy && done && trimask == 0u && mode == kTop;
+        if (busy && mode == kMesh && ((done && trimask == 0u) || (ANY && ts.res.occluded))) {
+            // The instance is done: the next of its leaf, or back to the instance level.
+            if (!ANY && ts.res.face != sentinel) {
+                bface = ts.res.face;
                 binst = cur;
-                ts.res.t = bt;
+            }
+            overflow |= ts.res.overflow;
+            done = false;
+            trimask = 0u;
+            st.sp = st.floor;
+            if (ANY && ts.res.occluded) {
+                end = true;
+            } else if (top[kItems][tid] != 0u) {
+                mode = kEnter;
+            } else if (top[kTopNode][tid] == kNoTopNode) {
+                end = true;
+            } else {
+                mode = kTop;
+                st.floor = 0;
+                nodes = reinterpret_cast<const U4 *>(sc.nodes);
+                ts.node = top[kTopNode][tid];
+                ts.cur_base = top[kTopBase][tid];
+                ts.cur_bits = top[kTopBits][tid];
+                ts.ox = top_ray[0][tid];
+                ts.oy = top_ray[1][tid];
+                ts.oz = top_ray[2][tid];
+                ts.invx = top_ray[3][tid];
+                ts.invy = top_ray[4][tid];
+                ts.invz = top_ray[5][tid];
+                const float e = sc.enlarge * (max_abs3(ts.ox, ts.oy, ts.oz) + sc.reach);
+                ts.ex = e * fabsf(ts.invx);
+                ts.ey = e * fabsf(ts.invy);
+                ts.ez = e * fabsf(ts.invz);
+                ts.oct = (float_to_bits(ts.invx) >> 31) | (float_to_bits(ts.invy) >> 31 << 1) |
+                         (float_to_bits(ts.invz) >> 31 << 2);
+                ts.res.overflow = false;
             }
         }
-    }
-    if (overflow && sc.fault) atomicOr(sc.fault, 1u);
-    if (ANY) {
-        occluded[i] = occ ? 1 : 0;
-    } else {
-        hits.t[i] = bt;
-        hits.b1[i] = bb1;
-        hits.b2[i] = bb2;
-        hits.face[i] = bface;
-        if (hits.instance) hits.instance[i] = binst;
+        if (end) {
+            if ((overflow || ts.res.overflow) && sc.fault) atomicOr(sc.fault, 1u);
+            if (ANY) {
+                occluded[ray] = ts.res.occluded ? 1 : 0;
+            } else {
+                const bool hit = bface >= 0;
+                hits.t[ray] = ts.res.t;
+                hits.b1[ray] = hit ? lds.tri_hit[1][tid] : 0.0f;
+                hits.b2[ray] = hit ? lds.tri_hit[2][tid] : 0.0f;
+                hits.face[ray] = bface;
+                if (hits.instance) hits.instance[ray] = binst;
+            }
+            ray = kNone;
+        }
     }
 }
 
@@ -687,7 +798,7 @@ uint32_t refill_grid(const void *kernel, uint32_t n, int block) {
         const void *k;
         uint32_t blocks;
     };
-    static Entry cache[16] = {};
+    static Entry cache[32] = {};
     static std::mutex lock;
     std::lock_guard<std::mutex> guard(lock);
     uint32_t resident = 0;
@@ -850,19 +961,17 @@ hipError_t launch_trace_tlas(const TlasScene &scene, const RayArgs &rays, const 
     }
     const int top = scene.depth > 1 ? (int)scene.depth - 1 : 1, bot = scene.blas_depth > 1 ? (int)scene.blas_depth - 1 : 1;
     if (top > 16 || bot > 24) return hipErrorInvalidValue;
-    dim3 grid((n + kBlock - 1) / kBlock), block(kBlock);
-#define VT_TLAS(T, B)                                                                                                  \
+    // One stack holds the instance level's pending groups and, above them, those of the mesh a ray is in.
+#define VT_TLAS(S)                                                                                                     \
     do {                                                                                                               \
-        if (any) hipLaunchKernelGGL((trace_tlas_kernel<true, T, B>), grid, block, 0, stream, scene, rays, hits, occluded, n); \
-        else hipLaunchKernelGGL((trace_tlas_kernel<false, T, B>), grid, block, 0, stream, scene, rays, hits, occluded, n); \
+        const uint32_t g = refill_grid(any ? (const void *)trace_tlas_kernel<true, S> : (const void *)trace_tlas_kernel<false, S>, n, kTlasBlock); \
+        if (any) hipLaunchKernelGGL((trace_tlas_kernel<true, S>), dim3(g), dim3(kTlasBlock), 0, stream, scene, rays, hits, occluded, n); \
+        else hipLaunchKernelGGL((trace_tlas_kernel<false, S>), dim3(g), dim3(kTlasBlock), 0, stream, scene, rays, hits, occluded, n); \
     } while (0)
-    if (top <= 8) {
-        if (bot <= 12) VT_TLAS(8, 12);
-        else VT_TLAS(8, 24);
-    } else {
-        if (bot <= 12) VT_TLAS(16, 12);
-        else VT_TLAS(16, 24);
-    }
+    if (top + bot <= 10) VT_TLAS(10);
+    else if (top + bot <= 16) VT_TLAS(16);
+    else if (top + bot <= 24) VT_TLAS(24);
+    else VT_TLAS(40);
 #undef VT_TLAS
     return hipGetLastError();
 }
