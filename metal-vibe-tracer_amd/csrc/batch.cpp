@@ -392,7 +392,7 @@ vt_status vt_batch_readback(vt_batch *b, uint32_t job, float *rgba, size_t bytes
         if (bytes < need) return fail(VT_ERROR_INVALID_ARGUMENT, "rgba buffer too small");
         check(hipSetDevice(b->ctx->device), "hipSetDevice");
         check(hipStreamSynchronize(b->stream), "hipStreamSynchronize");
-        check(hipMemcpy(rgba, b->accum.as<char>() + (size_t)b->first[job] * 16, need, hipMemcpyDeviceToHost), "hipMemcpy");
+        b->ctx->readback.copy(b->ctx->device, rgba, b->accum.as<char>() + (size_t)b->first[job] * 16, need);
         return VT_OK;
     });
 }

@@ -887,7 +887,7 @@ vt_status vt_accum_readback(vt_renderer *r, float *rgba, size_t bytes) {
         if (need == 0) return VT_OK;
         check(hipSetDevice(r->ctx->device), "hipSetDevice");
         check(hipDeviceSynchronize(), "hipDeviceSynchronize");
-        check(hipMemcpy(rgba, r->accum.ptr, need, hipMemcpyDeviceToHost), "hipMemcpy");
+        r->ctx->readback.copy(r->ctx->device, rgba, r->accum.ptr, need);
         return VT_OK;
     });
 }

@@ -9,6 +9,7 @@
 #include <string>
 #include <vector>
 
+#include "readback.h"
 #include "render_kernels.h"
 #include "spectral.h"
 #include "trace_kernels.h"
@@ -69,6 +70,7 @@ struct vt_context {
     bool energy_ready = false;
     // Traversal fault word (TraceScene::fault) of every scene of the context, read by vt_context_check.
     vt::DeviceBuffer fault;
+    vt::ReadbackStage readback;
 };
 
 namespace vt {

@@ -55,7 +55,7 @@ def test_ray_counts(gpu_ctx, n):
     _check(gpu_ctx, [(v, f)], inst, scenes.random_rays(n, n), f"{n} rays")
 
 
-@pytest.mark.parametrize("triangles,instances", [(1, 1), (1, 300), (60, 8), (60, 60), (150, 9), (150, 150), (300, 300)])
+@pytest.mark.parametrize("triangles,instances", [(1, 1), (1, 300), (60, 8), (60, 60), (150, 9), (150, 150), (400, 300)])
 def test_depths(gpu_ctx, triangles, instances):
     # Triangles and instances along geometric series: the surface-area splits peel them off a few at a
     # time, so the hierarchies are as deep as their counts allow.
