@@ -147,7 +147,7 @@ uint32_t persistent_grid(const vt_batch *b, uint32_t block) {
 }
 
 // Records one sample of every job: for each chunk of at most `capacity` pixels, the camera paths,
-// max_depth vertices (extend, shade, shadow, resolve) and the running mean; then the step to the
+// max_depth vertices (shade, then the next vertex's hits and this one's shadow rays) and the running mean; then the step to the
 // next sample.  Every count lives on the device, so the recorded launches replay unchanged.
 void record_sample(vt_batch *b, hipStream_t s) {
     const uint32_t cap = b->tuning.capacity;

@@ -1,8 +1,9 @@
-// bvh8.h -- the 8-wide BVH the gfx950 traversal kernels read, and its host builder.
+// bvh8.h -- the 8-wide BVH of the gfx950 traversal kernels, and its host builder.
 //
-// Layout in HBM (one scene):
-//   nodes:  Node8[node_count], 80 bytes each (five 16-byte words, one dwordx4 load each).  A
-//           node stores its eight child boxes quantised to 8 bits per plane on a per-node grid
+// What the builder makes (one scene):
+//   nodes:  Node8[node_count], 80 bytes each (five 16-byte words), re-encoded on the device in the same
+//           size when the scene is published (traverse8.h).  A node stores its eight child
+//           boxes quantised to 8 bits per plane on a per-node grid
 //           p + q * 2^e (power-of-two scale, so dequantisation fma(q, s, p) rounds once and the
 //           host verifies every dequantised box encloses its child exactly).  Internal children
 //           of a node are contiguous from child_base, in slot order; the leaves' triangles are

@@ -72,6 +72,7 @@ void ReadbackStage::copy(int device, void *dst, const void *src, size_t bytes) {
         // Pinned and device destinations are copied to directly.
         hipPointerAttribute_t attr{};
         const bool known = hipPointerGetAttributes(&attr, dst) == hipSuccess && attr.type != hipMemoryTypeUnregistered;
+        (void)hipGetLastError();  // an address that HIP does not know may be reported as an error
         std::unique_lock<std::mutex> lock(mutex_, std::try_to_lock);
         const bool done = !known && lock.owns_lock() && prepare() &&
                           staged(device, static_cast<char *>(dst), static_cast<const char *>(src), bytes);

@@ -1011,20 +1011,7 @@ __device__ __forceinline__ float gi_target(const Spectral &sp, const Mat &m, con
 }
 __device__ __forceinline__ S4 s4_of(float4 v) { return S4{{v.x, v.y, v.z, v.w}}; }
 
-// ---------------------------------------------------------------- wave-aggregated queue append
-__device__ __forceinline__ uint32_t wave_append(uint32_t *counter, bool pred) {
-    const unsigned long long mask = __ballot(pred);
-    const uint32_t lane = __lane_id();
-    const uint32_t rank = (uint32_t)__popcll(mask & ((1ull << lane) - 1ull));
-    uint32_t base = 0;
-    if (mask) {
-        const int leader = __ffsll((long long)mask) - 1;
-        if ((int)lane == leader) base = atomicAdd(counter, (uint32_t)__popcll(mask));
-        base = __shfl(base, leader);
-    }
-    return base + rank;
-}
-
+// ---------------------------------------------------------------- queue append
 // Queue slots for a whole block at once.  Two queues share one 64-bit counter (low and high word), so a
 // block of four waves makes one atomic for its continuations and shadow rays, and one more for its cache
 // queries and training records (pair p picks the LDS words).  The counters are single words that every

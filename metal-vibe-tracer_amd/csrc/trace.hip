@@ -1,9 +1,9 @@
 // trace.hip -- gfx950 closest-hit and any-hit traversal kernels over SoA ray buffers.
 //
-// One lane per ray, 64-lane wavefronts.  Ray components are read and hits
-// written as separate arrays, so every wavefront access is one coalesced 256-byte line.  The
-// per-ray traversal (traverse8.h) keeps its node-group stack in LDS, laid out [depth][lane] so
-// every lane's push/pop touches its own bank.
+// Persistent grids: a ray belongs to one lane of a 64-lane wavefront, which takes the next ray when its own
+// ends; the wave tests its lanes' triangles together.  Ray components are separate arrays, read a batch of 64
+// consecutive rays at a time.  The per-ray traversal (traverse8.h) keeps its node-group stack in LDS, laid
+// out [depth][lane] so every lane's push/pop touches its own bank.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -44,8 +44,9 @@ struct LdsStack {
     __device__ __forceinline__ bool empty() const { return sp == floor; }
 };
 
-template <bool ANY, bool STATS, int kStack>
-__global__ __launch_bounds__(kBlock) void trace_kernel(const U4 *__restrict__ nodes, const F4 *__restrict__ tris,
+// The counting traversal (node and triangle records a launch fetches): one ray per lane, one-lane triangle tests.
+template <bool ANY, int kStack>
+__global__ __launch_bounds__(kBlock) void count_kernel(const U4 *__restrict__ nodes, const F4 *__restrict__ tris,
                                                        RayArgs rays, HitArgs hits, uint8_t *__restrict__ occluded,
                                                        uint32_t n, const uint32_t *__restrict__ count,
                                                        float root_max, unsigned long long *__restrict__ counters,
@@ -58,7 +59,7 @@ __global__ __launch_bounds__(kBlock) void trace_kernel(const U4 *__restrict__ no
     if (i >= n) return;
     TraceRay r{rays.ox[i], rays.oy[i], rays.oz[i], rays.dx[i], rays.dy[i], rays.dz[i], rays.tmin[i], rays.tmax[i]};
     LdsStack<kStack> st{stack_base, stack_bits, lane, 0, cap};
-    TraceResult res = traverse<ANY, STATS>(nodes, tris, root_max, r, st);
+    TraceResult res = traverse<ANY, true>(nodes, tris, root_max, r, st);
     if (res.overflow && fault) atomicOr(fault, 1u);
     if (ANY) {
         occluded[i] = res.occluded ? 1 : 0;
@@ -69,11 +70,9 @@ __global__ __launch_bounds__(kBlock) void trace_kernel(const U4 *__restrict__ no
         hits.face[i] = res.face;
         if (hits.instance) hits.instance[i] = 0u;
     }
-    if (STATS) {
-        unsigned long long *c = counters + 2 * (blockIdx.x & 63u);
-        atomicAdd(c, (unsigned long long)res.nodes);
-        atomicAdd(c + 1, (unsigned long long)res.tris);
-    }
+    unsigned long long *c = counters + 2 * (blockIdx.x & 63u);
+    atomicAdd(c, (unsigned long long)res.nodes);
+    atomicAdd(c + 1, (unsigned long long)res.tris);
 }
 
 // Persistent traversal with lane refill.  The grid is sized to what the chip holds at once; the waves of a
@@ -81,7 +80,7 @@ __global__ __launch_bounds__(kBlock) void trace_kernel(const U4 *__restrict__ no
 // and a lane whose ray finishes takes the next index at once, so a wave no longer idles until its
 // slowest ray ends.  Node visits are per lane (trav_nodes); the triangles the wave's lanes reach in a
 // step are tested by the whole wave together (wave_triangles).  Per ray the arithmetic, the nodes
-// visited and the result are exactly the one-ray-per-lane kernel's (trav_step).
+// visited and the result are exactly a ray's alone (trav_step).
 // Source: where a ray's scene comes from -- one scene for the launch (OneScene) or the ray's job
 // (JobScenes, batched rendering).
 struct OneScene {
@@ -1006,7 +1005,7 @@ hipError_t launch_trace(const TraceScene &scene, const RayArgs &rays, const HitA
     const int cap = scene.stack_cap ? (int)scene.stack_cap : 24;
     if (!counters) {
         // Persistent refill kernel: as many blocks as the chip holds at once (never more than the rays
-        // need), each draining its own range.
+        // need), each drawing its share of the rays.
 #define VT_REFILL(S)                                                                                                   \
     do {                                                                                                               \
         constexpr int b = refill_block<S>();                                                                          \
@@ -1024,13 +1023,8 @@ hipError_t launch_trace(const TraceScene &scene, const RayArgs &rays, const HitA
     }
 #define VT_LAUNCH(S)                                                                                                   \
     do {                                                                                                               \
-        if (counters) {                                                                                                \
-            if (any) hipLaunchKernelGGL((trace_kernel<true, true, S>), grid, block, 0, stream, nd, tr, rays, hits, occluded, n, count, scene.root_max, counters, scene.fault, cap < S ? cap : S); \
-            else hipLaunchKernelGGL((trace_kernel<false, true, S>), grid, block, 0, stream, nd, tr, rays, hits, occluded, n, count, scene.root_max, counters, scene.fault, cap < S ? cap : S); \
-        } else {                                                                                                       \
-            if (any) hipLaunchKernelGGL((trace_kernel<true, false, S>), grid, block, 0, stream, nd, tr, rays, hits, occluded, n, count, scene.root_max, nullptr, scene.fault, cap < S ? cap : S); \
-            else hipLaunchKernelGGL((trace_kernel<false, false, S>), grid, block, 0, stream, nd, tr, rays, hits, occluded, n, count, scene.root_max, nullptr, scene.fault, cap < S ? cap : S); \
-        }                                                                                                              \
+        if (any) hipLaunchKernelGGL((count_kernel<true, S>), grid, block, 0, stream, nd, tr, rays, hits, occluded, n, count, scene.root_max, counters, scene.fault, cap < S ? cap : S); \
+        else hipLaunchKernelGGL((count_kernel<false, S>), grid, block, 0, stream, nd, tr, rays, hits, occluded, n, count, scene.root_max, counters, scene.fault, cap < S ? cap : S); \
     } while (0)
     if (need <= 8) VT_LAUNCH(8);
     else if (need <= 12) VT_LAUNCH(12);
