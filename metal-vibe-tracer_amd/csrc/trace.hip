@@ -285,14 +285,20 @@ struct RefillLds {
 // bounce rays 681 -> 640 us, field shadow rays 213 -> 189 us) and a launch of few rays over the CUs.
 // (Renumbering the blocks so that each XCD's share is contiguous lost it all again: the XCDs' shares
 // are uneven, and their L2s hold the same upper tree anyway.)
+// Each round of units starts at another block (golden-ratio steps): in an image whose width is a multiple of
+// the unit a block would otherwise stay in one column, and the columns' costs differ (2048 x 1024 camera rays:
+// field 228 -> 178 us, 1024 instances 404 -> 246; 1920 x 1080 unchanged).  Units of a batch per wave take 181
+// and 258 us there and 490 against 465 on the terrain's camera rays, units of one batch 162, 260 and 487.
 struct Deal {
-    uint32_t batches, shift;  // unit = 1 << shift: a batch per wave of the block, fewer when the rays are few
+    uint32_t batches, shift;  // unit = 1 << shift: half the block's waves, fewer when the rays are few
     __device__ __forceinline__ Deal(uint32_t n, uint32_t waves) : batches(n / 64u + (n % 64u != 0u)), shift(0) {
-        while ((2u << shift) <= waves && (2u << shift) <= batches / gridDim.x) ++shift;
+        while ((4u << shift) <= waves && (2u << shift) <= batches / gridDim.x) ++shift;
     }
     // The block's draw-th batch; none from `batches` on.
     __device__ __forceinline__ uint32_t batch(uint32_t draw) const {
-        return ((blockIdx.x + (draw >> shift) * gridDim.x) << shift) + (draw & ((1u << shift) - 1u));
+        const uint32_t round = draw >> shift, at = blockIdx.x + __umulhi(round * 0x9e3779b9u, gridDim.x);
+        const uint32_t unit = round * gridDim.x + (at < gridDim.x ? at : at - gridDim.x);
+        return (unit << shift) + (draw & ((1u << shift) - 1u));
     }
 };
 
