@@ -250,8 +250,9 @@ __device__ __forceinline__ uint32_t tri_rank(uint32_t tv, uint32_t p) { return _
 // testing them after the move gives the same result as testing them first.
 //
 // The kernels are bound by the instructions of this test.  Per child: six fused multiply-adds that read
-// their plane as fp16 in place (v_fma_mix_f32), four min / max, a compare and an add-with-carry that
-// shifts the result into the hit mask; per node: 24 byte permutes that pick the near and far planes by
+// their plane as fp16 in place (v_fma_mix_f32), four min / max, a compare and a select, with half an or, for
+// its bit of the hit mask (left to the compiler, which keeps two wait states between the compare and the
+// instruction that reads its mask, as this hardware wants); per node: 24 byte permutes that pick the near and far planes by
 // the ray's direction signs, and a few words' worth of bit arithmetic for the leaves' triangles and the
 // visiting order.  Converting each byte (48 v_cvt_f32_ubyte), choosing near and far words per axis and
 // handling each child's leaf or inner kind in a branch took about 290 vector and 140 scalar instructions
@@ -291,8 +292,7 @@ __device__ __forceinline__ bool trav_nodes(TravState &st, const U4 *__restrict__
             const float tnz = __builtin_fmaf((float)pnz[c], bz, nz), tfz = __builtin_fmaf((float)pfz[c], bz, fz);
             const float tn = fmaxf(fmaxf(tnx, tny), fmaxf(tnz, st.tmin));
             const float tf = fminf(fminf(tfx, tfy), fminf(tfz, st.res.t));
-            // hit = 2 hit + (tn <= tf)
-            asm("v_cmp_le_f32 vcc, %1, %2\n\tv_addc_co_u32 %0, vcc, %0, %0, vcc" : "+v"(hit) : "v"(tn), "v"(tf) : "vcc");
+            hit |= tn <= tf ? 1u << (2 * k + c) : 0u;
         }
         __builtin_amdgcn_sched_barrier(0);  // a pair of slots at a time: fewer registers, one wave more per SIMD
     }
