@@ -52,6 +52,7 @@ struct vt_batch {
     hipGraphExec_t exec = nullptr;
     bool layered = false;
     uint32_t tree_depth = 1;
+    float root_max = 0.0f;
     // vt_scene::generation of each scene when its views went into the tables: a rebuilt hierarchy or
     // new materials replace the buffers the captured graph reads, so a change re-uploads and recaptures.
     std::vector<uint64_t> scene_generation;
@@ -80,6 +81,7 @@ void upload_tables(vt_batch *b) {
     std::vector<vt::RenderScene> rs;
     b->layered = false;
     b->tree_depth = 1;
+    b->root_max = 0.0f;
     b->scene_generation.clear();
     for (vt_scene *s : b->scenes) {
         b->scene_generation.push_back(s->generation);
@@ -87,6 +89,7 @@ void upload_tables(vt_batch *b) {
         rs.push_back(s->render_view());
         b->layered = b->layered || s->has_layered;
         b->tree_depth = std::max(b->tree_depth, s->view.depth);
+        b->root_max = std::max(b->root_max, s->view.root_max);
     }
     b->scene_table.upload(rs.data(), rs.size() * sizeof(vt::RenderScene));
     std::vector<vt::TraceScene> jt;
@@ -176,7 +179,7 @@ void record_sample(vt_batch *b, hipStream_t s) {
         const auto trace = [&](const vt::PathQueue &q, int v) {
             check(vt::launch_trace_vertex_batch(jt, q.job, path_rays(q), hits, v < vertices ? pair(v) : nullptr, sh.job, srays,
                                                 b->occluded.as<uint8_t>(), v > 0 ? pair(v) + 1 : nullptr, resolve, n,
-                                                b->tree_depth, b->tuning.trace_block, tgrid, s),
+                                                b->tree_depth, b->root_max, b->tuning.trace_block, tgrid, s),
                   "trace");
         };
         int cur = 0;

@@ -112,7 +112,7 @@ static void publish_tree(vt_scene *s, const HostTree &t, const BuildOptions &opt
     s->nodes.upload(t.nodes.data(), t.nodes.size());
     if (t.kind == 0) {
         // Waited for: the first trace may come on any stream.
-        check(launch_encode_nodes(s->nodes.ptr, t.node_count, nullptr), "encode nodes");
+        check(launch_encode_nodes(s->nodes.ptr, t.node_count, t.root_max, nullptr), "encode nodes");
         check(hipStreamSynchronize(nullptr), "hipStreamSynchronize");
     }
     s->tris.upload(t.tris.data(), t.tris.size());

@@ -111,6 +111,7 @@ float round_up(double v) {
 void write_records(vt_tlas *t) {
     std::vector<InstanceRecord> rec(t->leaf_items.size());
     uint32_t blas_depth = 1;
+    float blas_max = 0.0f;
     for (size_t p = 0; p < rec.size(); ++p) {
         const uint32_t k = t->leaf_items[p];
         const vt_scene *s = t->list[k].mesh;
@@ -124,6 +125,7 @@ void write_records(vt_tlas *t) {
         r.index = k;
         r.faces = s->view.node_count ? s->info.face_count : 0u;
         blas_depth = std::max(blas_depth, s->view.depth);
+        blas_max = std::max(blas_max, s->view.root_max);
     }
     check(hipSetDevice(t->ctx->device), "hipSetDevice");
     t->ctx->resident -= t->records.bytes;
@@ -133,6 +135,7 @@ void write_records(vt_tlas *t) {
     t->accounted += t->records.bytes;
     t->view.instances = t->records.as<const InstanceRecord>();
     t->view.blas_depth = blas_depth;
+    t->view.blas_max = blas_max;
     t->info.blas_depth = blas_depth;
     for (size_t a = 0; a < t->assets.size(); ++a) t->asset_generation[a] = t->assets[a]->generation;
 }
@@ -224,8 +227,9 @@ std::unique_ptr<vt_tlas> build_tlas(vt_context *ctx, const vt_instance *list, ui
     const uint64_t bytes = top.nodes.size() * sizeof(Node8) + (uint64_t)count * sizeof(InstanceRecord);
     if (ctx->resident + bytes > ctx->budget) throw BudgetError("The imported meshes exceed the safe GPU memory budget.");
     t->nodes.upload(top.nodes.data(), top.nodes.size() * sizeof(Node8));
-    // Waited for: the first trace may come on any stream.
-    check(launch_encode_nodes(t->nodes.ptr, (uint32_t)top.nodes.size(), nullptr), "encode nodes");
+    // Instances lie within 1e8 (above), so their boxes are unscaled.  Waited for: the first trace may come on
+    // any stream.
+    check(launch_encode_nodes(t->nodes.ptr, (uint32_t)top.nodes.size(), 0.0f, nullptr), "encode nodes");
     check(hipStreamSynchronize(nullptr), "hipStreamSynchronize");
     t->accounted = t->nodes.bytes;
     ctx->resident += t->nodes.bytes;

@@ -59,7 +59,7 @@ __global__ __launch_bounds__(kBlock) void count_kernel(const U4 *__restrict__ no
     if (i >= n) return;
     TraceRay r{rays.ox[i], rays.oy[i], rays.oz[i], rays.dx[i], rays.dy[i], rays.dz[i], rays.tmin[i], rays.tmax[i]};
     LdsStack<kStack> st{stack_base, stack_bits, lane, 0, cap};
-    TraceResult res = traverse<ANY, true>(nodes, tris, root_max, r, st);
+    TraceResult res = traverse<ANY, true>(nodes, tris, root_max, box_scale(root_max), r, st);
     if (res.overflow && fault) atomicOr(fault, 1u);
     if (ANY) {
         occluded[i] = res.occluded ? 1 : 0;
@@ -82,7 +82,9 @@ __global__ __launch_bounds__(kBlock) void count_kernel(const U4 *__restrict__ no
 // step are tested by the whole wave together (wave_triangles).  Per ray the arithmetic, the nodes
 // visited and the result are exactly a ray's alone (trav_step).
 // Source: where a ray's scene comes from -- one scene for the launch (OneScene) or the ray's job
-// (JobScenes, batched rendering).
+// (JobScenes, batched rendering).  kScaled: for hierarchies whose box scale (traverse8.h) is not 1; theirs is
+// a kernel of its own, since the two multiplications a node visit takes for it cost 6 % on shadow rays.
+template <bool kScaled>
 struct OneScene {
     static constexpr bool kShared = true;  // every lane reads the same triangle array
     const U4 *nodes;
@@ -95,9 +97,11 @@ struct OneScene {
     __device__ __forceinline__ const U4 *node_ptr(const Lane &) const { return nodes; }
     __device__ __forceinline__ const F4 *tri_ptr(const Lane &) const { return tris; }
     __device__ __forceinline__ float root(const Lane &) const { return root_max; }
+    __device__ __forceinline__ float scale(const Lane &) const { return kScaled ? box_scale(root_max) : 1.0f; }
     __device__ __forceinline__ uint32_t *fault_word(const Lane &) const { return fault; }
     __device__ __forceinline__ int stack_cap(const Lane &, int k) const { return cap < k ? cap : k; }
 };
+template <bool kScaled>
 struct JobScenes {
     static constexpr bool kShared = false;
     const TraceScene *job_trace;
@@ -122,6 +126,7 @@ struct JobScenes {
     __device__ __forceinline__ const U4 *node_ptr(const Lane &l) const { return l.nodes; }
     __device__ __forceinline__ const F4 *tri_ptr(const Lane &l) const { return l.tris; }
     __device__ __forceinline__ float root(const Lane &l) const { return l.root_max; }
+    __device__ __forceinline__ float scale(const Lane &l) const { return kScaled ? box_scale(l.root_max) : 1.0f; }
     __device__ __forceinline__ uint32_t *fault_word(const Lane &l) const { return l.fault; }
     __device__ __forceinline__ int stack_cap(const Lane &l, int k) const {
         return l.cap && (int)l.cap < k ? (int)l.cap : k;
@@ -348,7 +353,7 @@ __device__ __forceinline__ void refill_trace(const Source &src, const RayArgs &r
                                  rays.tmin[idx], rays.tmax[idx]};
                 if (src.begin(idx, sl)) {
                     ray = idx;
-                    trav_init(ts, r, src.root(sl));
+                    trav_init(ts, r, src.root(sl), src.scale(sl));
                     lds.woop[threadIdx.x] = pack_woop(woop_ray(r.dx, r.dy, r.dz));
                     st.sp = 0;
                     st.cap = src.stack_cap(sl, kStack);
@@ -371,7 +376,7 @@ __device__ __forceinline__ void refill_trace(const Source &src, const RayArgs &r
         // so triangles of several steps are tested together: the wave flushes once a quarter of its
         // live lanes wait (a CPU replay of the benchmark rays: 0.97 -> 0.62 rounds per step on bounce
         // rays, about 11% fewer issue cycles).  Nodes visited and results are unchanged.
-        if (busy && !done && trimask == 0u) done = trav_nodes<false>(ts, src.node_ptr(sl), st, trimask, tri_base, tri_bits);
+        if (busy && !done && trimask == 0u) done = trav_nodes<false>(ts, src.node_ptr(sl), src.scale(sl), st, trimask, tri_base, tri_bits);
         const unsigned long long waiting = __ballot(busy && (done || trimask != 0u));
         if (4u * (uint32_t)__popcll(waiting) >= (uint32_t)__popcll(live)) {
             uint32_t pre, total;
@@ -415,7 +420,7 @@ constexpr int refill_waves() {
     return kStack > 12 ? 1 : ANY || kStack <= 8 ? 6 : 5;  // LDS bounds the deeper stacks
 }
 
-template <bool ANY, int kStack>
+template <bool ANY, int kStack, bool kScaled = false>
 __global__ __launch_bounds__(refill_block<kStack>(), (refill_waves<ANY, kStack>())) void trace_refill_kernel(
     const U4 *__restrict__ nodes, const F4 *__restrict__ tris, RayArgs rays, HitArgs hits, uint8_t *__restrict__ occluded,
     uint32_t n, const uint32_t *__restrict__ count, float root_max, uint32_t *__restrict__ fault, int cap) {
@@ -424,7 +429,7 @@ __global__ __launch_bounds__(refill_block<kStack>(), (refill_waves<ANY, kStack>(
     if (threadIdx.x == 0) lds.next[0] = 0;
     __syncthreads();
     if (count) n = min(n, *count);
-    refill_trace<ANY, kStack, kBlk>(OneScene{nodes, tris, root_max, fault, cap}, rays, hits, occluded, n, lds, lds.next[0]);
+    refill_trace<ANY, kStack, kBlk>(OneScene<kScaled>{nodes, tris, root_max, fault, cap}, rays, hits, occluded, n, lds, lds.next[0]);
 }
 
 // One wavefront vertex in one launch: each wave traces its part of the continuation rays, goes on with its
@@ -457,7 +462,7 @@ __global__ __launch_bounds__(refill_block<kStack>(), (refill_waves<false, kStack
     uint32_t *__restrict__ fault, int cap) {
     constexpr int kBlk = refill_block<kStack>();
     __shared__ RefillLds<kStack, kBlk, true> lds;
-    const OneScene src{nodes, tris, root_max, fault, cap};
+    const OneScene<false> src{nodes, tris, root_max, fault, cap};
     trace_vertex<kStack, kBlk>(src, rays, hits, path_count ? min(n, *path_count) : 0u, src, shadow, occluded,
                                min(n, *shadow_count), resolve, lds);
 }
@@ -496,7 +501,7 @@ struct InstanceTris {
 enum : int { kTopNode, kTopBase, kTopBits, kItems, kItemBase, kItemBits, kTopWords };
 constexpr uint32_t kNoTopNode = 0xffffffffu;
 
-template <bool ANY, int kStack>
+template <bool ANY, int kStack, bool kScaled = false>
 __global__ __launch_bounds__(kTlasBlock, (kStack <= 10 ? 4 : 1)) void trace_tlas_kernel(TlasScene sc, RayArgs rays, HitArgs hits,
                                                                    uint8_t *__restrict__ occluded, uint32_t n) {
     __shared__ RefillLds<kStack, kTlasBlock, !ANY> lds;
@@ -517,6 +522,7 @@ __global__ __launch_bounds__(kTlasBlock, (kStack <= 10 ? 4 : 1)) void trace_tlas
     uint32_t cur = 0, binst = 0xffffffffu;  // the instance the lane is in, and its closest hit's
     int32_t bface = -1, sentinel = -1;
     const U4 *nodes = nullptr;
+    float scale = 1.0f;  // box scale of the lane's level: 1 but in an asset when kScaled (instances lie within 1e8)
     int mode = kTop;
     bool done = false, overflow = false;  // done: no node left on the lane's level
     uint32_t batch = 0, used = 64;
@@ -544,7 +550,7 @@ __global__ __launch_bounds__(kTlasBlock, (kStack <= 10 ? 4 : 1)) void trace_tlas
                 const TraceRay r{rays.ox[idx], rays.oy[idx], rays.oz[idx], rays.dx[idx], rays.dy[idx], rays.dz[idx],
                                  rays.tmin[idx], rays.tmax[idx]};
                 ray = idx;
-                trav_init_e(ts, r, sc.enlarge * (max_abs3(r.ox, r.oy, r.oz) + sc.reach));
+                trav_init_e(ts, r, sc.enlarge * (max_abs3(r.ox, r.oy, r.oz) + sc.reach), 1.0f);
                 top_ray[0][tid] = ts.ox;
                 top_ray[1][tid] = ts.oy;
                 top_ray[2][tid] = ts.oz;
@@ -553,6 +559,7 @@ __global__ __launch_bounds__(kTlasBlock, (kStack <= 10 ? 4 : 1)) void trace_tlas
                 top_ray[5][tid] = ts.invz;
                 st.sp = st.floor = 0;
                 nodes = reinterpret_cast<const U4 *>(sc.nodes);
+                scale = 1.0f;
                 bface = -1;
                 binst = 0xffffffffu;
                 overflow = false;
@@ -576,7 +583,8 @@ __global__ __launch_bounds__(kTlasBlock, (kStack <= 10 ? 4 : 1)) void trace_tlas
                 const TraceRay r{rays.ox[ray], rays.oy[ray], rays.oz[ray], rays.dx[ray], rays.dy[ray], rays.dz[ray],
                                  ts.tmin, 0.0f};
                 const TraceRay l = instance_ray(R.local, r, ts.res.t);
-                trav_init(ts, l, R.root_max);
+                if (kScaled) scale = box_scale(R.root_max);
+                trav_init(ts, l, R.root_max, scale);
                 lds.woop[tid] = pack_woop(woop_ray(l.dx, l.dy, l.dz));
                 cur = R.index;
                 sentinel = (bface >= 0 && cur < binst) ? 0x7fffffff : -1;
@@ -589,7 +597,7 @@ __global__ __launch_bounds__(kTlasBlock, (kStack <= 10 ? 4 : 1)) void trace_tlas
         }
         if (busy && mode != kEnter && !done && trimask == 0u) {
             uint32_t mask;
-            done = trav_nodes<false>(ts, nodes, st, mask, tri_base, tri_bits);
+            done = trav_nodes<false>(ts, nodes, scale, st, mask, tri_base, tri_bits);
             if (mode == kMesh) {
                 trimask = mask;
             } else if (mask) {
@@ -647,6 +655,7 @@ __global__ __launch_bounds__(kTlasBlock, (kStack <= 10 ? 4 : 1)) void trace_tlas
                 ts.ex = e * fabsf(ts.invx);
                 ts.ey = e * fabsf(ts.invy);
                 ts.ez = e * fabsf(ts.invz);
+                scale = 1.0f;
                 ts.oct = (float_to_bits(ts.invx) >> 31) | (float_to_bits(ts.invy) >> 31 << 1) |
                          (float_to_bits(ts.invz) >> 31 << 2);
                 ts.res.overflow = false;
@@ -780,14 +789,14 @@ __global__ __launch_bounds__(256) void trace_median_kernel(const F4 *__restrict_
 // Batched rendering: a vertex's rays of many scenes in one persistent launch.  Ray i of a queue belongs to
 // job job[i], whose scene is job_trace[job[i]]; rays of one job are contiguous in the queues, so a wave
 // rarely spans two scenes.
-template <int kStack, int kBlk>
+template <int kStack, int kBlk, bool kScaled = false>
 __global__ __launch_bounds__(kBlk, (kStack <= 12 && kBlk <= 256 ? 5 : 1)) void batch_trace_kernel(
     const TraceScene *__restrict__ job_trace, const uint32_t *__restrict__ path_job, RayArgs rays, HitArgs hits,
     const uint32_t *path_count, const uint32_t *__restrict__ shadow_job, RayArgs shadow, uint8_t *occluded,
     const uint32_t *shadow_count, ResolveArgs resolve, uint32_t n) {
     __shared__ RefillLds<kStack, kBlk, true> lds;
-    trace_vertex<kStack, kBlk>(JobScenes{job_trace, path_job}, rays, hits, path_count ? min(n, *path_count) : 0u,
-                               JobScenes{job_trace, shadow_job}, shadow, occluded,
+    trace_vertex<kStack, kBlk>(JobScenes<kScaled>{job_trace, path_job}, rays, hits, path_count ? min(n, *path_count) : 0u,
+                               JobScenes<kScaled>{job_trace, shadow_job}, shadow, occluded,
                                shadow_count ? min(n, *shadow_count) : 0u, resolve, lds);
 }
 
@@ -881,44 +890,46 @@ hipError_t launch_trace_stats_scratch(int device, const TraceScene &scene, const
 }
 
 // Node8 records (bvh8.h) re-encoded in place for the traversal (traverse8.h), a record a thread.
-__global__ __launch_bounds__(256) void encode_nodes_kernel(U4 *nodes, uint32_t n) {
+__global__ __launch_bounds__(256) void encode_nodes_kernel(U4 *nodes, uint32_t n, float scale) {
     const uint32_t i = blockIdx.x * 256 + threadIdx.x;
     if (i >= n) return;
     U4 in[5], out[5];
 #pragma unroll
     for (int k = 0; k < 5; ++k) in[k] = nodes[5 * (size_t)i + k];
-    encode_node(in, out);
+    encode_node(in, out, scale);
 #pragma unroll
     for (int k = 0; k < 5; ++k) nodes[5 * (size_t)i + k] = out[k];
 }
-hipError_t launch_encode_nodes(void *nodes, uint32_t n, hipStream_t stream) {
+hipError_t launch_encode_nodes(void *nodes, uint32_t n, float root_max, hipStream_t stream) {
     if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(encode_nodes_kernel, dim3((n + 255) / 256), dim3(256), 0, stream, static_cast<U4 *>(nodes), n);
+    hipLaunchKernelGGL(encode_nodes_kernel, dim3((n + 255) / 256), dim3(256), 0, stream, static_cast<U4 *>(nodes), n,
+                       box_scale(root_max));
     return hipGetLastError();
 }
 
 hipError_t launch_trace_vertex_batch(const TraceScene *job_trace, const uint32_t *path_job, const RayArgs &rays,
                                      const HitArgs &hits, const uint32_t *path_count, const uint32_t *shadow_job,
                                      const RayArgs &shadow, uint8_t *occluded, const uint32_t *shadow_count,
-                                     const ResolveArgs &resolve, uint32_t n, uint32_t max_depth, uint32_t block, uint32_t grid,
-                                     hipStream_t stream) {
+                                     const ResolveArgs &resolve, uint32_t n, uint32_t max_depth, float max_root, uint32_t block,
+                                     uint32_t grid, hipStream_t stream) {
     if (n == 0) return hipSuccess;
     const int need = max_depth > 1 ? (int)max_depth - 1 : 1;
     if (need > 24 || (block != 64 && block != 128 && block != 256 && block != 512) || grid == 0) return hipErrorInvalidValue;
-#define VT_BATCH(S, B)                                                                                                 \
-    hipLaunchKernelGGL((batch_trace_kernel<S, B>), dim3(grid), dim3(B), 0, stream, job_trace, path_job, rays, hits,     \
+#define VT_BATCH(S, B, X)                                                                                              \
+    hipLaunchKernelGGL((batch_trace_kernel<S, B, X>), dim3(grid), dim3(B), 0, stream, job_trace, path_job, rays, hits,  \
                        path_count, shadow_job, shadow, occluded, shadow_count, resolve, n)
-#define VT_BATCH_STACK(S)                                                                                              \
+#define VT_BATCH_STACK(S, X)                                                                                           \
     do {                                                                                                               \
-        if (block == 64) VT_BATCH(S, 64);                                                                              \
-        else if (block == 128) VT_BATCH(S, 128);                                                                       \
-        else if (block == 256) VT_BATCH(S, 256);                                                                       \
-        else VT_BATCH(S, 512);                                                                                         \
+        if (block == 64) VT_BATCH(S, 64, X);                                                                           \
+        else if (block == 128) VT_BATCH(S, 128, X);                                                                    \
+        else if (block == 256) VT_BATCH(S, 256, X);                                                                    \
+        else VT_BATCH(S, 512, X);                                                                                      \
     } while (0)
-    if (need <= 8) VT_BATCH_STACK(8);
-    else if (need <= 12) VT_BATCH_STACK(12);
-    else if (need <= 16) VT_BATCH_STACK(16);
-    else VT_BATCH_STACK(24);
+    if (box_scale(max_root) != 1.0f) VT_BATCH_STACK(24, true);
+    else if (need <= 8) VT_BATCH_STACK(8, false);
+    else if (need <= 12) VT_BATCH_STACK(12, false);
+    else if (need <= 16) VT_BATCH_STACK(16, false);
+    else VT_BATCH_STACK(24, false);
 #undef VT_BATCH_STACK
 #undef VT_BATCH
     return hipGetLastError();
@@ -929,8 +940,8 @@ hipError_t launch_trace_vertex(const TraceScene &scene, const RayArgs &rays, con
                                const ResolveArgs &resolve, uint32_t n, hipStream_t stream) {
     if (n == 0) return hipSuccess;
     const int need = scene.depth > 1 ? (int)scene.depth - 1 : 1;
-    if (scene.node_count == 0 || scene.kind != 0u || need > 24) {
-        // No 8-wide hierarchy: a launch for each part.
+    if (scene.node_count == 0 || scene.kind != 0u || need > 24 || box_scale(scene.root_max) != 1.0f) {
+        // No 8-wide hierarchy, or one with scaled boxes: a launch for each part.
         hipError_t e = path_count ? launch_trace(scene, rays, hits, nullptr, n, false, nullptr, stream, path_count) : hipSuccess;
         if (e != hipSuccess) return e;
         e = launch_trace(scene, shadow, HitArgs{}, occluded, n, true, nullptr, stream, shadow_count);
@@ -967,16 +978,17 @@ hipError_t launch_trace_tlas(const TlasScene &scene, const RayArgs &rays, const 
     const int top = scene.depth > 1 ? (int)scene.depth - 1 : 1, bot = scene.blas_depth > 1 ? (int)scene.blas_depth - 1 : 1;
     if (top > 16 || bot > 24) return hipErrorInvalidValue;
     // One stack holds the instance level's pending groups and, above them, those of the mesh a ray is in.
-#define VT_TLAS(S)                                                                                                     \
+#define VT_TLAS(S, X)                                                                                                  \
     do {                                                                                                               \
-        const uint32_t g = refill_grid(any ? (const void *)trace_tlas_kernel<true, S> : (const void *)trace_tlas_kernel<false, S>, n, kTlasBlock); \
-        if (any) hipLaunchKernelGGL((trace_tlas_kernel<true, S>), dim3(g), dim3(kTlasBlock), 0, stream, scene, rays, hits, occluded, n); \
-        else hipLaunchKernelGGL((trace_tlas_kernel<false, S>), dim3(g), dim3(kTlasBlock), 0, stream, scene, rays, hits, occluded, n); \
+        const uint32_t g = refill_grid(any ? (const void *)trace_tlas_kernel<true, S, X> : (const void *)trace_tlas_kernel<false, S, X>, n, kTlasBlock); \
+        if (any) hipLaunchKernelGGL((trace_tlas_kernel<true, S, X>), dim3(g), dim3(kTlasBlock), 0, stream, scene, rays, hits, occluded, n); \
+        else hipLaunchKernelGGL((trace_tlas_kernel<false, S, X>), dim3(g), dim3(kTlasBlock), 0, stream, scene, rays, hits, occluded, n); \
     } while (0)
-    if (top + bot <= 10) VT_TLAS(10);
-    else if (top + bot <= 16) VT_TLAS(16);
-    else if (top + bot <= 24) VT_TLAS(24);
-    else VT_TLAS(40);
+    if (box_scale(scene.blas_max) != 1.0f) VT_TLAS(40, true);
+    else if (top + bot <= 10) VT_TLAS(10, false);
+    else if (top + bot <= 16) VT_TLAS(16, false);
+    else if (top + bot <= 24) VT_TLAS(24, false);
+    else VT_TLAS(40, false);
 #undef VT_TLAS
     return hipGetLastError();
 }
@@ -1012,18 +1024,19 @@ hipError_t launch_trace(const TraceScene &scene, const RayArgs &rays, const HitA
     if (!counters) {
         // Persistent refill kernel: as many blocks as the chip holds at once (never more than the rays
         // need), each drawing its share of the rays.
-#define VT_REFILL(S)                                                                                                   \
+#define VT_REFILL(S, X)                                                                                                \
     do {                                                                                                               \
         constexpr int b = refill_block<S>();                                                                          \
-        const uint32_t g = refill_grid(any ? (const void *)trace_refill_kernel<true, S> : (const void *)trace_refill_kernel<false, S>, n, b); \
-        if (any) hipLaunchKernelGGL((trace_refill_kernel<true, S>), dim3(g), dim3(b), 0, stream, nd, tr, rays, hits, occluded, n, count, scene.root_max, scene.fault, cap < S ? cap : S); \
-        else hipLaunchKernelGGL((trace_refill_kernel<false, S>), dim3(g), dim3(b), 0, stream, nd, tr, rays, hits, occluded, n, count, scene.root_max, scene.fault, cap < S ? cap : S); \
+        const uint32_t g = refill_grid(any ? (const void *)trace_refill_kernel<true, S, X> : (const void *)trace_refill_kernel<false, S, X>, n, b); \
+        if (any) hipLaunchKernelGGL((trace_refill_kernel<true, S, X>), dim3(g), dim3(b), 0, stream, nd, tr, rays, hits, occluded, n, count, scene.root_max, scene.fault, cap < S ? cap : S); \
+        else hipLaunchKernelGGL((trace_refill_kernel<false, S, X>), dim3(g), dim3(b), 0, stream, nd, tr, rays, hits, occluded, n, count, scene.root_max, scene.fault, cap < S ? cap : S); \
     } while (0)
-        if (need <= 8) VT_REFILL(8);
-        else if (need <= 10) VT_REFILL(10);
-        else if (need <= 12) VT_REFILL(12);
-        else if (need <= 16) VT_REFILL(16);
-        else VT_REFILL(24);
+        if (box_scale(scene.root_max) != 1.0f) VT_REFILL(24, true);
+        else if (need <= 8) VT_REFILL(8, false);
+        else if (need <= 10) VT_REFILL(10, false);
+        else if (need <= 12) VT_REFILL(12, false);
+        else if (need <= 16) VT_REFILL(16, false);
+        else VT_REFILL(24, false);
 #undef VT_REFILL
         return hipGetLastError();
     }

@@ -49,12 +49,14 @@ struct TlasScene {
     const InstanceRecord *instances;    // leaf order
     uint32_t node_count, depth;         // of the instance hierarchy
     uint32_t blas_depth;                // deepest asset hierarchy
+    float blas_max;                     // largest root_max of the assets
     float enlarge, reach;               // per-ray growth of the instance boxes: enlarge (|origin|max + reach)
     uint32_t *fault;                    // raised (bit 0) by a ray whose node-group stack filled
 };
-// Re-encodes n Node8 records (bvh8.h) in place, in device memory, as the traversal reads them
-// (traverse8.h).  Every 8-wide hierarchy goes through it once, when it is published.
-hipError_t launch_encode_nodes(void *nodes, uint32_t n, hipStream_t stream);
+// Re-encodes n Node8 records (bvh8.h) of a hierarchy with max |coordinate| root_max in place, in device
+// memory, as the traversal reads them (traverse8.h).  Every 8-wide hierarchy goes through it once, when it is
+// published.
+hipError_t launch_encode_nodes(void *nodes, uint32_t n, float root_max, hipStream_t stream);
 
 // Closest hit (hits.instance = the instance's index, 0xffffffff on a miss) or any hit over a
 // two-level scene.  Among hits at exactly equal t the smaller instance index wins, then the smaller
@@ -99,12 +101,13 @@ hipError_t launch_trace_stats_scratch(int device, const TraceScene &scene, const
                                       hipStream_t stream);
 
 // launch_trace_vertex of batched rendering: ray i of a queue traces the scene job_trace[job[i]], on a
-// persistent grid of `grid` blocks of `block` (64, 128, 256 or 512) lanes; max_depth is the deepest tree.
+// persistent grid of `grid` blocks of `block` (64, 128, 256 or 512) lanes; max_depth is the deepest tree, max_root
+// the largest root_max.
 // path_count or shadow_count null: none of those rays.
 hipError_t launch_trace_vertex_batch(const TraceScene *job_trace, const uint32_t *path_job, const RayArgs &rays,
                                      const HitArgs &hits, const uint32_t *path_count, const uint32_t *shadow_job,
                                      const RayArgs &shadow, uint8_t *occluded, const uint32_t *shadow_count,
-                                     const ResolveArgs &resolve, uint32_t n, uint32_t max_depth, uint32_t block, uint32_t grid,
-                                     hipStream_t stream);
+                                     const ResolveArgs &resolve, uint32_t n, uint32_t max_depth, float max_root, uint32_t block,
+                                     uint32_t grid, hipStream_t stream);
 
 }  // namespace vt

@@ -10,7 +10,8 @@
 //        children (bits 24 + s)
 //   w2-4 per axis, word k: low and high plane of slot 2 k, low and high plane of slot 2 k + 1
 // A step is a power of two, so its high 16 bits are all of it; it is stored times 2^24, because the node
-// test reads a plane byte as the fp16 number with those bits, q 2^-24.
+// test reads a plane byte as the fp16 number with those bits, q 2^-24.  Origin and steps are further stored
+// times the hierarchy's box scale (box_scale), 1 for all but scenes of astronomical size.
 //
 // The node-group stack is abstracted (Stack::push/pop/size) so a kernel keeps it in LDS.
 // Arithmetic follows the reference exactly where results depend on it:
@@ -145,8 +146,17 @@ struct TravState {
     TraceResult res;
 };
 
-// Starts a ray with box enlargement e (trav_init: the reference's e for a one-level hierarchy).
-VT_HD void trav_init_e(TravState &st, const TraceRay &r, float e) {
+// The power of two by which a hierarchy's node boxes are scaled, and with them the ray's origin and its
+// distances in the node test, given its max |coordinate|: 1 below 2^82.  The steps times 2^24 times
+// 1 / direction, at most 1e8, must stay finite: unscaled they do up to steps of 2^76, and extents below 2^83
+// have no larger ones.
+// Above, 2^-64 keeps every product finite up to the largest extent a float holds; what it rounds away is
+// below 2^-62, and the boxes are enlarged by at least 2^62 there.
+VT_HD float box_scale(float root_max) { return root_max < 0x1p82f ? 1.0f : 0x1p-64f; }
+
+// Starts a ray with box enlargement e (trav_init: the reference's e for a one-level hierarchy) in a
+// hierarchy of box scale `scale`.
+VT_HD void trav_init_e(TravState &st, const TraceRay &r, float e, float scale) {
     st.res.t = r.tmax;
     st.res.b1 = st.res.b2 = 0.0f;
     st.res.face = -1;
@@ -165,6 +175,7 @@ VT_HD void trav_init_e(TravState &st, const TraceRay &r, float e) {
     st.invx = 1.0f / (fabsf(r.dx) < 1e-8f ? (sx ? -1e-8f : 1e-8f) : r.dx);
     st.invy = 1.0f / (fabsf(r.dy) < 1e-8f ? (sy ? -1e-8f : 1e-8f) : r.dy);
     st.invz = 1.0f / (fabsf(r.dz) < 1e-8f ? (sz ? -1e-8f : 1e-8f) : r.dz);
+    e *= scale;
     st.ex = e * fabsf(st.invx);
     st.ey = e * fabsf(st.invy);
     st.ez = e * fabsf(st.invz);
@@ -177,8 +188,8 @@ VT_HD void trav_init_e(TravState &st, const TraceRay &r, float e) {
 VT_HD float max_abs3(float x, float y, float z) { return fmaxf(fabsf(x), fmaxf(fabsf(y), fabsf(z))); }
 
 // main.swift:1790-1792: e = 1.1920929e-6 (|origin|max + root max).
-VT_HD void trav_init(TravState &st, const TraceRay &r, float root_max) {
-    trav_init_e(st, r, 1.1920929e-6f * (max_abs3(r.ox, r.oy, r.oz) + root_max));
+VT_HD void trav_init(TravState &st, const TraceRay &r, float root_max, float scale) {
+    trav_init_e(st, r, 1.1920929e-6f * (max_abs3(r.ox, r.oy, r.oz) + root_max), scale);
 }
 
 // The object-space ray of an instance (main.swift:1634-1637 instance_ray): origin and direction by
@@ -198,17 +209,16 @@ VT_HD TraceRay instance_ray(const float (&local)[3][4], const TraceRay &r, float
     return l;
 }
 
-#if defined(__HIPCC__)
-// The traversal's node (see the head of this file) of a builder's Node8, both as five 16-byte words.
-__device__ __forceinline__ void encode_node(const U4 (&n)[5], U4 (&o)[5]) {
+// The traversal's node (see the head of this file) of a builder's Node8, both as five 16-byte words, in a
+// hierarchy of box scale `scale`.
+VT_HD void encode_node(const U4 (&n)[5], U4 (&o)[5], float scale) {
     const uint32_t imask = n[0].w >> 24;
     uint32_t half[3];
     for (int a = 0; a < 3; ++a) {
-        // 2^(e - 127) as the builder's grid has it (0 for e = 0), times 2^24.  Beyond the float range the
-        // step is infinite and the node is never entered; geometry of that size has no hits, since the
-        // triangle test's products overflow long before.
-        const uint32_t e = (n[0].w >> (8 * a)) & 0xffu;
-        half[a] = e == 0u ? 0u : (e + 24u < 255u ? e + 24u : 255u) << 7;
+        // 2^(e - 127) as the builder's grid has it (0 for e = 0), times 2^24 and the box scale; 0 where
+        // that is below the normal floats (a step below 2^-86 of a scene of 2^82).
+        const int e = (int)((n[0].w >> (8 * a)) & 0xffu), x = e + 24 + (int)(float_to_bits(scale) >> 23) - 127;
+        half[a] = e == 0 || x < 1 ? 0u : (uint32_t)(x < 255 ? x : 255) << 7;
     }
     uint32_t tri = 0;
     for (int s = 0; s < 8; ++s) {
@@ -216,7 +226,8 @@ __device__ __forceinline__ void encode_node(const U4 (&n)[5], U4 (&o)[5]) {
         if (meta & 0x80u) continue;
         tri |= ((1u << (meta & 3u)) - 1u) << (3 * s);
     }
-    o[0] = U4{n[0].x, n[0].y, n[0].z, half[0] | (half[1] << 16)};
+    o[0] = U4{float_to_bits(bits_to_float(n[0].x) * scale), float_to_bits(bits_to_float(n[0].y) * scale),
+              float_to_bits(bits_to_float(n[0].z) * scale), half[0] | (half[1] << 16)};
     o[1] = U4{n[1].x, n[1].y, half[2] << 16, tri | (imask << 24)};
     const uint32_t lo[3][2] = {{n[2].x, n[2].y}, {n[2].z, n[2].w}, {n[3].x, n[3].y}};
     const uint32_t hi[3][2] = {{n[3].z, n[3].w}, {n[4].x, n[4].y}, {n[4].z, n[4].w}};
@@ -233,17 +244,24 @@ __device__ __forceinline__ void encode_node(const U4 (&n)[5], U4 (&o)[5]) {
 
 // Two bytes of w as two fp16 numbers q 2^-24: bytes 0 and 2 (sel kPlaneLo) or 1 and 3 (kPlaneHi).
 constexpr uint32_t kPlaneLo = 0x0c020c00u, kPlaneHi = 0x0c030c01u;
-typedef _Float16 h2v __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ h2v plane_pair(uint32_t w, uint32_t sel) {
-    return __builtin_bit_cast(h2v, __builtin_amdgcn_perm(w, w, sel));
+#if defined(__HIP_DEVICE_COMPILE__)
+typedef _Float16 PlanePair __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ PlanePair plane_pair(uint32_t w, uint32_t sel) {
+    return __builtin_bit_cast(PlanePair, __builtin_amdgcn_perm(w, w, sel));
 }
+__device__ __forceinline__ float plane(PlanePair p, int c) { return (float)p[c]; }
+#else
+typedef uint32_t PlanePair;
+VT_HD PlanePair plane_pair(uint32_t w, uint32_t sel) { return (sel == kPlaneLo ? w : w >> 8) & 0x00ff00ffu; }
+VT_HD float plane(PlanePair p, int c) { return (float)((p >> (16 * c)) & 0xffu) * 0x1p-24f; }
+#endif
 
 // Position of triangle bit p of a node with triangle bits tv (24 bits, tv's high byte ignored): the
 // triangles below it.
-__device__ __forceinline__ uint32_t tri_rank(uint32_t tv, uint32_t p) { return __builtin_popcount(tv & ((1u << p) - 1u)); }
+VT_HD uint32_t tri_rank(uint32_t tv, uint32_t p) { return __builtin_popcount(tv & ((1u << p) - 1u)); }
 
-// Node half of a step: tests st.node's 8 child boxes, pushes the current group if inner children were
-// hit, and moves st.node to the next node near to far.  Returns the triangles of the leaf children hit
+// Node half of a step in a hierarchy of box scale `scale`: tests st.node's 8 child boxes, pushes the current
+// group if inner children were hit, and moves st.node to the next node near to far.  Returns the triangles of the leaf children hit
 // (trimask: bits of the node's triangle word tri_bits, whose first triangle is tri_base; triangle p of
 // trimask is record tri_base + tri_rank(tri_bits, p)) and true when no node is left to visit (the
 // triangles returned must still be tested).  The next node does not depend on those triangles, so
@@ -252,26 +270,28 @@ __device__ __forceinline__ uint32_t tri_rank(uint32_t tv, uint32_t p) { return _
 // The kernels are bound by the instructions of this test.  Per child: six fused multiply-adds that read
 // their plane as fp16 in place (v_fma_mix_f32), four min / max, a compare and a select, with half an or, for
 // its bit of the hit mask (left to the compiler, which keeps two wait states between the compare and the
-// instruction that reads its mask, as this hardware wants); per node: 24 byte permutes that pick the near and far planes by
-// the ray's direction signs, and a few words' worth of bit arithmetic for the leaves' triangles and the
-// visiting order.  Converting each byte (48 v_cvt_f32_ubyte), choosing near and far words per axis and
+// instruction that reads its mask, as this hardware wants); per node: 24 byte permutes that pick the near and
+// far planes by the ray's direction signs, and a few words' worth of bit arithmetic for the leaves' triangles
+// and the visiting order.  Converting each byte (48 v_cvt_f32_ubyte), choosing near and far words per axis and
 // handling each child's leaf or inner kind in a branch took about 290 vector and 140 scalar instructions
 // a visit where this takes 200 and 40 (camera rays of the icosphere field 209 -> 168 us with the dealing
 // of rays in trace.hip, bounce rays of the 10 M terrain 775 -> 630 us, 2 M rays each).
 template <bool STATS, class Stack>
-__device__ __forceinline__ bool trav_nodes(TravState &st, const U4 *__restrict__ nodes, Stack &stack, uint32_t &trimask,
-                                           uint32_t &tri_base, uint32_t &tri_bits) {
+VT_HD bool trav_nodes(TravState &st, const U4 *__restrict__ nodes, float scale, Stack &stack, uint32_t &trimask,
+                      uint32_t &tri_base, uint32_t &tri_bits) {
     const U4 *np = nodes + 5 * (size_t)st.node;
     const U4 w0 = np[0], w1 = np[1], w2 = np[2], w3 = np[3], w4 = np[4];
     if (STATS) ++st.res.nodes;
     // Slab distances of plane q of an axis: ((q s + p) - o -+ e) / d = q (s / d) + (p - o) / d -+ e / |d|,
-    // one fma per plane.  The near plane of an axis is its low plane for a positive direction, its high
-    // plane otherwise.  The boxes are the reference's e-enlarged ones; the rounding differs from the
-    // reference's (plane - o -+ e) / d by a few ulps of terms no larger than the scene, far inside the
+    // one fma per plane, all in units of the box scale.  The near plane of an axis is its low plane for a
+    // positive direction, its high plane otherwise.  The boxes are the reference's e-enlarged ones; the rounding
+    // differs from the reference's (plane - o -+ e) / d by a few ulps of terms no larger than the scene, far inside the
     // enlargement, so no box the reference enters is culled.
     const float bx = bits_to_float(w0.w << 16) * st.invx, by = bits_to_float(w0.w & 0xffff0000u) * st.invy;
     const float bz = bits_to_float(w1.z) * st.invz;
-    const float dx = bits_to_float(w0.x) - st.ox, dy = bits_to_float(w0.y) - st.oy, dz = bits_to_float(w0.z) - st.oz;
+    const float dx = __builtin_fmaf(-st.ox, scale, bits_to_float(w0.x)), dy = __builtin_fmaf(-st.oy, scale, bits_to_float(w0.y));
+    const float dz = __builtin_fmaf(-st.oz, scale, bits_to_float(w0.z));
+    const float tmin = st.tmin * scale, tmax = st.res.t * scale;
     const float nx = __builtin_fmaf(dx, st.invx, -st.ex), fx = __builtin_fmaf(dx, st.invx, st.ex);
     const float ny = __builtin_fmaf(dy, st.invy, -st.ey), fy = __builtin_fmaf(dy, st.invy, st.ey);
     const float nz = __builtin_fmaf(dz, st.invz, -st.ez), fz = __builtin_fmaf(dz, st.invz, st.ez);
@@ -282,19 +302,21 @@ __device__ __forceinline__ bool trav_nodes(TravState &st, const U4 *__restrict__
     uint32_t hit = 0;  // bit s: the box of slot s is hit (slots without a child are masked below)
 #pragma unroll
     for (int k = 3; k >= 0; --k) {
-        const h2v pnx = plane_pair(wx[k], selx), pfx = plane_pair(wx[k], selx ^ kOther);
-        const h2v pny = plane_pair(wy[k], sely), pfy = plane_pair(wy[k], sely ^ kOther);
-        const h2v pnz = plane_pair(wz[k], selz), pfz = plane_pair(wz[k], selz ^ kOther);
+        const PlanePair pnx = plane_pair(wx[k], selx), pfx = plane_pair(wx[k], selx ^ kOther);
+        const PlanePair pny = plane_pair(wy[k], sely), pfy = plane_pair(wy[k], sely ^ kOther);
+        const PlanePair pnz = plane_pair(wz[k], selz), pfz = plane_pair(wz[k], selz ^ kOther);
 #pragma unroll
         for (int c = 1; c >= 0; --c) {
-            const float tnx = __builtin_fmaf((float)pnx[c], bx, nx), tfx = __builtin_fmaf((float)pfx[c], bx, fx);
-            const float tny = __builtin_fmaf((float)pny[c], by, ny), tfy = __builtin_fmaf((float)pfy[c], by, fy);
-            const float tnz = __builtin_fmaf((float)pnz[c], bz, nz), tfz = __builtin_fmaf((float)pfz[c], bz, fz);
-            const float tn = fmaxf(fmaxf(tnx, tny), fmaxf(tnz, st.tmin));
-            const float tf = fminf(fminf(tfx, tfy), fminf(tfz, st.res.t));
+            const float tnx = __builtin_fmaf(plane(pnx, c), bx, nx), tfx = __builtin_fmaf(plane(pfx, c), bx, fx);
+            const float tny = __builtin_fmaf(plane(pny, c), by, ny), tfy = __builtin_fmaf(plane(pfy, c), by, fy);
+            const float tnz = __builtin_fmaf(plane(pnz, c), bz, nz), tfz = __builtin_fmaf(plane(pfz, c), bz, fz);
+            const float tn = fmaxf(fmaxf(tnx, tny), fmaxf(tnz, tmin));
+            const float tf = fminf(fminf(tfx, tfy), fminf(tfz, tmax));
             hit |= tn <= tf ? 1u << (2 * k + c) : 0u;
         }
+#if defined(__HIP_DEVICE_COMPILE__)
         __builtin_amdgcn_sched_barrier(0);  // a pair of slots at a time: fewer registers, one wave more per SIMD
+#endif
     }
     // Each slot's bit spread to its three triangle bits.
     uint32_t spread = (hit | (hit << 8)) & 0x00f00fu;
@@ -333,7 +355,6 @@ __device__ __forceinline__ bool trav_nodes(TravState &st, const U4 *__restrict__
     st.node = st.cur_base + __builtin_popcount((st.cur_bits >> 8) & ((1u << slot) - 1u));
     return false;
 }
-#endif
 
 // A hit of the ray at t on face: the closest-hit rule (nearest t in [tmin, current t), equal t going
 // to the smaller face index).  For the any-hit query any t in [tmin, tmax) ends the ray.
@@ -345,10 +366,9 @@ VT_HD bool trav_accept(const TravState &st, float t, int32_t face) {
 
 // Triangle half of a step, one lane alone: tests the triangles trav_nodes returned.  Returns true
 // when an any-hit query found a hit.
-#if defined(__HIPCC__)
 template <bool ANY, bool STATS>
-__device__ __forceinline__ bool trav_tris(TravState &st, const WoopRay &w, const F4 *__restrict__ tris, uint32_t trimask, uint32_t tri_base,
-                                          uint32_t tri_bits) {
+VT_HD bool trav_tris(TravState &st, const WoopRay &w, const F4 *__restrict__ tris, uint32_t trimask, uint32_t tri_base,
+                     uint32_t tri_bits) {
     while (trimask) {
         const uint32_t b = __builtin_ctz(trimask);
         trimask &= trimask - 1u;
@@ -374,24 +394,24 @@ __device__ __forceinline__ bool trav_tris(TravState &st, const WoopRay &w, const
 // One step of one ray: a node visit and the triangles of the leaves it hits.  Returns true when the
 // ray is finished (result in st.res).
 template <bool ANY, bool STATS, class Stack>
-__device__ __forceinline__ bool trav_step(TravState &st, const WoopRay &w, const U4 *__restrict__ nodes, const F4 *__restrict__ tris, Stack &stack) {
+VT_HD bool trav_step(TravState &st, const WoopRay &w, const U4 *__restrict__ nodes, float scale,
+                     const F4 *__restrict__ tris, Stack &stack) {
     uint32_t trimask, tri_base, tri_bits;
-    const bool done = trav_nodes<STATS>(st, nodes, stack, trimask, tri_base, tri_bits);
+    const bool done = trav_nodes<STATS>(st, nodes, scale, stack, trimask, tri_base, tri_bits);
     if (trav_tris<ANY, STATS>(st, w, tris, trimask, tri_base, tri_bits)) return true;
     return done;
 }
 
 // Traverses one ray.  nodes: encoded nodes as 5 U4 each; tris: TriRecord as 3 F4 each.
 template <bool ANY, bool STATS, class Stack>
-__device__ __forceinline__ TraceResult traverse(const U4 *__restrict__ nodes, const F4 *__restrict__ tris, float root_max,
-                                                const TraceRay &r, Stack &stack) {
+VT_HD TraceResult traverse(const U4 *__restrict__ nodes, const F4 *__restrict__ tris, float root_max, float scale,
+                           const TraceRay &r, Stack &stack) {
     TravState st;
-    trav_init(st, r, root_max);
+    trav_init(st, r, root_max, scale);
     const WoopRay w = woop_ray(r.dx, r.dy, r.dz);
-    while (!trav_step<ANY, STATS>(st, w, nodes, tris, stack)) {
+    while (!trav_step<ANY, STATS>(st, w, nodes, scale, tris, stack)) {
     }
     return st.res;
 }
-#endif
 
 }  // namespace vt

@@ -89,6 +89,21 @@ def scattered_triangles(n=3000, seed=5):
     return mesh_from_triangles((c + e).astype(np.float32))
 
 
+def long_strip(length, axis):
+    """64 triangles of width 4 in a row along `axis` over [-length, length], with a ray parallel to another
+    axis at each triangle and as many beside the strip."""
+    ends = np.linspace(-length, length, 65)
+    tri = np.array([[[-2, 0, a], [2, 0, a], [0, 0, b]] for a, b in zip(ends[:-1], ends[1:])])
+    rays = np.zeros((8, 128), np.float32)
+    rays[0:3, :64] = tri.mean(axis=1).T
+    rays[0:3, 64:] = rays[0:3, :64] + np.array([[9.0], [0.0], [0.0]], np.float32)
+    rays[1], rays[4], rays[7] = 5.0, -1.0, 1e20
+    turn = axis - 2
+    rays[0:3], rays[3:6] = np.roll(rays[0:3], turn, axis=0), np.roll(rays[3:6], turn, axis=0)
+    v, f = mesh_from_triangles(np.roll(tri, turn, axis=2).astype(np.float32))
+    return v, f, rays
+
+
 def random_rays(n, seed, box=1.2, tmin=0.0, tmax=1e20):
     rng = np.random.default_rng(seed)
     o = rng.uniform(-box, box, (n, 3)).astype(np.float32)
