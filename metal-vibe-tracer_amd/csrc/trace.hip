@@ -651,10 +651,7 @@ __global__ __launch_bounds__(kTlasBlock, (kStack <= 10 ? 4 : 1)) void trace_tlas
                 ts.invx = top_ray[3][tid];
                 ts.invy = top_ray[4][tid];
                 ts.invz = top_ray[5][tid];
-                const float e = sc.enlarge * (max_abs3(ts.ox, ts.oy, ts.oz) + sc.reach);
-                ts.ex = e * fabsf(ts.invx);
-                ts.ey = e * fabsf(ts.invy);
-                ts.ez = e * fabsf(ts.invz);
+                set_enlargement(ts, sc.enlarge * (max_abs3(ts.ox, ts.oy, ts.oz) + sc.reach));
                 scale = 1.0f;
                 ts.oct = (float_to_bits(ts.invx) >> 31) | (float_to_bits(ts.invy) >> 31 << 1) |
                          (float_to_bits(ts.invz) >> 31 << 2);

@@ -146,6 +146,22 @@ struct TravState {
     TraceResult res;
 };
 
+// Sets the axes' box enlargements in units of the ray, e / |direction|.  Where one overflows (box scale 1 and
+// an origin beyond 1e36) the infinity would take every box into that axis' slab, and a ray that enters
+// nothing would visit the whole tree.  From an origin farther out on the axis than e (the scene, below 2^82,
+// is nothing beside it) the slab is infinitely far ahead or behind instead, as without enlargement; within e
+// of the scene it is indeed unbounded.
+VT_HD void set_enlargement(TravState &st, float e) {
+    st.ex = e * fabsf(st.invx);
+    st.ey = e * fabsf(st.invy);
+    st.ez = e * fabsf(st.invz);
+    if (__builtin_expect(e > 3.4e30f, 0)) {  // 1 / direction is at most 1e8
+        if (st.ex > 3.4028234664e38f && fabsf(st.ox) > 2.0f * e) st.ex = 0.0f;
+        if (st.ey > 3.4028234664e38f && fabsf(st.oy) > 2.0f * e) st.ey = 0.0f;
+        if (st.ez > 3.4028234664e38f && fabsf(st.oz) > 2.0f * e) st.ez = 0.0f;
+    }
+}
+
 // The power of two by which a hierarchy's node boxes are scaled, and with them the ray's origin and its
 // distances in the node test, given its max |coordinate|: 1 below 2^82.  The steps times 2^24 times
 // 1 / direction, at most 1e8, must stay finite: unscaled they do up to steps of 2^76, and extents below 2^83
@@ -175,10 +191,7 @@ VT_HD void trav_init_e(TravState &st, const TraceRay &r, float e, float scale) {
     st.invx = 1.0f / (fabsf(r.dx) < 1e-8f ? (sx ? -1e-8f : 1e-8f) : r.dx);
     st.invy = 1.0f / (fabsf(r.dy) < 1e-8f ? (sy ? -1e-8f : 1e-8f) : r.dy);
     st.invz = 1.0f / (fabsf(r.dz) < 1e-8f ? (sz ? -1e-8f : 1e-8f) : r.dz);
-    e *= scale;
-    st.ex = e * fabsf(st.invx);
-    st.ey = e * fabsf(st.invy);
-    st.ez = e * fabsf(st.invz);
+    set_enlargement(st, e * scale);
     st.oct = sx | (sy << 1) | (sz << 2);
     st.cur_base = 0;
     st.cur_bits = 0;

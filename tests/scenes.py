@@ -104,6 +104,17 @@ def long_strip(length, axis):
     return v, f, rays
 
 
+def far_rays(distance):
+    """Rays far from a scene around the origin, along directions with parallel axes or none at all, that reach
+    no box of it: at most one component of the origin is near."""
+    rays = []
+    for o in ((1, 1, 1), (-1, -1, -1), (1, 1, 0), (0, 1, -1), (1, 0, 1)):
+        for d in ((0, 0, 1), (0, 1, 0), (1, 0, 0), (0, 0, 0), (1e-9, 2e-9, 1), (0, -1, 0)):
+            for tmax in (1.0, 1e20):
+                rays.append([*(distance * np.array(o, np.float64)), *d, 0.0, tmax])
+    return np.array(rays).T.astype(np.float32)
+
+
 def random_rays(n, seed, box=1.2, tmin=0.0, tmax=1e20):
     rng = np.random.default_rng(seed)
     o = rng.uniform(-box, box, (n, 3)).astype(np.float32)

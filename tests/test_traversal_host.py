@@ -77,3 +77,13 @@ def test_uneven_extents(lib, extents):
         if along:
             rays[3:6] *= scale[:, None].astype(np.float32)
         check(lib, v, f, rays)
+
+
+@pytest.mark.parametrize("distance", [1e30, 2.8e36, 3e36, 1e37, 3.4e38])
+def test_far_origins_enter_nothing(lib, distance):
+    # From 2.9e36 on e / |direction| overflows for parallel axes.  No ray gets past the root node.
+    v, f = scenes.scattered_triangles(500, seed=2)
+    rays = scenes.far_rays(distance)
+    got, ref = check(lib, v, f, rays)
+    assert (ref["face"] < 0).all()
+    assert got["visits"].tolist() == [rays.shape[1], 0]

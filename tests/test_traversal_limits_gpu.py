@@ -107,3 +107,21 @@ def test_render_with_far_geometry(gpu_ctx):
     b.close()
     for s in built:
         s.close()
+
+
+@pytest.mark.parametrize("distance", [2.8e36, 3e36, 3.4e38])
+def test_far_origins(gpu_ctx, distance):
+    # They enter nothing (the node count shows it); the rays among them that do hit keep doing so.
+    v, f = scenes.scattered_triangles(500, seed=2)
+    far = scenes.far_rays(distance)
+    scene = gpu_ctx.set_mesh(vt.Mesh(v, f))
+    assert scene.trace_stats(_dev(far)) == (far.shape[1], 0)
+    assert scene.trace_stats(_dev(far), any_hit=True) == (far.shape[1], 0)
+    scene.close()
+    _check(gpu_ctx, v, f, np.concatenate([far, scenes.random_rays(1000, 2)], axis=1), f"origins at {distance:g}")
+    world = np.eye(3, 4, dtype=np.float32)
+    built = gpu_ctx.set_mesh(vt.Mesh(v, f))
+    tl = vt.Tlas(gpu_ctx, [(built, world)])
+    assert (tl.trace_closest(_dev(far))["face"].cpu().numpy() == -1).all()
+    tl.close()
+    built.close()
