@@ -1,6 +1,8 @@
 #include "readback.h"
 
+#include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <cstring>
 #include <system_error>
 #include <thread>
@@ -10,46 +12,39 @@
 namespace vt {
 
 ReadbackStage::~ReadbackStage() {
-    for (auto &t : done_)
-        for (hipEvent_t e : t)
-            if (e) (void)hipEventDestroy(e);
-    if (ready_) (void)hipEventDestroy(ready_);
-    if (stream_) (void)hipStreamDestroy(stream_);
+    for (hipEvent_t e : done_)
+        if (e) (void)hipEventDestroy(e);
     if (pinned_) (void)hipHostFree(pinned_);
 }
 
 // False when something could not be had; what was stays for the next attempt.
 bool ReadbackStage::prepare() {
-    if (!stream_ && hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking) != hipSuccess) return false;
-    if (!ready_ && hipEventCreateWithFlags(&ready_, hipEventDisableTiming) != hipSuccess) return false;
-    for (auto &t : done_)
-        for (hipEvent_t &e : t)
-            if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) return false;
-    return pinned_ || hipHostMalloc(reinterpret_cast<void **>(&pinned_), kThreads * 2 * kChunk, hipHostMallocDefault) == hipSuccess;
+    for (hipEvent_t &e : done_)
+        if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) return false;
+    return pinned_ || hipHostMalloc(reinterpret_cast<void **>(&pinned_), kThreads * kChunk, hipHostMallocDefault) == hipSuccess;
 }
 
-bool ReadbackStage::staged(int device, char *dst, const char *src, size_t bytes) {
-    if (hipEventRecord(ready_, nullptr) != hipSuccess || hipStreamWaitEvent(stream_, ready_, 0) != hipSuccess) return false;
-    const size_t chunks = (bytes + kChunk - 1) / kChunk;
+// The bytes copied from the front.
+size_t ReadbackStage::staged(int device, char *dst, const char *src, size_t bytes) {
+    using Clock = std::chrono::steady_clock;
+    const size_t chunk = bytes < kSmall ? kChunk / 2 : kChunk, chunks = (bytes + chunk - 1) / chunk;
     std::atomic<size_t> next{0};
-    std::atomic<bool> ok{true};
+    std::atomic<bool> ok{true}, busy{false};
     const auto work = [&](int t) {
-        char *const buf = pinned_ + (size_t)t * 2 * kChunk;
-        const auto size = [&](size_t c) { return c + 1 < chunks ? kChunk : bytes - c * kChunk; };
-        const auto start = [&](size_t c, int b) {
-            if (hipMemcpyAsync(buf + b * kChunk, src + c * kChunk, size(c), hipMemcpyDeviceToHost, stream_) != hipSuccess ||
-                hipEventRecord(done_[t][b], stream_) != hipSuccess)
-                ok = false;
-        };
+        char *const buf = pinned_ + (size_t)t * kChunk;
         if (hipSetDevice(device) != hipSuccess) ok = false;
-        size_t c = ok ? next++ : chunks;
-        if (c < chunks) start(c, 0);
-        for (int b = 0; c < chunks && ok; b ^= 1) {
-            const size_t n = next++;
-            if (n < chunks) start(n, b ^ 1);
-            if (hipEventSynchronize(done_[t][b]) != hipSuccess) ok = false;
-            if (ok) std::memcpy(dst + c * kChunk, buf + b * kChunk, size(c));
-            c = n;
+        while (ok && !busy) {
+            const size_t c = next++;
+            if (c >= chunks) return;
+            const size_t at = c * chunk, n = std::min(chunk, bytes - at);
+            const Clock::time_point start = Clock::now();
+            if (launch_copy_out(src + at, buf, n, nullptr) != hipSuccess || hipEventRecord(done_[t], nullptr) != hipSuccess ||
+                hipEventSynchronize(done_[t]) != hipSuccess) {
+                ok = false;
+                return;
+            }
+            if (Clock::now() - start > kBusy) busy = true;
+            std::memcpy(dst + at, buf, n);
         }
     };
     std::thread pool[kThreads];
@@ -63,23 +58,26 @@ bool ReadbackStage::staged(int device, char *dst, const char *src, size_t bytes)
     work(0);
     for (std::thread &t : pool)
         if (t.joinable()) t.join();
-    if (!ok) (void)hipStreamSynchronize(stream_);  // nothing is under way to the buffers any more
-    return ok;
+    if (ok) return std::min(bytes, next * chunk);
+    (void)hipStreamSynchronize(nullptr);  // nothing is under way to the buffers any more
+    return 0;
 }
 
 void ReadbackStage::copy(int device, void *dst, const void *src, size_t bytes) {
-    if (bytes >= 4 * kChunk) {
+    size_t done = 0;
+    if (bytes >= kStaged) {
         // Pinned and device destinations are copied to directly.
         hipPointerAttribute_t attr{};
         const bool known = hipPointerGetAttributes(&attr, dst) == hipSuccess && attr.type != hipMemoryTypeUnregistered;
         (void)hipGetLastError();  // an address that HIP does not know may be reported as an error
         std::unique_lock<std::mutex> lock(mutex_, std::try_to_lock);
-        const bool done = !known && lock.owns_lock() && prepare() &&
-                          staged(device, static_cast<char *>(dst), static_cast<const char *>(src), bytes);
-        if (done) return;
+        if (!known && lock.owns_lock() && prepare())
+            done = staged(device, static_cast<char *>(dst), static_cast<const char *>(src), bytes);
+        if (done == bytes) return;
         (void)hipGetLastError();
     }
-    check(hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost), "hipMemcpy");
+    check(hipMemcpy(static_cast<char *>(dst) + done, static_cast<const char *>(src) + done, bytes - done, hipMemcpyDeviceToHost),
+          "hipMemcpy");
 }
 
 }  // namespace vt

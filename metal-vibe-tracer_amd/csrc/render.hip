@@ -2084,6 +2084,15 @@ __global__ __launch_bounds__(256) void batch_accumulate_kernel(BatchTables bt, u
     }
 }
 
+// Image words to pinned host memory, past the caches.  Bound by the link to the host: 32 MB in 0.67 ms from 16
+// blocks on (8: 0.69), 50 GB/s; stores that stay in the caches reach 44 GB/s with 16 blocks.
+typedef uint32_t Words __attribute__((ext_vector_type(4)));
+constexpr uint32_t kCopyOutBlocks = 16;
+__global__ __launch_bounds__(256) void copy_out_kernel(const Words *src, Words *dst, uint32_t n) {
+    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256)
+        __builtin_nontemporal_store(src[i], dst + i);
+}
+
 // After every chunk of a sample: each job's next sample index, and the accumulated sample count.
 __global__ __launch_bounds__(256) void batch_advance_kernel(BatchTables bt) {
     const uint32_t j = blockIdx.x * 256 + threadIdx.x;
@@ -2214,6 +2223,15 @@ hipError_t launch_bake_metal(float *out, hipStream_t s) {
 
 hipError_t launch_reset_counters(uint32_t *counters, uint32_t n, hipStream_t s) {
     hipLaunchKernelGGL(reset_kernel, dim3(1), dim3(64), 0, s, counters, n);
+    return hipGetLastError();
+}
+
+hipError_t launch_copy_out(const void *src, void *dst, size_t bytes, hipStream_t s) {
+    const size_t n = bytes / 16;
+    if (bytes % 16 != 0 || n > 0x7fffffffu || ((uintptr_t)src | (uintptr_t)dst) % 16 != 0) return hipErrorInvalidValue;
+    if (n == 0) return hipSuccess;
+    hipLaunchKernelGGL(copy_out_kernel, dim3(kCopyOutBlocks), dim3(256), 0, s, static_cast<const Words *>(src),
+                       static_cast<Words *>(dst), (uint32_t)n);
     return hipGetLastError();
 }
 

@@ -233,6 +233,8 @@ hipError_t launch_decode_light_tree(const RenderScene &sc, float4 *out, hipStrea
 // Energy-table bake: ideal-metal complements (129 x 129, Hammersley 16384 per node).
 hipError_t launch_bake_metal(float *out, hipStream_t s);
 hipError_t launch_reset_counters(uint32_t *counters, uint32_t n, hipStream_t s);
+// dst = src, bytes a multiple of 16 and both 16-byte aligned; dst: pinned host memory.
+hipError_t launch_copy_out(const void *src, void *dst, size_t bytes, hipStream_t s);
 hipError_t launch_accumulate(const FrameArgs &f, const float *radiance, float *accum, uint32_t frame_index,
                              hipStream_t s);
 

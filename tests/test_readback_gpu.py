@@ -35,7 +35,7 @@ def _pinned(r, count):
     return t.numpy()
 
 
-# 16 bytes a pixel: 2 MiB chunks of 131072 pixels, staged from four of them on.
+# 16 bytes a pixel: staged from 8 MiB (524288 pixels) on, in chunks of 512 KiB, from 16 MiB on of 1 MiB.
 @pytest.mark.parametrize("w,h", [(1, 1), (512, 512), (524287, 1), (1024, 512), (524289, 1), (1024, 640), (1024, 1024), (1031, 1021)])
 def test_sizes_and_destinations(gpu_ctx, w, h):
     scene = _scene(gpu_ctx)
