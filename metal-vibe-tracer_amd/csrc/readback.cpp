@@ -4,7 +4,7 @@
 #include <atomic>
 #include <chrono>
 #include <cstring>
-#include <system_error>
+#include <exception>
 #include <thread>
 
 #include "scene.h"
@@ -51,7 +51,7 @@ size_t ReadbackStage::staged(int device, char *dst, const char *src, size_t byte
     for (int t = 1; t < kThreads && (size_t)t < chunks; ++t) {
         try {
             pool[t] = std::thread(work, t);
-        } catch (const std::system_error &) {
+        } catch (const std::exception &) {
             break;  // the threads there are draw all chunks
         }
     }

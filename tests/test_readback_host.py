@@ -41,7 +41,7 @@ def test_known_destination(program):
     assert _run(program, "known") == [("known", 20 * MB, 0, 20 * MB, 0, 0)]
 
 
-@pytest.mark.parametrize("mode", ["failures", "threads"])
+@pytest.mark.parametrize("mode", ["failures", "threads", "memory"])
 def test_failures(program, mode):
     assert _run(program, mode)
 
