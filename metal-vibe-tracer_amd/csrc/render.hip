@@ -1184,7 +1184,8 @@ __global__ __launch_bounds__(256) void restir_gbuffer_kernel(RenderScene sc, Fra
 //
 // It runs over the list of diffuse pixels that restir_gbuffer_kernel made: only they have reservoirs, and
 // run over the image the kernel, bound by vector issue, had idle lanes for all others (terrain of half
-// Lambert, half GGX faces, 1080p, 32 candidates: 5.03 ms, now 3.51 and 0.11 for the list).
+// Lambert, half GGX faces, 1080p, 32 candidates: 5.03 ms, now 3.51 and 0.11 for the list; where every pixel is
+// diffuse the list gains nothing and costs its 0.11 ms of a 6.7 ms frame).
 template <bool kEnv>
 __global__ __launch_bounds__(256, kEnv ? 1 : 4) void restir_initial_kernel(RenderScene sc, FrameArgs fa, PathQueue q,
                                                                           HitArgs hits, RestirArgs ra,
@@ -1199,100 +1200,87 @@ __global__ __launch_bounds__(256, kEnv ? 1 : 4) void restir_initial_kernel(Rende
     const uint32_t k = blockIdx.x * 256 + threadIdx.x;
     if (k >= *count) return;
     const uint32_t pix = list[k];
-    float4 gpos = make_float4(0.0f, 0.0f, 0.0f, -1.0f);
-    uint2 gnorm = pack_half4(0.0f, 0.0f, 0.0f, -1.0f);
-    float4 posdir = make_float4(0.0f, 0.0f, 0.0f, 0.0f), emitpdf = posdir, weights = posdir;
-    const int face = hits.face[pix];
-    if (face >= 0) {
-        const V3 dir = v3(q.dx[pix], q.dy[pix], q.dz[pix]);
-        const Surface s = surface_at(sc, (uint32_t)face, hits.b1[pix], hits.b2[pix], dir);
-        const Mat m = material(sc, s.slot);
-        const float t = hits.t[pix];
-        gpos = make_float4(s.p.x, s.p.y, s.p.z, t);
-        gnorm = pack_half4(s.n.x, s.n.y, s.n.z, (float)m.type);
-        if (m.type == kDiffuse) {
-            const Spectral sp{sc.icdf, reinterpret_cast<const float4 *>(sc.cmf), reinterpret_cast<const float4 *>(sc.basis)};
-            // The PCG stream for the resampling decisions; in Z mode each light candidate i is
-            // candidate i of the vertex-1 Z_DI event under the pixel's key (restir_di_initial,
-            // main.swift:4635-4652), so the candidates are stratified.
-            Rng rng{pix ^ (f.sample_index0 * 1999999973u), ZSampler{0u, 0u, 0u, 0u}, f.sampler == 1u};
-            if (rng.z) rng.zs.key = z_pixel_key(pix % f.width, pix / f.width, f.frame0 + 1u, f.sample_index0, f.z_temporal);
-            const uint32_t bits = ra.candidates > 1u ? 32u - (uint32_t)__clz(ra.candidates - 1u) : 0u;
-            // The primary's BSDF continuation covers the compensated table's zeros unless the depth is 1.
-            const uint32_t table = f.scattering_limit > 0 ? kEnvCompensated : kEnvOriginal;
-            const float u = q.wl[pix];
-            const Lanes lanes = lanes_of(sp, u);
-            const S4 rho_pi = scale(reflectance(sp, lanes, m.lagrange), 1.0f / kPi);
-            DiSample sel = di_empty();
-            float wsum = 0.0f, M = 0.0f;
-            if (cached && ra.candidates != 0u) lt_top_importances<256>(sc, top, s.p, top_l, top_r);
-            const V3 sp_p = s.p;
-            for (uint32_t i = 0; i < ra.candidates; ++i) {
-                if (rng.z) rng.zs.candidate(1u, kZDi, i, bits);
-                const LightSample ls =
-                    cached ? sample_emitter_via(sc, f, sp_p, rng, table,
-                                                [&](float u, float &pmf) { return lt_sample_top<256>(sc, sp_p, u, pmf, top, top_l, top_r); })
-                           : sample_emitter(sc, f, sp_p, rng, table);
-                DiSample c;
-                c.position = ls.light == 1u ? ls.wi : ls.position;
-                c.emission = ls.emission;
-                c.light = ls.light;
-                c.pdf = ls.pdf;
-                c.u = u;
-                M += 1.0f;
-                if (c.pdf > 0.0f) {
-                    const float ph = target_pdf(sp, lanes, rho_pi, s, dir, c, ls.geometry);
-                    const float proposal = c.pdf * ls.geometry;
-                    const float w = proposal > 0.0f ? ph / proposal : 0.0f;
-                    wsum += w;
-                    if (rand_f(rng.pcg) * wsum < w) sel = c;
-                }
-            }
-            if (ra.temporal) {
-                // restir_backproject through the previous sample's camera.
-                const V3 d = s.p - load_v3(ra.prev_eye);
-                const float w = dot(d, load_v3(ra.prev_forward));
-                if (w > 0.0f) {
-                    const float x = dot(d, load_v3(ra.prev_right)) / (w * ra.prev_aspect * ra.prev_fov_scale);
-                    const float y = dot(d, load_v3(ra.prev_up)) / (w * ra.prev_fov_scale);
-                    const float ux = x * 0.5f + 0.5f, uy = y * -0.5f + 0.5f;
-                    if (ux >= 0.0f && uy >= 0.0f && ux < 1.0f && uy < 1.0f) {
-                        const int px = (int)(ux * (float)f.width), py = (int)(uy * (float)f.height);
-                        if (px >= 0 && px < (int)f.width && py >= 0 && py < (int)f.height) {
-                            const uint32_t hp = (uint32_t)py * f.width + (uint32_t)px;
-                            const float4 hw = ra.hist.weights[hp];
-                            const float4 og = ra.hist.gpos[hp];
-                            const float4 on = unpack_half4(ra.hist.gnorm[hp]);
-                            // restir_same_surface (main.swift:4816-4823).
-                            const bool same = og.w > 0.0f && on.w == (float)m.type &&
-                                              dot(v3(on.x, on.y, on.z), s.n) > 0.95f &&
-                                              length(v3(og.x, og.y, og.z) - s.p) < fmaxf(0.01f, t * 0.01f);
-                            if (same && hw.y > 0.0f && hw.z > 0.0f) {
-                                const DiSample hs = di_stored(ra.hist.posdir[hp], ra.hist.emitpdf[hp], hw);
-                                const float ph = target_pdf_at(sc, f, sp, m, s, dir, hs);
-                                const float cm = fminf(hw.y, 20.0f);
-                                const float wt = ph * hw.z * cm;
-                                M += cm;
-                                wsum += wt;
-                                if (rand_f(rng.pcg) * wsum < wt) sel = hs;
-                            }
-                        }
+    const V3 dir = v3(q.dx[pix], q.dy[pix], q.dz[pix]);
+    const Surface s = surface_at(sc, (uint32_t)hits.face[pix], hits.b1[pix], hits.b2[pix], dir);
+    const Mat m = material(sc, s.slot);
+    const float t = hits.t[pix];
+    const Spectral sp{sc.icdf, reinterpret_cast<const float4 *>(sc.cmf), reinterpret_cast<const float4 *>(sc.basis)};
+    // The PCG stream for the resampling decisions; in Z mode each light candidate i is
+    // candidate i of the vertex-1 Z_DI event under the pixel's key (restir_di_initial,
+    // main.swift:4635-4652), so the candidates are stratified.
+    Rng rng{pix ^ (f.sample_index0 * 1999999973u), ZSampler{0u, 0u, 0u, 0u}, f.sampler == 1u};
+    if (rng.z) rng.zs.key = z_pixel_key(pix % f.width, pix / f.width, f.frame0 + 1u, f.sample_index0, f.z_temporal);
+    const uint32_t bits = ra.candidates > 1u ? 32u - (uint32_t)__clz(ra.candidates - 1u) : 0u;
+    // The primary's BSDF continuation covers the compensated table's zeros unless the depth is 1.
+    const uint32_t table = f.scattering_limit > 0 ? kEnvCompensated : kEnvOriginal;
+    const float u = q.wl[pix];
+    const Lanes lanes = lanes_of(sp, u);
+    const S4 rho_pi = scale(reflectance(sp, lanes, m.lagrange), 1.0f / kPi);
+    DiSample sel = di_empty();
+    float wsum = 0.0f, M = 0.0f;
+    if (cached && ra.candidates != 0u) lt_top_importances<256>(sc, top, s.p, top_l, top_r);
+    const V3 sp_p = s.p;
+    for (uint32_t i = 0; i < ra.candidates; ++i) {
+        if (rng.z) rng.zs.candidate(1u, kZDi, i, bits);
+        const LightSample ls =
+            cached ? sample_emitter_via(sc, f, sp_p, rng, table,
+                                        [&](float u, float &pmf) { return lt_sample_top<256>(sc, sp_p, u, pmf, top, top_l, top_r); })
+                   : sample_emitter(sc, f, sp_p, rng, table);
+        DiSample c;
+        c.position = ls.light == 1u ? ls.wi : ls.position;
+        c.emission = ls.emission;
+        c.light = ls.light;
+        c.pdf = ls.pdf;
+        c.u = u;
+        M += 1.0f;
+        if (c.pdf > 0.0f) {
+            const float ph = target_pdf(sp, lanes, rho_pi, s, dir, c, ls.geometry);
+            const float proposal = c.pdf * ls.geometry;
+            const float w = proposal > 0.0f ? ph / proposal : 0.0f;
+            wsum += w;
+            if (rand_f(rng.pcg) * wsum < w) sel = c;
+        }
+    }
+    if (ra.temporal) {
+        // restir_backproject through the previous sample's camera.
+        const V3 d = s.p - load_v3(ra.prev_eye);
+        const float w = dot(d, load_v3(ra.prev_forward));
+        if (w > 0.0f) {
+            const float x = dot(d, load_v3(ra.prev_right)) / (w * ra.prev_aspect * ra.prev_fov_scale);
+            const float y = dot(d, load_v3(ra.prev_up)) / (w * ra.prev_fov_scale);
+            const float ux = x * 0.5f + 0.5f, uy = y * -0.5f + 0.5f;
+            if (ux >= 0.0f && uy >= 0.0f && ux < 1.0f && uy < 1.0f) {
+                const int px = (int)(ux * (float)f.width), py = (int)(uy * (float)f.height);
+                if (px >= 0 && px < (int)f.width && py >= 0 && py < (int)f.height) {
+                    const uint32_t hp = (uint32_t)py * f.width + (uint32_t)px;
+                    const float4 hw = ra.hist.weights[hp];
+                    const float4 og = ra.hist.gpos[hp];
+                    const float4 on = unpack_half4(ra.hist.gnorm[hp]);
+                    // restir_same_surface (main.swift:4816-4823).
+                    const bool same = og.w > 0.0f && on.w == (float)m.type &&
+                                      dot(v3(on.x, on.y, on.z), s.n) > 0.95f &&
+                                      length(v3(og.x, og.y, og.z) - s.p) < fmaxf(0.01f, t * 0.01f);
+                    if (same && hw.y > 0.0f && hw.z > 0.0f) {
+                        const DiSample hs = di_stored(ra.hist.posdir[hp], ra.hist.emitpdf[hp], hw);
+                        const float ph = target_pdf_at(sc, f, sp, m, s, dir, hs);
+                        const float cm = fminf(hw.y, 20.0f);
+                        const float wt = ph * hw.z * cm;
+                        M += cm;
+                        wsum += wt;
+                        if (rand_f(rng.pcg) * wsum < wt) sel = hs;
                     }
                 }
             }
-            const float ph = target_pdf_at(sc, f, sp, m, s, dir, sel);
-            const float W = (M > 0.0f && ph > 0.0f) ? wsum / (M * ph) : 0.0f;
-            posdir = make_float4(sel.position.x, sel.position.y, sel.position.z, pack_light(sel.light));
-            emitpdf = make_float4(sel.emission.x, sel.emission.y, sel.emission.z, sel.pdf);
-            weights = make_float4(wsum, M, W, sel.u);
-            if (ra.gi) ra.gw.seed[pix] = rng.pcg;  // ReSTIR GI's draws continue this stream
         }
     }
-    ra.cur.gpos[pix] = gpos;
-    ra.cur.gnorm[pix] = gnorm;
-    ra.cur.posdir[pix] = posdir;
-    ra.cur.emitpdf[pix] = emitpdf;
-    ra.cur.weights[pix] = weights;
+    const float ph = target_pdf_at(sc, f, sp, m, s, dir, sel);
+    const float W = (M > 0.0f && ph > 0.0f) ? wsum / (M * ph) : 0.0f;
+    ra.cur.gpos[pix] = make_float4(s.p.x, s.p.y, s.p.z, t);
+    ra.cur.gnorm[pix] = pack_half4(s.n.x, s.n.y, s.n.z, (float)m.type);
+    ra.cur.posdir[pix] = make_float4(sel.position.x, sel.position.y, sel.position.z, pack_light(sel.light));
+    ra.cur.emitpdf[pix] = make_float4(sel.emission.x, sel.emission.y, sel.emission.z, sel.pdf);
+    ra.cur.weights[pix] = make_float4(wsum, M, W, sel.u);
+    if (ra.gi) ra.gw.seed[pix] = rng.pcg;  // ReSTIR GI's draws continue this stream
 }
 
 // ReSTIR GI stage 1 (restir_gi_initial, main.swift:4733-4743): at a diffuse primary hit, the x1 -> x2
