@@ -104,6 +104,23 @@ def long_strip(length, axis):
     return v, f, rays
 
 
+def series(count, ratio=0.6):
+    """Triangles (count, 3, 3) along a geometric series toward the origin: surface-area splits peel them off a
+    few at a time, so their hierarchy is far deeper than their number asks for."""
+    s = ratio ** np.arange(count)
+    return np.stack([np.stack([s, s, 0 * s], 1), np.stack([1.2 * s, s, 0.1 * s], 1), np.stack([s, 1.2 * s, 0.1 * s], 1)], 1)
+
+
+def series_rays(tri, n, seed):
+    """Rays at random points of the series' triangles, from origins at every scale."""
+    rng = np.random.default_rng(seed)
+    p = np.einsum("nk,nkj->nj", rng.dirichlet((1, 1, 1), n), tri[rng.integers(0, len(tri), n)])
+    o = p + rng.normal(size=(n, 3)) * (10.0 ** rng.uniform(-3, 0.5, n))[:, None]
+    d = p - o
+    return np.concatenate([o.T, (d / np.linalg.norm(d, axis=1, keepdims=True)).T, np.zeros((1, n)),
+                           np.full((1, n), 1e30)]).astype(np.float32)
+
+
 def far_rays(distance):
     """Rays far from a scene around the origin, along directions with parallel axes or none at all, that reach
     no box of it: at most one component of the origin is near."""

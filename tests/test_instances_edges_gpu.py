@@ -1,5 +1,5 @@
 """GPU tests of the two-level traversal at its edges: ray counts around a wave and a block, hierarchies of
-every stack depth the launcher tells apart, mirrored coincident instances whose hits tie at face 0 with other
+growing depth on both levels, mirrored coincident instances whose hits tie at face 0 with other
 barycentrics, and rays with NaN and exact limits, against the two-level oracle bit for bit."""
 import numpy as np
 import pytest
