@@ -23,7 +23,8 @@ constexpr int kNrcW5 = kNrcOutPad * kNrcHidden;             // 1024
 constexpr int kNrcParams = kNrcW1 + 3 * kNrcWh + kNrcW5;    // 30720
 constexpr float kNrcEmaDecay = 0.95f;
 
-// Blocks of a training launch at most, and so sets of partial gradients (one per CU).
+// Blocks of a training launch at most, and so sets of partial gradients (one per CU): 31.5 MB a cache, beside
+// 0.7 MB for all else, allocated with it whether it is trained or not, so that no training step allocates.
 constexpr uint32_t kNrcTrainBlocks = 256;
 
 struct NrcDevice {
