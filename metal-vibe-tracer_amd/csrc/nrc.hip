@@ -312,8 +312,9 @@ __global__ __launch_bounds__(kInferBlock) void nrc_infer_kernel(const uint16_t *
 //
 // Bound by LDS traffic and the encodings' sines at the sizes a frame trains on (16384 records: 128 blocks
 // on half the CUs, two waves a SIMD): a step takes 22.5 us, a quarter of it reading the weights the last
-// step's Adam wrote.  With one fp32 atomic per weight and block (7.9M a step), 64 samples a block of 4
-// waves and 2-byte strided LDS reads for the weight gradients it took 57.6 us.
+// step's Adam wrote; the kernel stands at its 256 registers and spills 11 (48 bytes of scratch a lane).  With
+// one fp32 atomic per weight and block (7.9M a step), 64 samples a block of 4 waves and 2-byte strided LDS
+// reads for the weight gradients it took 57.6 us.
 constexpr int kTrainBlock = 512, kTrainWaves = kTrainBlock / 64, kTrainSamples = 16 * kTrainWaves;
 constexpr int kTileSlots = 15;                        // gradient tiles per wave
 constexpr int kTPitch = kTrainSamples + 8;            // bf16 per transposed row: 272 bytes, 16 rows of

@@ -404,9 +404,10 @@ __device__ __forceinline__ void refill_trace(const Source &src, const RayArgs &r
     }
 }
 
-// Work-group of the persistent kernel: 512 lanes while LDS then holds 5 to 6 waves per SIMD, 256 for the
-// deepest stacks.  Trees up to depth 11, which the 10 M triangle terrain has, get a stack of 10 groups:
-// with one of 12 their blocks were 256 lanes and 5 % slower on its camera rays.
+// Work-group of the persistent kernel: 512 lanes up to a stack of 10 groups, 256 for deeper ones, of which
+// LDS holds too few otherwise.  Trees up to depth 11, which the 10 M triangle terrain has, get a stack of 10
+// groups: with one of 12 their blocks were 256 lanes and 5 % slower on its camera rays, though 5 waves per
+// SIMD are resident then and 4 (two blocks a CU) with 512.
 template <int kStack>
 constexpr int refill_block() {
     return kStack <= 10 ? 512 : 256;
@@ -415,6 +416,7 @@ constexpr int refill_block() {
 // shallow stacks of small scenes (Cornell image 9.49 against 9.83 ms), five for closest hits in deep
 // trees, whose rays wait on memory and whose caches a sixth wave only divides (10 M terrain, 2 M rays:
 // camera 480 -> 456 us, bounce 641 -> 630 us).
+// At six, trace_vertex_kernel<8> spills two registers (12 bytes of scratch a lane); no other kernel here does.
 template <bool ANY, int kStack>
 constexpr int refill_waves() {
     return kStack > 12 ? 1 : ANY || kStack <= 8 ? 6 : 5;  // LDS bounds the deeper stacks
