@@ -4,6 +4,7 @@
 #include <cmath>
 #include <cstring>
 #include <memory>
+#include <mutex>
 #include <vector>
 
 #include "nrc.h"
@@ -16,12 +17,13 @@ using vt::fail;
 
 struct vt_nrc {
     vt_context *ctx = nullptr;
-    // One allocation: params, grads, m, v, ema (fp32), the two bf16 copies, the loss sum, and the partial
-    // gradients of a backward launch's blocks.
+    // One allocation: params, grads, m, v, ema (fp32), the two bf16 copies and the loss sum.
     DeviceBuffer store;
     static constexpr size_t kSet = (size_t)vt::kNrcParams * 4;
-    static constexpr size_t kBf16 = 5 * kSet, kLoss = kBf16 + kSet, kPartials = kLoss + 256;
-    static constexpr size_t kBytes = kPartials + kSet * vt::kNrcTrainBlocks;
+    static constexpr size_t kBf16 = 5 * kSet, kLoss = kBf16 + kSet, kBytes = kLoss + 256;
+    // The partial gradients of a backward launch's blocks, from the first training on.
+    DeviceBuffer partials;
+    std::mutex partials_lock;
     uint32_t step = 0;
     float *params() const { return store.as<float>(); }
     float *grads() const { return params() + vt::kNrcParams; }
@@ -30,12 +32,27 @@ struct vt_nrc {
         float *p = params();
         uint16_t *w = reinterpret_cast<uint16_t *>(store.as<char>() + kBf16);
         return vt::NrcDevice{p, p + 2 * vt::kNrcParams, p + 3 * vt::kNrcParams, p + 4 * vt::kNrcParams,
-                             reinterpret_cast<float *>(store.as<char>() + kPartials), w, w + vt::kNrcParams};
+                             partials.as<float>(), w, w + vt::kNrcParams};
+    }
+    // A first training may be recorded into a graph: the relaxed capture mode lets the thread allocate meanwhile.
+    vt::NrcDevice training_view() {
+        std::lock_guard<std::mutex> guard(partials_lock);
+        if (!partials.ptr) {
+            hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+            check(hipThreadExchangeStreamCaptureMode(&mode), "hipThreadExchangeStreamCaptureMode");
+            void *p = nullptr;
+            const hipError_t e = hipMalloc(&p, kSet * vt::kNrcTrainBlocks);
+            (void)hipThreadExchangeStreamCaptureMode(&mode);
+            check(e, "hipMalloc");
+            partials.ptr = p;
+            partials.bytes = kSet * vt::kNrcTrainBlocks;
+        }
+        return view();
     }
 };
 
 namespace vt {
-NrcDevice nrc_device(vt_nrc *n) { return n->view(); }
+NrcDevice nrc_device(vt_nrc *n, bool train) { return train ? n->training_view() : n->view(); }
 uint32_t nrc_next_step(vt_nrc *n) { return ++n->step; }
 }  // namespace vt
 
@@ -140,8 +157,9 @@ vt_status vt_nrc_train(vt_nrc *n, const float *inputs, const float *targets, uin
         if (count == 0) return VT_OK;
         check(hipSetDevice(n->ctx->device), "hipSetDevice");
         hipStream_t s = (hipStream_t)stream;
-        check(vt::launch_nrc_backward(n->view(), inputs, targets, count, (float)count * vt::kNrcOut, nullptr, s), "nrc backward");
-        check(vt::launch_nrc_adam(n->view(), ++n->step, learning_rate, s, count), "nrc adam");
+        const vt::NrcDevice d = n->training_view();
+        check(vt::launch_nrc_backward(d, inputs, targets, count, (float)count * vt::kNrcOut, nullptr, s), "nrc backward");
+        check(vt::launch_nrc_adam(d, ++n->step, learning_rate, s, count), "nrc adam");
         return VT_OK;
     });
 }
@@ -151,10 +169,10 @@ vt_status vt_nrc_gradients(vt_nrc *n, const float *inputs, const float *targets,
     return vt::guarded_call([&]() -> vt_status {
         if (!n || (count && (!inputs || !targets)) || !grads) return fail(VT_ERROR_INVALID_ARGUMENT, "arguments must not be NULL");
         check(hipSetDevice(n->ctx->device), "hipSetDevice");
+        const vt::NrcDevice d = n->training_view();
         check(vt::launch_nrc_zero(n->loss(), 1, nullptr), "nrc zero");
-        check(vt::launch_nrc_backward(n->view(), inputs, targets, count, (float)count * vt::kNrcOut, n->loss(), nullptr),
-              "nrc backward");
-        check(vt::launch_nrc_reduce(n->view(), count, n->grads(), nullptr), "nrc reduce");
+        check(vt::launch_nrc_backward(d, inputs, targets, count, (float)count * vt::kNrcOut, n->loss(), nullptr), "nrc backward");
+        check(vt::launch_nrc_reduce(d, count, n->grads(), nullptr), "nrc reduce");
         check(hipDeviceSynchronize(), "hipDeviceSynchronize");
         check(hipMemcpy(grads, n->grads(), (size_t)vt::kNrcParams * 4, hipMemcpyDeviceToHost), "hipMemcpy");
         float l = 0.0f;

@@ -23,8 +23,8 @@ constexpr int kNrcW5 = kNrcOutPad * kNrcHidden;             // 1024
 constexpr int kNrcParams = kNrcW1 + 3 * kNrcWh + kNrcW5;    // 30720
 constexpr float kNrcEmaDecay = 0.95f;
 
-// Blocks of a training launch at most, and so sets of partial gradients (one per CU): 31.5 MB a cache, beside
-// 0.7 MB for all else, allocated with it whether it is trained or not, so that no training step allocates.
+// Blocks of a training launch at most, and so sets of partial gradients (one per CU): 31.5 MB, which a cache
+// has from its first training on, beside 0.7 MB for all else.
 constexpr uint32_t kNrcTrainBlocks = 256;
 
 struct NrcDevice {
@@ -64,6 +64,6 @@ hipError_t launch_nrc_zero(float *p, uint32_t n, hipStream_t s);
 struct vt_nrc;
 namespace vt {
 // Device view and the next Adam step number of a cache object (nrc.cpp).
-NrcDevice nrc_device(vt_nrc *n);
+NrcDevice nrc_device(vt_nrc *n, bool train);  // train: with room for the partial gradients
 uint32_t nrc_next_step(vt_nrc *n);
 }  // namespace vt

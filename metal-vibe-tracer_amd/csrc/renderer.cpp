@@ -64,7 +64,7 @@ struct vt_renderer {
     vt_nrc *cache = nullptr;
     DeviceBuffer nrc_queries, nrc_records, nrc_sacc;
     uint32_t nrc_capacity = 0, nrc_rcap = 0;
-    vt::NrcDevice cache_device() const { return vt::nrc_device(cache); }
+    vt::NrcDevice cache_device(bool train) const { return vt::nrc_device(cache, train); }
     uint32_t cache_next_step() { return vt::nrc_next_step(cache); }
     ~vt_renderer() {
         if (host_count) (void)hipHostFree(host_count);
@@ -848,7 +848,7 @@ static vt_status render_frame(vt_renderer *r, vt_scene *scene, const vt_frame_pa
                 // The cache answers the paths that ended at its vertices, then learns from this
                 // wavefront's training records: 4 Adam steps over equal slices of them (at most 16384
                 // records a step), the slices sized on the device from the record count.
-                const vt::NrcDevice nd = r->cache_device();
+                const vt::NrcDevice nd = r->cache_device(train_cache);
                 check(vt::launch_nrc_infer(nd, na.q_in, n, na.q_out, s, na.q_count, na.q_stride), "cache infer");
                 check(vt::launch_cache_resolve(sc, na, n, r->radiance.as<float>(), s), "cache resolve");
                 check(vt::launch_build_targets(na, s), "cache targets");
