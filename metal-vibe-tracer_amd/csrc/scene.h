@@ -74,6 +74,8 @@ struct vt_context {
 };
 
 namespace vt {
+// Uploads a builder's n nodes (Node8) into dst, encoded for the traversal; complete on return.
+void publish_nodes(DeviceBuffer &dst, const void *nodes, uint32_t n, float root_max);
 // Bakes ctx->energy_metal / energy_luts once (GPU bakes, host averages and unorm16 quantisation).
 void ensure_energy_tables(vt_context *ctx);
 // The pinhole camera of the reference's orbit view (eye, target, +y up, vertical fov) and the image

@@ -226,11 +226,7 @@ std::unique_ptr<vt_tlas> build_tlas(vt_context *ctx, const vt_instance *list, ui
     check(hipSetDevice(ctx->device), "hipSetDevice");
     const uint64_t bytes = top.nodes.size() * sizeof(Node8) + (uint64_t)count * sizeof(InstanceRecord);
     if (ctx->resident + bytes > ctx->budget) throw BudgetError("The imported meshes exceed the safe GPU memory budget.");
-    t->nodes.upload(top.nodes.data(), top.nodes.size() * sizeof(Node8));
-    // Instances lie within 1e8 (above), so their boxes are unscaled.  Waited for: the first trace may come on
-    // any stream.
-    check(launch_encode_nodes(t->nodes.ptr, (uint32_t)top.nodes.size(), 0.0f, nullptr), "encode nodes");
-    check(hipStreamSynchronize(nullptr), "hipStreamSynchronize");
+    publish_nodes(t->nodes, top.nodes.data(), (uint32_t)top.nodes.size(), 0.0f);  // instances lie within 1e8 (above)
     t->accounted = t->nodes.bytes;
     ctx->resident += t->nodes.bytes;
     t->view.nodes = t->nodes.ptr;

@@ -54,8 +54,7 @@ struct TlasScene {
     uint32_t *fault;                    // raised (bit 0) by a ray whose node-group stack filled
 };
 // Re-encodes n Node8 records (bvh8.h) of a hierarchy with max |coordinate| root_max in place, in device
-// memory, as the traversal reads them (traverse8.h).  Every 8-wide hierarchy goes through it once, when it is
-// published.
+// memory, as the traversal reads them (traverse8.h).
 hipError_t launch_encode_nodes(void *nodes, uint32_t n, float root_max, hipStream_t stream);
 
 // Closest hit (hits.instance = the instance's index, 0xffffffff on a miss) or any hit over a

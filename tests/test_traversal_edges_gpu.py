@@ -87,3 +87,12 @@ def test_ray_limits(gpu_ctx):
     assert (h["b1"].cpu().numpy() == 0).all()
     assert (scene.trace_any(_dev(r)).cpu().numpy() == 0).all()
     scene.close()
+
+
+@pytest.mark.parametrize("count,nodes", [(640, 63), (624, 64), (660, 65), (716, 67)])
+def test_where_nodes_are_encoded(gpu_ctx, count, nodes):
+    # Up to 64 nodes are encoded by the host, more by a kernel.
+    v, f = scenes.scattered_triangles(count, seed=1)
+    assert len(vt.build_bvh8_host(vt.Mesh(v, f))[0]) == nodes
+    rays = np.concatenate([scenes.random_rays(6000, count), scenes.axis_rays(600, count)], axis=1)
+    _check(gpu_ctx, v, f, rays, f"{nodes} nodes")
