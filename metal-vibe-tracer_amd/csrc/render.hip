@@ -1142,36 +1142,72 @@ __global__ __launch_bounds__(256) void generate_kernel(FrameArgs f, PathQueue q,
 
 // The pixels of ReSTIR's pass 1: the G-buffer and an empty reservoir for a pixel whose camera ray missed or
 // met another than a diffuse surface; the diffuse pixels are listed, block by block in image order, for
-// restir_initial_kernel.
-__global__ __launch_bounds__(256) void restir_gbuffer_kernel(RenderScene sc, FrameArgs f, PathQueue q, HitArgs hits,
-                                                             RestirBuffers cur, uint32_t *list, unsigned long long *count) {
-    __shared__ AppendShared append;
-    const uint32_t pix = blockIdx.x * kShadeBlock + threadIdx.x;
-    bool diffuse = false;
-    if (pix < f.npix) {
+// restir_initial_kernel.  With `all` the other pixels are listed from the list's end, so that it is also the
+// primary vertex' order of shading (ordered_slot): the layered BSDF runs in waves of its own but for the few misses
+// and emitters.  One atomic per list and 2048 pixels: such adds retire 10 ns apart, and with one per 256
+// pixels they were most of this kernel's time (Cornell box, 1280 x 720: 40 us, now 12.5; terrain of 10 M
+// half Lambert, half GGX faces, 1920 x 1080: 110 us and 25 for a classification of its own, now 78).
+constexpr uint32_t kListBlock = 1024, kListPixels = 2;  // pixels per thread
+__global__ __launch_bounds__(kListBlock) void restir_gbuffer_kernel(RenderScene sc, FrameArgs f, PathQueue q, HitArgs hits,
+                                                                    RestirBuffers cur, uint32_t *list, uint32_t *counts,
+                                                                    uint32_t all) {
+    __shared__ uint32_t wave_counts[kListPixels][kListBlock / 64][2], base[2];
+    const uint32_t first = blockIdx.x * (kListBlock * kListPixels) + threadIdx.x;
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const unsigned long long below = (1ull << lane) - 1ull;
+    uint32_t kind[kListPixels], rank[kListPixels];  // 0 a diffuse hit, 1 another pixel, 2 none
+#pragma unroll
+    for (uint32_t j = 0; j < kListPixels; ++j) {
+        const uint32_t pix = first + j * kListBlock;
+        kind[j] = 2u;
+        if (pix < f.npix) {
+            const int face = hits.face[pix];
+            kind[j] = face >= 0 && material(sc, sc.faces[4 * (size_t)face + 3]).type == kDiffuse ? 0u : 1u;
+        }
+        const unsigned long long m0 = __ballot(kind[j] == 0u), m1 = __ballot(kind[j] == 1u);
+        rank[j] = (uint32_t)__popcll((kind[j] == 1u ? m1 : m0) & below);
+        if (lane == 0) {
+            wave_counts[j][wave][0] = (uint32_t)__popcll(m0);
+            wave_counts[j][wave][1] = (uint32_t)__popcll(m1);
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < 1u + all) {
+        uint32_t sum = 0;
+        for (uint32_t j = 0; j < kListPixels; ++j)
+            for (uint32_t w = 0; w < kListBlock / 64; ++w) {
+                const uint32_t c = wave_counts[j][w][threadIdx.x];
+                wave_counts[j][w][threadIdx.x] = sum;
+                sum += c;
+            }
+        base[threadIdx.x] = sum ? atomicAdd(counts + threadIdx.x, sum) : 0u;
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t j = 0; j < kListPixels; ++j) {
+        const uint32_t pix = first + j * kListBlock;
+        if (kind[j] == 2u) continue;
+        if (kind[j] <= all) {
+            const uint32_t at = base[kind[j]] + wave_counts[j][wave][kind[j]] + rank[j];
+            list[kind[j] ? f.npix - 1u - at : at] = pix;
+        }
+        if (kind[j] == 0u) continue;
+        const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         float4 gpos = make_float4(0.0f, 0.0f, 0.0f, -1.0f);
         uint2 gnorm = pack_half4(0.0f, 0.0f, 0.0f, -1.0f);
         const int face = hits.face[pix];
         if (face >= 0) {
             const V3 dir = v3(q.dx[pix], q.dy[pix], q.dz[pix]);
             const Surface s = surface_at(sc, (uint32_t)face, hits.b1[pix], hits.b2[pix], dir);
-            const uint32_t type = material(sc, s.slot).type;
-            diffuse = type == kDiffuse;
             gpos = make_float4(s.p.x, s.p.y, s.p.z, hits.t[pix]);
-            gnorm = pack_half4(s.n.x, s.n.y, s.n.z, (float)type);
+            gnorm = pack_half4(s.n.x, s.n.y, s.n.z, (float)material(sc, s.slot).type);
         }
-        if (!diffuse) {
-            const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            cur.gpos[pix] = gpos;
-            cur.gnorm[pix] = gnorm;
-            cur.posdir[pix] = zero;
-            cur.emitpdf[pix] = zero;
-            cur.weights[pix] = zero;
-        }
+        cur.gpos[pix] = gpos;
+        cur.gnorm[pix] = gnorm;
+        cur.posdir[pix] = zero;
+        cur.emitpdf[pix] = zero;
+        cur.weights[pix] = zero;
     }
-    uint32_t at[2];
-    block_append(append, 0, count, diffuse, false, at);
-    if (diffuse) list[at[0]] = pix;
 }
 
 // Pass 1 of ReSTIR DI for one sample (restir_temporal_kernel, main.swift:4842-4940): one thread per
@@ -1184,8 +1220,8 @@ __global__ __launch_bounds__(256) void restir_gbuffer_kernel(RenderScene sc, Fra
 //
 // It runs over the list of diffuse pixels that restir_gbuffer_kernel made: only they have reservoirs, and
 // run over the image the kernel, bound by vector issue, had idle lanes for all others (terrain of half
-// Lambert, half GGX faces, 1080p, 32 candidates: 5.03 ms, now 3.51 and 0.11 for the list; where every pixel is
-// diffuse the list gains nothing and costs its 0.11 ms of a 6.7 ms frame).
+// Lambert, half GGX faces, 1080p, 32 candidates: 5.03 ms, now 3.49 and 0.08 for the list; where every pixel is
+// diffuse the list gains nothing and costs 12 us at 1280 x 720).
 template <bool kEnv>
 __global__ __launch_bounds__(256, kEnv ? 1 : 4) void restir_initial_kernel(RenderScene sc, FrameArgs fa, PathQueue q,
                                                                           HitArgs hits, RestirArgs ra,
@@ -2126,11 +2162,10 @@ hipError_t launch_shade(const RenderScene &sc, const FrameArgs &f, const PathQue
 
 hipError_t launch_shade_restir(const RenderScene &sc, const FrameArgs &f, const PathQueue &in, const HitArgs &hits,
                                const PathQueue &out, const ShadowQueue &sh, const Counters &c, uint32_t capacity,
-                               float *radiance, const RestirArgs &ra, const NrcArgs &nrc, uint32_t *perm,
-                               uint32_t *classes, hipStream_t s) {
+                               float *radiance, const RestirArgs &ra, const NrcArgs &nrc, const uint32_t *perm,
+                               const uint32_t *classes, hipStream_t s) {
     const dim3 grid((capacity + kShadeBlock - 1) / kShadeBlock);
     const ShadeOrder order{perm, classes};
-    if (perm) launch_classify(sc, hits, c.in, capacity, perm, classes, s);
     const bool env = frame_has_env(sc, f);
     if (sc.layered && env)
         hipLaunchKernelGGL((shade_kernel<true, true, true>), grid, dim3(256), 0, s, sc, f, in, hits, out, sh, c,
@@ -2148,14 +2183,15 @@ hipError_t launch_shade_restir(const RenderScene &sc, const FrameArgs &f, const 
 }
 
 hipError_t launch_restir_initial(const RenderScene &sc, const FrameArgs &f, const PathQueue &q, const HitArgs &hits,
-                                 const RestirArgs &ra, uint32_t *list, uint32_t *count, hipStream_t s) {
+                                 const RestirArgs &ra, uint32_t *list, uint32_t *counts, bool all, hipStream_t s) {
+    constexpr uint32_t kPer = kListBlock * kListPixels;
+    hipLaunchKernelGGL(restir_gbuffer_kernel, dim3((f.npix + kPer - 1) / kPer), dim3(kListBlock), 0, s, sc, f, q, hits, ra.cur, list,
+                       counts, all ? 1u : 0u);
     const dim3 grid((f.npix + 255) / 256);
-    hipLaunchKernelGGL(restir_gbuffer_kernel, grid, dim3(kShadeBlock), 0, s, sc, f, q, hits, ra.cur, list,
-                       reinterpret_cast<unsigned long long *>(count));
     if (frame_has_env(sc, f))
-        hipLaunchKernelGGL(restir_initial_kernel<true>, grid, dim3(256), 0, s, sc, f, q, hits, ra, list, count);
+        hipLaunchKernelGGL(restir_initial_kernel<true>, grid, dim3(256), 0, s, sc, f, q, hits, ra, list, counts);
     else
-        hipLaunchKernelGGL(restir_initial_kernel<false>, grid, dim3(256), 0, s, sc, f, q, hits, ra, list, count);
+        hipLaunchKernelGGL(restir_initial_kernel<false>, grid, dim3(256), 0, s, sc, f, q, hits, ra, list, counts);
     return hipGetLastError();
 }
 

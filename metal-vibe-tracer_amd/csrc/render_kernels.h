@@ -202,9 +202,10 @@ hipError_t launch_shade(const RenderScene &sc, const FrameArgs &f, const PathQue
                         float *radiance, const NrcArgs &nrc, uint32_t *perm, uint32_t *classes, hipStream_t s);
 // Pass 1 of ReSTIR DI (restir_temporal_kernel): G-buffer, RIS candidates, temporal merge, encode,
 // for the wavefront's single sample (q holds the camera paths in pixel order, hits their hits).  list: room
-// for npix pixel indices; count: two cleared counter words, 8-byte aligned.
+// for npix pixel indices; counts: two cleared counter words.  With `all` the list then holds every pixel in the
+// order launch_shade_restir takes, diffuse ones first, and counts[0] their number.
 hipError_t launch_restir_initial(const RenderScene &sc, const FrameArgs &f, const PathQueue &q, const HitArgs &hits,
-                                 const RestirArgs &ra, uint32_t *list, uint32_t *count, hipStream_t s);
+                                 const RestirArgs &ra, uint32_t *list, uint32_t *counts, bool all, hipStream_t s);
 // ReSTIR GI after pass 1: the x1 -> x2 rays (ra.gw); once they are traced, the light sample at each
 // diffuse x2 and its shadow ray (stage 2); then, with the shadow rays traced, the initial reservoir,
 // the temporal merge and the encode into ra.gcur.
@@ -217,11 +218,12 @@ hipError_t launch_restir_gi_finish(const RenderScene &sc, const FrameArgs &f, co
 // contribution of each connection that is not occluded.
 hipError_t launch_restir_gi_resolve(const FrameArgs &f, const RestirArgs &ra, float *radiance, hipStream_t s);
 // launch_shade with ReSTIR DI at the primary vertex (sampling mode 0): spatial reuse of ra.cur,
-// shading with one visibility ray, then the path suffix.
+// shading with one visibility ray, then the path suffix.  perm, classes (or null): launch_restir_initial's list
+// of all pixels and its counts.
 hipError_t launch_shade_restir(const RenderScene &sc, const FrameArgs &f, const PathQueue &in, const HitArgs &hits,
                                const PathQueue &out, const ShadowQueue &sh, const Counters &c, uint32_t capacity,
-                               float *radiance, const RestirArgs &ra, const NrcArgs &nrc, uint32_t *perm,
-                               uint32_t *classes, hipStream_t s);
+                               float *radiance, const RestirArgs &ra, const NrcArgs &nrc, const uint32_t *perm,
+                               const uint32_t *classes, hipStream_t s);
 // Adds each cache query's answer: radiance[id] += rgb(thr * max(y, 0)) at the path's wavelengths.
 hipError_t launch_cache_resolve(const RenderScene &sc, const NrcArgs &nrc, uint32_t capacity, float *radiance,
                                 hipStream_t s);

@@ -805,7 +805,7 @@ static vt_status render_frame(vt_renderer *r, vt_scene *scene, const vt_frame_pa
                 const vt::PathQueue qin = r->q[cur].view(r->capacity), qout = r->q[1 - cur].view(r->capacity);
                 const vt::Counters c{pair(b), reinterpret_cast<unsigned long long *>(pair(b + 1))};
                 if (restir && b == 0) {
-                    check(vt::launch_restir_initial(sc, f, qin, hits, ra, r->perm.as<uint32_t>(), cnt + 2, s), "restir pass 1");
+                    check(vt::launch_restir_initial(sc, f, qin, hits, ra, r->perm.as<uint32_t>(), cnt + 2, perm != nullptr, s), "restir pass 1");
                     if (gi) {
                         // ReSTIR GI's x1 -> x2 rays, the light samples at x2 and their shadow rays, then
                         // the reservoirs.
@@ -821,8 +821,7 @@ static vt_status render_frame(vt_renderer *r, vt_scene *scene, const vt_frame_pa
                         check(vt::launch_restir_gi_finish(sc, f, qin, hits, ra, s), "restir gi reservoirs");
                     }
                     check(vt::launch_shade_restir(sc, f, qin, hits, qout, sh, c, n, r->radiance.as<float>(), ra, na,
-                                                  perm,
-                                           cnt + vt::kCounterClasses + 2 * b, s),
+                                                  perm, cnt + 2, s),
                           "shade");
                 } else {
                     check(vt::launch_shade(sc, f, qin, hits, qout, sh, c, n, r->radiance.as<float>(), na, perm,
