@@ -1172,15 +1172,18 @@ __global__ __launch_bounds__(kListBlock) void restir_gbuffer_kernel(RenderScene 
         }
     }
     __syncthreads();
-    if (threadIdx.x < 1u + all) {
-        uint32_t sum = 0;
-        for (uint32_t j = 0; j < kListPixels; ++j)
-            for (uint32_t w = 0; w < kListBlock / 64; ++w) {
-                const uint32_t c = wave_counts[j][w][threadIdx.x];
-                wave_counts[j][w][threadIdx.x] = sum;
-                sum += c;
-            }
-        base[threadIdx.x] = sum ? atomicAdd(counts + threadIdx.x, sum) : 0u;
+    if (wave == 0u) {
+        // Exclusive sums of either kind's counts, half a wave each.
+        static_assert(kListPixels * (kListBlock / 64) == 32, "a count per lane");
+        const uint32_t which = lane >> 5, j = (lane >> 4) & 1u, w = lane & 15u, c = wave_counts[j][w][which];
+        uint32_t sum = c;
+#pragma unroll
+        for (uint32_t d = 1; d < 32u; d <<= 1) {
+            const uint32_t v = __shfl_up(sum, d, 32);
+            sum += (lane & 31u) >= d ? v : 0u;
+        }
+        wave_counts[j][w][which] = sum - c;
+        if ((lane & 31u) == 31u) base[which] = sum && which <= all ? atomicAdd(counts + which, sum) : 0u;
     }
     __syncthreads();
 #pragma unroll
