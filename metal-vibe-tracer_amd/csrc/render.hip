@@ -1140,6 +1140,30 @@ __global__ __launch_bounds__(256) void generate_kernel(FrameArgs f, PathQueue q,
     generate_path(f, i - s * f.npix, f.sample_index0 + s, q, i, radiance);
 }
 
+// Whether a pixel's camera ray met a diffuse surface: only then has it a reservoir.
+__device__ __forceinline__ bool restir_diffuse(const RenderScene &sc, const HitArgs &hits, uint32_t pix) {
+    const int face = hits.face[pix];
+    return face >= 0 && material(sc, sc.faces[4 * (size_t)face + 3]).type == kDiffuse;
+}
+// The G-buffer and the empty reservoir of any other pixel.
+__device__ __forceinline__ void restir_other(const RenderScene &sc, const PathQueue &q, const HitArgs &hits,
+                                             const RestirBuffers &cur, uint32_t pix) {
+    const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    float4 gpos = make_float4(0.0f, 0.0f, 0.0f, -1.0f);
+    uint2 gnorm = pack_half4(0.0f, 0.0f, 0.0f, -1.0f);
+    const int face = hits.face[pix];
+    if (face >= 0) {
+        const V3 dir = v3(q.dx[pix], q.dy[pix], q.dz[pix]);
+        const Surface s = surface_at(sc, (uint32_t)face, hits.b1[pix], hits.b2[pix], dir);
+        gpos = make_float4(s.p.x, s.p.y, s.p.z, hits.t[pix]);
+        gnorm = pack_half4(s.n.x, s.n.y, s.n.z, (float)material(sc, s.slot).type);
+    }
+    cur.gpos[pix] = gpos;
+    cur.gnorm[pix] = gnorm;
+    cur.posdir[pix] = zero;
+    cur.emitpdf[pix] = zero;
+    cur.weights[pix] = zero;
+}
 // The pixels of ReSTIR's pass 1: the G-buffer and an empty reservoir for a pixel whose camera ray missed or
 // met another than a diffuse surface; the diffuse pixels are listed, block by block in image order, for
 // restir_initial_kernel.  With `all` the other pixels are listed from the list's end, so that it is also the
@@ -1160,10 +1184,7 @@ __global__ __launch_bounds__(kListBlock) void restir_gbuffer_kernel(RenderScene 
     for (uint32_t j = 0; j < kListPixels; ++j) {
         const uint32_t pix = first + j * kListBlock;
         kind[j] = 2u;
-        if (pix < f.npix) {
-            const int face = hits.face[pix];
-            kind[j] = face >= 0 && material(sc, sc.faces[4 * (size_t)face + 3]).type == kDiffuse ? 0u : 1u;
-        }
+        if (pix < f.npix) kind[j] = restir_diffuse(sc, hits, pix) ? 0u : 1u;
         const unsigned long long m0 = __ballot(kind[j] == 0u), m1 = __ballot(kind[j] == 1u);
         rank[j] = (uint32_t)__popcll((kind[j] == 1u ? m1 : m0) & below);
         if (lane == 0) {
@@ -1194,22 +1215,7 @@ __global__ __launch_bounds__(kListBlock) void restir_gbuffer_kernel(RenderScene 
             const uint32_t at = base[kind[j]] + wave_counts[j][wave][kind[j]] + rank[j];
             list[kind[j] ? f.npix - 1u - at : at] = pix;
         }
-        if (kind[j] == 0u) continue;
-        const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        float4 gpos = make_float4(0.0f, 0.0f, 0.0f, -1.0f);
-        uint2 gnorm = pack_half4(0.0f, 0.0f, 0.0f, -1.0f);
-        const int face = hits.face[pix];
-        if (face >= 0) {
-            const V3 dir = v3(q.dx[pix], q.dy[pix], q.dz[pix]);
-            const Surface s = surface_at(sc, (uint32_t)face, hits.b1[pix], hits.b2[pix], dir);
-            gpos = make_float4(s.p.x, s.p.y, s.p.z, hits.t[pix]);
-            gnorm = pack_half4(s.n.x, s.n.y, s.n.z, (float)material(sc, s.slot).type);
-        }
-        cur.gpos[pix] = gpos;
-        cur.gnorm[pix] = gnorm;
-        cur.posdir[pix] = zero;
-        cur.emitpdf[pix] = zero;
-        cur.weights[pix] = zero;
+        if (kind[j] == 1u) restir_other(sc, q, hits, cur, pix);
     }
 }
 
@@ -1222,7 +1228,7 @@ __global__ __launch_bounds__(kListBlock) void restir_gbuffer_kernel(RenderScene 
 // light-tree walk is latency-bound and a fourth wave is worth more than the few registers it saves).
 //
 // It runs over the list of diffuse pixels that restir_gbuffer_kernel made: only they have reservoirs, and
-// run over the image the kernel, bound by vector issue, had idle lanes for all others (terrain of half
+// run over the image (list null: small frames, launch_restir_initial's caller) the kernel, bound by vector issue, had idle lanes for all others (terrain of half
 // Lambert, half GGX faces, 1080p, 32 candidates: 5.03 ms, now 3.49 and 0.08 for the list; where every pixel is
 // diffuse the list gains nothing and costs 12 us at 1280 x 720).
 template <bool kEnv>
@@ -1232,13 +1238,18 @@ __global__ __launch_bounds__(256, kEnv ? 1 : 4) void restir_initial_kernel(Rende
     const FrameArgs f = frame_env<kEnv>(fa);
     __shared__ LtTop top;
     __shared__ float top_l[kLtTopInner][256], top_r[kLtTopInner][256];
-    if (blockIdx.x * 256 >= *count) return;  // the whole block
+    const uint32_t n = list ? *count : f.npix;
+    if (blockIdx.x * 256 >= n) return;  // the whole block
     const bool cached = sc.tree_node_count != 0u;
     if (cached && threadIdx.x < (unsigned)kLtTopAll) lt_top_fill(sc, top, threadIdx.x);
     __syncthreads();
     const uint32_t k = blockIdx.x * 256 + threadIdx.x;
-    if (k >= *count) return;
-    const uint32_t pix = list[k];
+    if (k >= n) return;
+    const uint32_t pix = list ? list[k] : k;
+    if (!list && !restir_diffuse(sc, hits, pix)) {
+        restir_other(sc, q, hits, ra.cur, pix);
+        return;
+    }
     const V3 dir = v3(q.dx[pix], q.dy[pix], q.dz[pix]);
     const Surface s = surface_at(sc, (uint32_t)hits.face[pix], hits.b1[pix], hits.b2[pix], dir);
     const Mat m = material(sc, s.slot);
@@ -2188,8 +2199,10 @@ hipError_t launch_shade_restir(const RenderScene &sc, const FrameArgs &f, const 
 hipError_t launch_restir_initial(const RenderScene &sc, const FrameArgs &f, const PathQueue &q, const HitArgs &hits,
                                  const RestirArgs &ra, uint32_t *list, uint32_t *counts, bool all, hipStream_t s) {
     constexpr uint32_t kPer = kListBlock * kListPixels;
-    hipLaunchKernelGGL(restir_gbuffer_kernel, dim3((f.npix + kPer - 1) / kPer), dim3(kListBlock), 0, s, sc, f, q, hits, ra.cur, list,
-                       counts, all ? 1u : 0u);
+    if (all && !list) return hipErrorInvalidValue;
+    if (list)
+        hipLaunchKernelGGL(restir_gbuffer_kernel, dim3((f.npix + kPer - 1) / kPer), dim3(kListBlock), 0, s, sc, f, q, hits, ra.cur, list,
+                           counts, all ? 1u : 0u);
     const dim3 grid((f.npix + 255) / 256);
     if (frame_has_env(sc, f))
         hipLaunchKernelGGL(restir_initial_kernel<true>, grid, dim3(256), 0, s, sc, f, q, hits, ra, list, counts);

@@ -202,8 +202,8 @@ hipError_t launch_shade(const RenderScene &sc, const FrameArgs &f, const PathQue
                         float *radiance, const NrcArgs &nrc, uint32_t *perm, uint32_t *classes, hipStream_t s);
 // Pass 1 of ReSTIR DI (restir_temporal_kernel): G-buffer, RIS candidates, temporal merge, encode,
 // for the wavefront's single sample (q holds the camera paths in pixel order, hits their hits).  list: room
-// for npix pixel indices; counts: two cleared counter words.  With `all` the list then holds every pixel in the
-// order launch_shade_restir takes, diffuse ones first, and counts[0] their number.
+// for npix pixel indices, or null to go over the image; counts: two cleared counter words.  With `all` the list
+// then holds every pixel in the order launch_shade_restir takes, diffuse ones first, and counts[0] their number.
 hipError_t launch_restir_initial(const RenderScene &sc, const FrameArgs &f, const PathQueue &q, const HitArgs &hits,
                                  const RestirArgs &ra, uint32_t *list, uint32_t *counts, bool all, hipStream_t s);
 // ReSTIR GI after pass 1: the x1 -> x2 rays (ra.gw); once they are traced, the light sample at each
