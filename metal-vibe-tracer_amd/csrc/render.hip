@@ -1228,9 +1228,10 @@ __global__ __launch_bounds__(kListBlock) void restir_gbuffer_kernel(RenderScene 
 // light-tree walk is latency-bound and a fourth wave is worth more than the few registers it saves).
 //
 // It runs over the list of diffuse pixels that restir_gbuffer_kernel made: only they have reservoirs, and
-// run over the image (list null: small frames, launch_restir_initial's caller) the kernel, bound by vector issue, had idle lanes for all others (terrain of half
+// run over the image the kernel, bound by vector issue, had idle lanes for all others (terrain of half
 // Lambert, half GGX faces, 1080p, 32 candidates: 5.03 ms, now 3.49 and 0.08 for the list; where every pixel is
-// diffuse the list gains nothing and costs 12 us at 1280 x 720).
+// diffuse the list gains nothing and costs 12 us at 1280 x 720).  Without a list (null: small frames, where
+// render_frame has the figures) it does run over the image and writes the other pixels itself.
 template <bool kEnv>
 __global__ __launch_bounds__(256, kEnv ? 1 : 4) void restir_initial_kernel(RenderScene sc, FrameArgs fa, PathQueue q,
                                                                           HitArgs hits, RestirArgs ra,
@@ -2201,8 +2202,8 @@ hipError_t launch_restir_initial(const RenderScene &sc, const FrameArgs &f, cons
     constexpr uint32_t kPer = kListBlock * kListPixels;
     if (all && !list) return hipErrorInvalidValue;
     if (list)
-        hipLaunchKernelGGL(restir_gbuffer_kernel, dim3((f.npix + kPer - 1) / kPer), dim3(kListBlock), 0, s, sc, f, q, hits, ra.cur, list,
-                           counts, all ? 1u : 0u);
+        hipLaunchKernelGGL(restir_gbuffer_kernel, dim3((f.npix + kPer - 1) / kPer), dim3(kListBlock), 0, s, sc, f, q,
+                           hits, ra.cur, list, counts, all ? 1u : 0u);
     const dim3 grid((f.npix + 255) / 256);
     if (frame_has_env(sc, f))
         hipLaunchKernelGGL(restir_initial_kernel<true>, grid, dim3(256), 0, s, sc, f, q, hits, ra, list, counts);
